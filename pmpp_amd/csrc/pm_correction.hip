@@ -15,8 +15,8 @@
 // g phi + r tanh(o) scale applied to the source instead (phi is linear in S), which keeps the
 // correction inside the banded spectral step with no extra FFT pair.
 //
-// Reductions are deterministic: one float64 partial per block, summed in block order by
-// the consumer.
+// Reductions are deterministic: one float64 partial per block, summed by one wave of the
+// consumer in a fixed order.
 #include <hip/hip_bf16.h>
 
 #include <algorithm>
@@ -46,11 +46,6 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
   return t;  // valid on thread 0
 }
 
-__device__ __forceinline__ double sum_partials(const double* __restrict__ p, int nb) {
-  double t = 0.0;
-  for (int i = 0; i < nb; ++i) t += p[i];
-  return t;
-}
 
 // ----------------------------------------------------------- features ----
 // sum ((rho + shift) c)^2: float4 loads with four independent float64 chains per thread (rho
@@ -82,8 +77,8 @@ __global__ void __launch_bounds__(kBlock) k_source_sumsq(const float* __restrict
 __global__ void k_source_scale(const double* __restrict__ partials, int nb, int64_t n, float r,
                                const float* __restrict__ lin, float a, float om, float s8,
                                float* __restrict__ stats) {
+  const double ms = wave_sum(partials, nb) / (double)n;
   if (threadIdx.x != 0) return;
-  const double ms = sum_partials(partials, nb) / (double)n;
   const float sigma = sqrtf((float)ms + 1e-6f);
   const float th = tanhf(lin[0] * a + lin[1] * om + lin[2] * s8 + lin[3]);
   stats[0] = sigma;
@@ -93,8 +88,8 @@ __global__ void k_source_scale(const double* __restrict__ partials, int nb, int6
 
 // stats[3] = sigma_p = sqrt(mean phi^2 + 1e-6)
 __global__ void k_potential_scale(const double* __restrict__ partials, int nb, int64_t n, float* __restrict__ stats) {
-  if (threadIdx.x != 0) return;
-  stats[3] = sqrtf((float)(sum_partials(partials, nb) / (double)n) + 1e-6f);
+  const double ms = wave_sum(partials, nb) / (double)n;
+  if (threadIdx.x == 0) stats[3] = sqrtf((float)ms + 1e-6f);
 }
 
 __global__ void __launch_bounds__(kBlock) k_features(const float* __restrict__ rho, const float* __restrict__ phi,
@@ -162,8 +157,8 @@ __global__ void __launch_bounds__(kBlock) k_residual_bwd(const float* __restrict
 // d/d[w0, w1, w2, b] of the gain layer
 __global__ void k_gain_bwd(const double* __restrict__ partials, int nb, float r, const float* __restrict__ stats,
                            float a, float om, float s8, float* __restrict__ dlin) {
+  const float dg = (float)wave_sum(partials, nb);
   if (threadIdx.x != 0) return;
-  const float dg = (float)sum_partials(partials, nb);
   const float th = stats[2];
   const float dp = dg * r * (1.f - th * th);
   dlin[0] = dp * a;
@@ -225,18 +220,19 @@ __global__ void __launch_bounds__(kBlock) k_input_sums(const float* __restrict__
 __global__ void k_input_scalars(const double* __restrict__ partials, int nb, int64_t n, float c, float r,
                                 const float* __restrict__ stats, const float* __restrict__ lin, int potential,
                                 float* __restrict__ scal) {
+  const double p1 = wave_sum(partials, nb);
+  const double p2 = wave_sum(partials + kMaxBlocks, nb);
+  const double p3 = wave_sum(partials + 2 * kMaxBlocks, nb);
+  const double p4 = wave_sum(partials + 3 * kMaxBlocks, nb);
+  const double p5 = potential ? wave_sum(partials + 4 * kMaxBlocks, nb) : 0.0;  // uniform
   if (threadIdx.x != 0) return;
-  const double p1 = sum_partials(partials, nb);
-  const double p2 = sum_partials(partials + kMaxBlocks, nb);
-  const double p3 = sum_partials(partials + 2 * kMaxBlocks, nb);
-  const double p4 = sum_partials(partials + 3 * kMaxBlocks, nb);
   const double sigma = stats[0];
   const double th = stats[2];
   scal[0] = (float)((double)r / c * p1 - p2 / (sigma * sigma));
   scal[1] = (float)(p3 - 1.5 * (double)r * sigma / ((double)c * c) * p1 + (double)r * (1.0 - th * th) * lin[1] * p4);
   if (potential) {
     const double sp = stats[3];
-    scal[2] = (float)(sum_partials(partials + 4 * kMaxBlocks, nb) / ((double)n * sp * sp * sp));
+    scal[2] = (float)(p5 / ((double)n * sp * sp * sp));
   }
 }
 
@@ -278,10 +274,9 @@ __global__ void __launch_bounds__(kBlock) k_input_bwd(const float* __restrict__ 
 
 __global__ void k_input_omega(const double* __restrict__ partials, int nb, const float* __restrict__ scal, float om,
                               int potential, float* __restrict__ omega_cot) {
-  if (threadIdx.x != 0) return;
-  double t = 1.5 * sum_partials(partials, nb) + (double)scal[1];
-  if (potential) t += sum_partials(partials + kMaxBlocks, nb) / (double)om;
-  omega_cot[0] += (float)t;
+  double t = 1.5 * wave_sum(partials, nb) + (double)scal[1];
+  if (potential) t += wave_sum(partials + kMaxBlocks, nb) / (double)om;  // uniform
+  if (threadIdx.x == 0) omega_cot[0] += (float)t;
 }
 
 // ---------------------------------------------------------------- loss ----
@@ -306,9 +301,9 @@ __global__ void __launch_bounds__(kBlock) k_loss_partials(const float* __restric
 }
 
 __global__ void k_loss_finalize(const double* __restrict__ partials, int nb, double* __restrict__ loss) {
+  const double num = wave_sum(partials, nb);
+  const double den = wave_sum(partials + kMaxBlocks, nb);
   if (threadIdx.x != 0) return;
-  const double num = sum_partials(partials, nb);
-  const double den = sum_partials(partials + kMaxBlocks, nb);
   loss[0] = den > 0.0 ? num / den : 0.0;
   loss[1] = den > 0.0 ? 1.0 / den : 0.0;
 }
@@ -342,8 +337,9 @@ __global__ void __launch_bounds__(kBlock) k_adamax(float* __restrict__ p, const 
                                                    float b2, float eps, float clip, __bf16* __restrict__ pbf) {
   __shared__ float s_scale, s_bc;
   __shared__ int s_ok;
+  const double sumsq = threadIdx.x < 64 ? wave_sum(partials, nb) : 0.0;  // the first wave
   if (threadIdx.x == 0) {
-    const double norm = sqrt(sum_partials(partials, nb));
+    const double norm = sqrt(sumsq);
     s_ok = isfinite(norm) ? 1 : 0;
     s_scale = (clip > 0.f && norm >= (double)clip) ? (float)(clip / norm) : 1.f;
     const int t = count[0] + 1;
@@ -365,8 +361,8 @@ __global__ void __launch_bounds__(kBlock) k_adamax(float* __restrict__ p, const 
 }
 
 __global__ void k_count(int32_t* __restrict__ count, const double* __restrict__ partials, int nb) {
-  if (threadIdx.x != 0) return;
-  if (isfinite(sum_partials(partials, nb))) count[0] = count[0] + 1;
+  const double sumsq = wave_sum(partials, nb);
+  if (threadIdx.x == 0 && isfinite(sumsq)) count[0] = count[0] + 1;
 }
 
 __global__ void __launch_bounds__(kBlock) k_to_bf16(const float* __restrict__ src, int64_t n,

@@ -795,9 +795,10 @@ __global__ void __launch_bounds__(kBlock) k_cot_sorted(const int32_t* __restrict
 // reciprocal) with it, so every mesh cotangent and with them every particle's displacement
 // cotangent and the Omega_m cotangent come out NaN, as the unfused float chain would give.
 __global__ void k_cot_scale(const float* __restrict__ pmax, int nb, float* __restrict__ scale) {
-  if (threadIdx.x != 0) return;
   float m = 0.f;
-  for (int i = 0; i < nb; ++i) m = fmaxf(m, pmax[i]);
+  for (int i = threadIdx.x; i < nb; i += 64) m = fmaxf(m, pmax[i]);  // one wave
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  if (threadIdx.x != 0) return;
   scale[0] = !(m <= 3.402823466e38f) ? __int_as_float(0x7fc00000) : (m > 0.f ? fminf(1.f / m, 1.7014118e38f) : 1.f);
 }
 
@@ -877,12 +878,10 @@ __global__ void __launch_bounds__(kBlock) k_source_bwd(float* __restrict__ src_c
   }
 }
 
-// omega_cot[0] += 1.5 * (the block partials of k_source_bwd, summed in block order)
+// omega_cot[0] += 1.5 * (the block partials of k_source_bwd, summed in a fixed order)
 __global__ void k_source_bwd_sum(const double* __restrict__ part, int nb, float* __restrict__ omega_cot) {
-  if (threadIdx.x != 0) return;
-  double t = 0.0;
-  for (int b = 0; b < nb; ++b) t += part[b];
-  omega_cot[0] += 1.5f * (float)t;
+  const double t = wave_sum(part, nb);
+  if (threadIdx.x == 0) omega_cot[0] += 1.5f * (float)t;
 }
 
 constexpr int kSrcBlocks = 2048;  // blocks of k_source_bwd (and its partials)
