@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PM_ABI_VERSION 9
+#define PM_ABI_VERSION 10
 
 enum pm_status {
   PM_SUCCESS = 0,
@@ -338,6 +338,9 @@ int pm_power_spectrum_bwd(const float* spec, const int32_t shape[3], int32_t mas
  *                      gact is given.
  * pm_conv3d_bwd_weight dw_db = [dW (27*16*cin floats), db (16 floats)] for pre-activation
  *                      gradient dz and layer input x; workspace from the query.
+ * pm_conv3d_bwd_weight_out1  the same for a one-output-channel layer (16 input channels) from its
+ *                      one-channel gradient dz0 (n floats): dw_db in the 16-channel layout, channel
+ *                      0's entries and zeros; workspace as pm_conv3d_bwd_weight's for cin = 16.
  * pm_conv3d_stem       act = gelu(conv(x0; w[27][16][8]) + bias) for the network input x0 that
  *                      pm_correction_features would write from the density rho (float32
  *                      mesh), the potential phi (NULL: no potential channel) and their stats,
@@ -356,6 +359,8 @@ int pm_conv3d_bwd_data_out1(const float* dz0, const void* w, const float* gact, 
 int pm_conv3d_bwd_weight_workspace(const int32_t shape[3], int32_t cin, size_t* bytes);
 int pm_conv3d_bwd_weight(const float* dz, const void* x, int32_t cin, const int32_t shape[3], float* dw_db,
                          void* workspace, size_t workspace_bytes, void* stream);
+int pm_conv3d_bwd_weight_out1(const float* dz0, const void* x, const int32_t shape[3], float* dw_db, void* workspace,
+                              size_t workspace_bytes, void* stream);
 int pm_conv3d_stem(const float* rho, const float* phi, const int32_t shape[3], float omega_m, float a, float sigma8,
                    const float* stats, const void* w, const float* bias, void* act, void* stream);
 int pm_conv3d_out_residual(const void* x, const void* w, const float* bias, const float* rho,

@@ -74,9 +74,14 @@ def conv3d_bwd_data_out1(dz0, w, gact=None, dtype=torch.float32):
 def conv3d_bwd_weight(dz, x, out=None):
     """(dW (27, 16, C_in) float32, db (16,) float32) of a layer with input x.
 
-    ``out`` (optional) is a contiguous float32 tensor of 27*16*C_in + 16 elements that receives
-    [dW, db] in place (a slice of a flat gradient vector)."""
-    shape = _shape(dz)
+    ``dz`` is (X, Y, Z, 16), or (X, Y, Z) for a layer whose only output channel is channel 0 (the
+    other channels' gradients are zero; 16 input channels).  ``out`` (optional) is a contiguous
+    float32 tensor of 27*16*C_in + 16 elements that receives [dW, db] in place (a slice of a flat
+    gradient vector)."""
+    one = dz.ndim == 3
+    if one and int(x.shape[3]) != 16:
+        raise ValueError("a one-channel dz needs 16 input channels")
+    shape = tuple(int(s) for s in dz.shape) if one else _shape(dz)
     cin = int(x.shape[3])
     nbytes = _lib.size_query("pm_conv3d_bwd_weight_workspace", _lib.int3(shape), cin)
     ws = workspace(nbytes, dz.device)
@@ -84,6 +89,10 @@ def conv3d_bwd_weight(dz, x, out=None):
         out = torch.empty(27 * 16 * cin + 16, dtype=torch.float32, device=dz.device)
     elif out.numel() != 27 * 16 * cin + 16 or not out.is_contiguous() or out.dtype != torch.float32:
         raise ValueError("out must be a contiguous float32 tensor of 27*16*C_in + 16 elements")
-    _lib.call("pm_conv3d_bwd_weight", ptr(dz.contiguous()), ptr(x.contiguous()), cin, _lib.int3(shape), ptr(out),
-              ptr(ws), nbytes, stream_handle(dz.device))
+    if one:
+        _lib.call("pm_conv3d_bwd_weight_out1", ptr(dz.contiguous()), ptr(x.contiguous()), _lib.int3(shape), ptr(out),
+                  ptr(ws), nbytes, stream_handle(dz.device))
+    else:
+        _lib.call("pm_conv3d_bwd_weight", ptr(dz.contiguous()), ptr(x.contiguous()), cin, _lib.int3(shape), ptr(out),
+                  ptr(ws), nbytes, stream_handle(dz.device))
     return out[:-16].view(27, 16, cin), out[-16:]

@@ -379,8 +379,7 @@ def residual_backward(model: MeshCNNPotentialCorrection, tape: Tape, rho_cot, gr
     density cotangent (mesh) and ``omega_bar`` a device float (``pm_correction_input_bwd``).
     With ``input_grad`` it returns only the gradient of the network input x0's first four
     channels (a float32 (X, Y, Z, 4) mesh, what the input path reads); ``weights=False`` skips
-    the weight gradients (the output layer's gradient then stays one channel wide:
-    ``pm_conv3d_bwd_data_out1``)."""
+    the weight gradients."""
     dev = tape.rho.device
     n = tape.rho.numel()
     shape = tuple(tape.rho.shape)
@@ -391,12 +390,11 @@ def residual_backward(model: MeshCNNPotentialCorrection, tape: Tape, rho_cot, gr
     if rc.dtype != torch.float32 or tuple(rc.shape) != shape:
         raise ValueError("rho_cot must be a float32 mesh shaped like rho")
     ws = _workspace(dev)
-    # the output layer's weight gradient reads its 16-channel dz; without it one channel suffices
-    dz_ch = CHANNELS if weights else 1
-    dz = torch.empty(shape + ((CHANNELS,) if weights else ()), dtype=torch.float32, device=dev)
+    # the output layer has one live channel: its gradient stays one channel wide
+    dz = torch.empty(shape, dtype=torch.float32, device=dev)
     g = model.gain_offset if weights else 0
     _lib.call("pm_correction_residual_bwd", ptr(rc), ptr(tape.out), ptr(tape.rho), n, tape.omega_m, tape.a,
-              float(model.sigma8_value), float(model.max_residual), ptr(tape.stats), ptr(dz), dz_ch,
+              float(model.sigma8_value), float(model.max_residual), ptr(tape.stats), ptr(dz), 1,
               ptr(grads[g:g + 4]), ptr(ws), ws.numel(), stream_handle(dev))
     layers = model.layers
 
@@ -409,10 +407,7 @@ def residual_backward(model: MeshCNNPotentialCorrection, tape: Tape, rho_cot, gr
     # without the weight gradients, the pre-activation gradients only feed further data
     # gradients, whose matrix cores read them as bf16: they are stored as bf16
     gdt = torch.float32 if weights else torch.bfloat16
-    if weights:
-        dz = conv3d_bwd_data(dz, model.weight(layers[-1]), gact=tape.pres[-1])
-    else:
-        dz = conv3d_bwd_data_out1(dz, model.weight(layers[-1]), gact=tape.pres[-1], dtype=gdt)
+    dz = conv3d_bwd_data_out1(dz, model.weight(layers[-1]), gact=tape.pres[-1], dtype=gdt)
     for i in reversed(range(model.depth - 1)):
         if model.block == "plain":
             # dz is the gradient of block i's pre-activation; its input is acts[i] = gelu(pres[i])

@@ -1133,94 +1133,260 @@ __global__ void __launch_bounds__(kOThreads) k_conv_out1(const __bf16* __restric
 
 
 // Weight and bias gradients: dw[tap][co][ci] = sum_v dz[v][co] x[v + off(tap)][ci],
-// db[co] = sum_v dz[v][co].  A persistent grid walks the voxel blocks; each workgroup keeps
-// its partial sums in registers (MFMA accumulators, K = voxels) and writes them to
-// partial[blockIdx.x]; k_reduce_partials adds the partials in a fixed order.
-template <int CIN>
-__global__ void __launch_bounds__(kThreads) k_conv_bwd_weight(const float* __restrict__ dz,
-                                                              const __bf16* __restrict__ x, int n0, int n1, int n2,
-                                                              float* __restrict__ partial) {
-  // channel-major staging so the 8 voxels of an MFMA K group are contiguous along z
-  __shared__ __align__(16) __bf16 xs[CIN * kH * kH * kH];
-  __shared__ __align__(16) __bf16 gs[kCout * kVox];
-  __shared__ float bsum[kThreads / 64][kCout];
-  constexpr int NW = kTaps * kCout * CIN;  // weight gradients per workgroup
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int m = lane % 16, g = lane / 16;
-  // wave w owns taps w, w+4, ...: up to 7 taps, one 16x16 (co x ci) block each (CIN <= 16)
+// db[co] = sum_v dz[v][co], on MFMA with K = voxels: A[co][voxel] = bf16(dz), B[voxel][ci] = x.
+//
+// A lane's eight K elements must lie together in LDS and stay 16-byte aligned under the shift
+// of every tap.  So they are not eight neighbours along an axis but eight rows 8 apart: K element
+// j of a fragment is row y0 + 8 j + yb, and the tile is stored as vectors of those eight rows,
+// [channel][x plane][z][yb]; a tap then moves (z, yb) by whole vectors and each fragment is one
+// 16-byte read (eight 2-byte reads, of an unaligned z run, before).  The vectors are transposed
+// in registers while staging (one byte permute per output word).  Channel strides are 1 vector
+// modulo 16, so the 16 channels of a read fall on disjoint banks.
+//
+// A work item is a column of 64 y rows (eight runs of 8; runs past the mesh are zero) x 8 z, walked
+// along `seg` x planes with three staged x planes of x in a ring and the next plane's loads in
+// registers under the current plane's matrix work.  The 8 waves split the taps four ways and
+// the K steps two ways.  One workgroup per CU (95 KB of LDS); each keeps its sums in MFMA
+// accumulators over all of its items and writes one partial row, which k_reduce_partials adds
+// in a fixed order.  Bound by HBM (96 bytes per voxel and 1.56x halo of x): 416 -> 68 us for a
+// 16 -> 16 layer at 128^3 (2.9 TB/s of its 201 MB), 194 -> 49 us for the stem, 52 us with DZ1.  With CIN = 8 the
+// fragment's columns hold two taps' channels.  DZ1: dz has one channel (a one-output-channel layer): only output
+// channel 0's gradients are non-zero, and 4 instead of 64 bytes per voxel are read.
+constexpr int kWThreads = 512;
+constexpr int kWY = 8, kWZ = 8, kWJ = 8;           // yb positions, z extent, rows per vector
+constexpr int kWPos = (kWY + 2) * (kWZ + 2);       // staged x vectors per channel and plane
+constexpr int kWCsx = 3 * kWPos + 5;               // channel stride of the x ring (305 = 1 mod 16)
+constexpr int kWDz = kWY * kWZ;                    // staged dz vectors per channel
+constexpr int kWCsd = kWDz + 1;
+static_assert(kWCsx % 16 == 1 && kWCsd % 16 == 1, "channel strides: conflict-free fragment reads");
+
+template <int CIN, bool DZ1>
+__global__ void __launch_bounds__(kWThreads) k_conv_bwd_weight(const float* __restrict__ dz,
+                                                               const __bf16* __restrict__ x, int n0, int n1, int n2,
+                                                               int seg, int aligned, float* __restrict__ partial) {
   static_assert(CIN == 8 || CIN == 16, "CIN must be 8 or 16");
-  f32x4 acc[7];
+  constexpr int V = CIN / 8;               // 8-channel halves of a voxel of x
+  constexpr int NW = kTaps * kCout * CIN;  // weight gradients per workgroup
+  constexpr int TPS = 16 / CIN;            // taps per fragment (columns)
+  constexpr int SLOTS = (kTaps + TPS - 1) / TPS;
+  constexpr int NT = (SLOTS + 3) / 4;      // fragments per wave
+  constexpr int DCH = DZ1 ? 1 : kCout;
+  constexpr int XVEC = CIN * kWCsx, DVEC = DCH * kWCsd, RVEC = 4 * NT * 64;
+  __shared__ uint4 lds[XVEC + DVEC > RVEC ? XVEC + DVEC : RVEC];
+  __shared__ float bsum[kWThreads / 64][kCout];
+  uint4* xs = lds;
+  uint4* ds = lds + XVEC;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int m = lane % 16, g = lane / 16;
+  const int tg = wave % 4, kh = wave / 4;
+  f32x4 acc[NT];
+  int tbase[NT], tdx[NT];  // per fragment: vector offset of this lane's tap within a plane, its x plane
 #pragma unroll
-  for (int t = 0; t < 7; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bacc = 0.f;
-  const int nbz = n2 / kB, nby = n1 / kB, nblk = (n0 / kB) * nby * nbz;
-  for (int blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-    const int bz = blk % nbz, by = (blk / nbz) % nby, bx = blk / (nbz * nby);
-    const int ox = bx * kB, oy = by * kB, oz = bz * kB;
-    __syncthreads();
-    for (int it = threadIdx.x; it < kH * kH * kH * CIN; it += kThreads) {
-      const int c = it % CIN, vox = it / CIN;
-      const int z = vox % kH, y = (vox / kH) % kH, xx = vox / (kH * kH);
-      const int gx = wrap(ox + xx - 1, n0), gy = wrap(oy + y - 1, n1), gz = wrap(oz + z - 1, n2);
-      xs[c * kH * kH * kH + vox] = x[(((int64_t)gx * n1 + gy) * n2 + gz) * CIN + c];
+  for (int t = 0; t < NT; ++t) {
+    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int tap = min((tg + 4 * t) * TPS + m / CIN, kTaps - 1);  // clamped taps are not written out
+    tdx[t] = tap / 9;
+    tbase[t] = (m % CIN) * kWCsx + (4 * kh + tap % 3) * (kWY + 2) + (tap / 3) % 3 + g;
+  }
+  const int abase = (DZ1 ? 0 : m) * kWCsd + 4 * kh * kWY + g;
+  // staging roles: threads 0 .. 255 (DZ1: 0 .. 63) one vector position and channel quad of dz, the
+  // next 100 V one position and channel half of x
+  constexpr int DITEMS = DZ1 ? kWDz : 4 * kWDz;
+  const bool dzt = tid < DITEMS;
+  const int xi = tid - 256;
+  const bool xt = xi >= 0 && xi < kWPos * V;
+  const int quad = DZ1 ? 0 : tid % 4, dpos = DZ1 ? tid : tid / 4;
+  const int dyb = dpos / kWZ, dzz = dpos % kWZ;
+  const int half = xt ? xi % V : 0, xpos = xt ? xi / V : 0;
+  const int xyb = xpos / (kWZ + 2), xzz = xpos % (kWZ + 2);
+  typedef uint32_t Prefetch __attribute__((ext_vector_type(4 * kWJ)));  // a value, never a private array
+  float bacc[4] = {0.f, 0.f, 0.f, 0.f};
+  const int nzb = n2 / kWZ, nyb = (n1 + 63) / 64, nseg = (n0 + seg - 1) / seg;
+  const int nitems = nyb * nzb * nseg;
+  const int64_t plane = (int64_t)n1 * n2;
+  for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
+    const int col = item % (nyb * nzb), z0 = (col % nzb) * kWZ, y0 = (col / nzb) * 64;
+    const int x0 = (item / (nyb * nzb)) * seg, x1 = min(n0, x0 + seg);
+    // this thread's row offsets of its eight rows (invalid runs read row 0 and are zeroed)
+    typedef int Rows __attribute__((ext_vector_type(kWJ)));
+    Rows row;
+    const int zc = xt ? wrap(z0 + xzz - 1, n2) : z0 + dzz;
+#pragma unroll
+    for (int j = 0; j < kWJ; ++j) {
+      const bool live = y0 + 8 * j < n1;  // uniform
+      const int y = xt ? wrap(y0 + 8 * j + xyb - 1, n1) : y0 + 8 * j + dyb;
+      row[j] = (live ? y : 0) * n2 + zc;
     }
-    for (int it = threadIdx.x; it < kVox * kCout; it += kThreads) {
-      const int c = it % kCout, vox = it / kCout;
-      const int z = vox % kB, y = (vox / kB) % kB, xx = vox / (kB * kB);
-      const float v = dz[(((int64_t)(ox + xx) * n1 + (oy + y)) * n2 + (oz + z)) * kCout + c];
-      gs[c * kVox + vox] = (__bf16)v;
-      bacc += (threadIdx.x % kCout == c) ? v : 0.f;  // c == threadIdx.x % 16 since 256 % 16 == 0
-    }
-    __syncthreads();
-    // K step k covers voxels 32k .. 32k+31: x plane k/2, y rows 4*(k%2) .. +3, all 8 z
-#pragma unroll 1
-    for (int k = 0; k < kVox / 32; ++k) {
-      // lane group g covers voxels 32k + 8g .. +7: x plane k/2, y row 4*(k%2) + g, z 0..7
-      const int vx = k / 2, gy = 4 * (k % 2) + g;
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(gs + m * kVox + (vx * kB + gy) * kB);
+    auto load_x = [&](Prefetch& pf, int xp) {
+      const int64_t base = (int64_t)wrap(xp, n0) * plane;
 #pragma unroll
-      for (int t = 0; t < 7; ++t) {
-        const int tap = wave + 4 * t;
-        if (tap >= kTaps) break;
-        const int dx_ = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz_ = tap % 3 - 1;
-        // x[v + off]: staged voxel (vx+1+dx, gy+1+dy, z+1+dz), z = 0..7 contiguous
-        const int base = ((vx + 1 + dx_) * kH + (gy + 1 + dy)) * kH + (1 + dz_);
-        const int ci = m < CIN ? m : 0;  // CIN = 8: lanes 8..15 feed zero columns
-        bf16x8 b;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[j] = m < CIN ? xs[ci * kH * kH * kH + base + j] : (__bf16)0.f;
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+      for (int j = 0; j < kWJ; ++j) {
+        const __bf16* p = x + (base + row[j]) * CIN + 8 * half;
+        uint4 v;
+        if (aligned) {
+          v = *reinterpret_cast<const uint4*>(p);
+        } else {
+          const uint16_t* q = reinterpret_cast<const uint16_t*>(p);
+          v = make_uint4(q[0] | (uint32_t)q[1] << 16, q[2] | (uint32_t)q[3] << 16, q[4] | (uint32_t)q[5] << 16,
+                         q[6] | (uint32_t)q[7] << 16);
+        }
+        pf[4 * j] = v.x;
+        pf[4 * j + 1] = v.y;
+        pf[4 * j + 2] = v.z;
+        pf[4 * j + 3] = v.w;
       }
+    };
+    auto load_dz = [&](Prefetch& pf, int xp) {
+      const int64_t base = (int64_t)xp * plane;
+#pragma unroll
+      for (int j = 0; j < kWJ; ++j) {
+        const float* p = dz + (base + row[j]) * DCH + 4 * quad;
+        if constexpr (DZ1) {
+          pf[4 * j] = __float_as_uint(p[0]);
+        } else {
+          float4 v;
+          if (aligned)
+            v = *reinterpret_cast<const float4*>(p);
+          else
+            v = make_float4(p[0], p[1], p[2], p[3]);
+          pf[4 * j] = __float_as_uint(v.x);
+          pf[4 * j + 1] = __float_as_uint(v.y);
+          pf[4 * j + 2] = __float_as_uint(v.z);
+          pf[4 * j + 3] = __float_as_uint(v.w);
+        }
+      }
+    };
+    auto zero_dead = [&](Prefetch& pf) {
+#pragma unroll
+      for (int j = 0; j < kWJ; ++j) {
+        const bool live = y0 + 8 * j < n1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pf[4 * j + i] = live ? pf[4 * j + i] : 0u;
+      }
+    };
+    // eight rows x eight channels (bf16 pairs) -> eight vectors of eight rows
+    auto store_x = [&](Prefetch& pf, int slot) {
+      zero_dead(pf);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const uint32_t sel = c % 2 ? 0x07060302u : 0x05040100u;
+        uint32_t o[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = __builtin_amdgcn_perm(pf[4 * (2 * q + 1) + c / 2], pf[4 * (2 * q) + c / 2], sel);
+        xs[(8 * half + c) * kWCsx + slot * kWPos + xzz * (kWY + 2) + xyb] = make_uint4(o[0], o[1], o[2], o[3]);
+      }
+    };
+    auto store_dz = [&](Prefetch& pf) {
+      zero_dead(pf);
+#pragma unroll
+      for (int c = 0; c < (DZ1 ? 1 : 4); ++c) {
+        bf16x8 o;
+#pragma unroll
+        for (int j = 0; j < kWJ; ++j) {
+          const float v = __uint_as_float(pf[4 * j + c]);
+          bacc[c] += v;
+          o[j] = (__bf16)v;
+        }
+        ds[(4 * quad + c) * kWCsd + dzz * kWY + dyb] = __builtin_bit_cast(uint4, o);
+      }
+    };
+    Prefetch pf;
+    __syncthreads();  // the previous item's last plane is done with the tiles
+    if (xt) {
+      load_x(pf, x0 - 1);
+      store_x(pf, 0);
+      load_x(pf, x0);
+      store_x(pf, 1);
+      load_x(pf, x0 + 1);
+    } else if (dzt) {
+      load_dz(pf, x0);
+    }
+    int s0 = 0;  // ring slot of plane xp - 1
+    for (int xp = x0; xp < x1; ++xp) {
+      const int s1 = s0 == 2 ? 0 : s0 + 1, s2 = s1 == 2 ? 0 : s1 + 1;
+      if (xp > x0) __syncthreads();  // the previous plane's fragments are read
+      if (xt) {
+        store_x(pf, s2);
+        load_x(pf, xp + 2);  // one plane past the last is loaded and not used (wrapped: in bounds)
+      } else if (dzt) {
+        store_dz(pf);
+        load_dz(pf, min(xp + 1, x1 - 1));
+      }
+      __syncthreads();
+      int off[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) off[t] = tbase[t] + kWPos * (tdx[t] == 0 ? s0 : (tdx[t] == 1 ? s1 : s2));
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {  // K step: z = 4 kh + k / 2, yb = 4 (k % 2) + g, eight rows each
+        uint4 av = ds[abase + (k / 2) * kWY + 4 * (k % 2)];
+        if constexpr (DZ1) {
+          if (m != 0) av = make_uint4(0u, 0u, 0u, 0u);
+        }
+        const bf16x8 a = __builtin_bit_cast(bf16x8, av);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const bf16x8 b = __builtin_bit_cast(bf16x8, xs[off[t] + (k / 2) * (kWY + 2) + 4 * (k % 2)]);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+        }
+      }
+      s0 = s1;
     }
   }
-  // bias partials: lanes with the same channel (threadIdx.x % 16) are summed per wave
-  for (int off = 16; off < 64; off <<= 1) bacc += __shfl_xor(bacc, off);
-  if (lane < 16) bsum[wave][lane] = bacc;
+  // bias: this thread's channels 4 quad .. 4 quad + 3 (DZ1: channel 0) over the threads of a wave,
+  // then the waves in order
+#pragma unroll
+  for (int c = 0; c < (DZ1 ? 1 : 4); ++c) {
+    float v = dzt ? bacc[c] : 0.f;
+    for (int off = DZ1 ? 1 : 4; off < 64; off <<= 1) v += __shfl_xor(v, off);
+    if (lane < (DZ1 ? 1 : 4)) bsum[wave][4 * lane + c] = v;
+  }
+  // the two halves of the K steps: waves 4 .. 7 hand their sums to waves 0 .. 3
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
+  if (kh == 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) red[(tg * NT + t) * 64 + lane] = acc[t];
+  }
   __syncthreads();
   float* out = partial + (int64_t)blockIdx.x * (NW + kCout);
-  // acc[t][cb] lane holds rows co = 4g+i, column ci = cb*16 + m
+  if (kh == 0) {
+    // the lane holds rows co = 4 g + i of its column: tap slot m / CIN, input channel m % CIN
 #pragma unroll
-  for (int t = 0; t < 7; ++t) {
-    const int tap = wave + 4 * t;
-    if (tap >= kTaps) break;
-    if (m < CIN) {
+    for (int t = 0; t < NT; ++t) {
+      const int tap = (tg + 4 * t) * TPS + m / CIN;
+      if (tap >= kTaps) continue;
+      const f32x4 v = acc[t] + red[(tg * NT + t) * 64 + lane];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[(tap * kCout + 4 * g + i) * CIN + m] = acc[t][i];
+      for (int i = 0; i < 4; ++i) out[(tap * kCout + 4 * g + i) * CIN + m % CIN] = v[i];
     }
   }
-  if (threadIdx.x < kCout) {
+  if (tid < kCout) {
     float b = 0.f;
-    for (int w2 = 0; w2 < kThreads / 64; ++w2) b += bsum[w2][threadIdx.x];
-    out[NW + threadIdx.x] = b;
+    if (!DZ1 || tid == 0)
+      for (int w2 = 0; w2 < (DZ1 ? 1 : 4); ++w2) b += bsum[w2][tid];  // the waves with dz threads
+    out[NW + tid] = b;
   }
 }
 
-// sum over partial rows in a fixed order: out[i] = sum_r partial[r][i]
-__global__ void k_reduce_partials(const float* __restrict__ partial, int rows, int width, float* __restrict__ out) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < width; i += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int r = 0; r < rows; ++r) s += partial[(int64_t)r * width + i];
-    out[i] = s;
+// out[i] = sum_r partial[r][i] in a fixed order: a workgroup takes 64 columns, its 16 waves a
+// stride of rows each: 5 us for 256 rows of 6928 (a thread walking all rows alone took 240 us for
+// 1024 rows: one dependent read after the other)
+constexpr int kRedThreads = 1024;
+__global__ void __launch_bounds__(kRedThreads) k_reduce_partials(const float* __restrict__ partial, int rows, int width,
+                                                                 float* __restrict__ out) {
+  __shared__ float part[kRedThreads / 64][64];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int i = min((int)blockIdx.x * 64 + lane, width - 1);
+  float s = 0.f;
+#pragma unroll 4
+  for (int r = wave; r < rows; r += kRedThreads / 64) s += partial[(int64_t)r * width + i];
+  part[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && blockIdx.x * 64 + lane < width) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < kRedThreads / 64; ++w) t += part[w][lane];
+    out[i] = t;
   }
 }
 
@@ -1307,7 +1473,22 @@ int launch_out1(const __bf16* x, const __bf16* w, const float* bias, float* pre,
 
 bool out1_blocks(const int32_t* shape) { return shape[0] % conv::kOBX == 0 && shape[2] % conv::kOBZ == 0; }
 
-constexpr int kWGrid = 1024;  // persistent workgroups of the weight-gradient pass
+constexpr int kWGrid = 256;  // persistent workgroups of the weight-gradient pass: one per CU
+
+// x planes per work item of the weight-gradient pass: whole x lines when the (y, z) columns
+// alone are enough items for the grid, else halved (down to 4 planes, where the two halo planes of
+// an item cost half as much again) until they are
+int weight_segment(const int32_t* shape) {
+  const int64_t cols = ceil_div(shape[1], 64) * (shape[2] / conv::kWZ);
+  int seg = shape[0];
+  while (seg > 4 && cols * ceil_div(shape[0], seg) < kWGrid) seg = (seg + 1) / 2;
+  return seg;
+}
+
+unsigned weight_grid(const int32_t* shape) {
+  const int64_t items = ceil_div(shape[1], 64) * (shape[2] / conv::kWZ) * ceil_div(shape[0], weight_segment(shape));
+  return (unsigned)std::min<int64_t>(items, kWGrid);
+}
 
 }  // namespace
 
@@ -1503,33 +1684,44 @@ int pm_conv3d_bwd_weight_workspace(const int32_t shape[3], int32_t cin, size_t* 
   PM_TRY(check_shape(shape));
   PM_RETURN_IF(cin != 8 && cin != 16, PM_ERROR_UNSUPPORTED, "conv3d input channels must be 8 or 16");
   PM_RETURN_IF(bytes == nullptr, PM_ERROR_INVALID_ARGUMENT, "bytes is NULL");
-  const int64_t grid = std::min<int64_t>(nblocks(shape), kWGrid);
-  *bytes = sizeof(float) * grid * (conv::kTaps * conv::kCout * cin + conv::kCout);
+  *bytes = sizeof(float) * weight_grid(shape) * (conv::kTaps * conv::kCout * cin + conv::kCout);
+  return PM_SUCCESS;
+}
+
+static int bwd_weight(const float* dz, bool one_channel, const void* x, int32_t cin, const int32_t shape[3],
+                      float* dw_db, void* workspace, size_t workspace_bytes, void* stream) {
+  size_t need = 0;
+  PM_TRY(pm_conv3d_bwd_weight_workspace(shape, cin, &need));
+  PM_RETURN_IF(dz == nullptr || x == nullptr || dw_db == nullptr, PM_ERROR_INVALID_ARGUMENT, "NULL argument");
+  PM_RETURN_IF(workspace == nullptr || workspace_bytes < need, PM_ERROR_WORKSPACE, "conv3d workspace too small");
+  PM_RETURN_IF((int64_t)shape[1] * shape[2] >= (int64_t(1) << 31), PM_ERROR_UNSUPPORTED,
+               "conv3d: mesh too large for 32-bit row offsets");
+  hipStream_t s = as_stream(stream);
+  const unsigned grid = weight_grid(shape);
+  const int seg = weight_segment(shape);
+  const int aligned = ((reinterpret_cast<uintptr_t>(dz) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
+  float* partial = static_cast<float*>(workspace);
+  const __bf16* xb = static_cast<const __bf16*>(x);
+  auto kern = one_channel ? conv::k_conv_bwd_weight<16, true>
+                          : (cin == 8 ? conv::k_conv_bwd_weight<8, false> : conv::k_conv_bwd_weight<16, false>);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(conv::kWThreads), 0, s, dz, xb, shape[0], shape[1], shape[2], seg,
+                     aligned, partial);
+  PM_LAUNCHED("k_conv_bwd_weight", s);
+  const int width = conv::kTaps * conv::kCout * cin + conv::kCout;
+  hipLaunchKernelGGL(conv::k_reduce_partials, dim3((unsigned)ceil_div(width, 64)), dim3(conv::kRedThreads), 0, s,
+                     partial, (int)grid, width, dw_db);
+  PM_LAUNCHED("k_reduce_partials", s);
   return PM_SUCCESS;
 }
 
 int pm_conv3d_bwd_weight(const float* dz, const void* x, int32_t cin, const int32_t shape[3], float* dw_db,
                          void* workspace, size_t workspace_bytes, void* stream) {
-  size_t need = 0;
-  PM_TRY(pm_conv3d_bwd_weight_workspace(shape, cin, &need));
-  PM_RETURN_IF(dz == nullptr || x == nullptr || dw_db == nullptr, PM_ERROR_INVALID_ARGUMENT, "NULL argument");
-  PM_RETURN_IF(workspace == nullptr || workspace_bytes < need, PM_ERROR_WORKSPACE, "conv3d workspace too small");
-  hipStream_t s = as_stream(stream);
-  const unsigned grid = (unsigned)std::min<int64_t>(nblocks(shape), kWGrid);
-  float* partial = static_cast<float*>(workspace);
-  const __bf16* xb = static_cast<const __bf16*>(x);
-  if (cin == 8)
-    hipLaunchKernelGGL(conv::k_conv_bwd_weight<8>, dim3(grid), dim3(conv::kThreads), 0, s, dz, xb, shape[0],
-                       shape[1], shape[2], partial);
-  else
-    hipLaunchKernelGGL(conv::k_conv_bwd_weight<16>, dim3(grid), dim3(conv::kThreads), 0, s, dz, xb, shape[0],
-                       shape[1], shape[2], partial);
-  PM_LAUNCHED("k_conv_bwd_weight", s);
-  const int width = conv::kTaps * conv::kCout * cin + conv::kCout;
-  hipLaunchKernelGGL(conv::k_reduce_partials, dim3((unsigned)ceil_div(width, 256)), dim3(256), 0, s, partial,
-                     (int)grid, width, dw_db);
-  PM_LAUNCHED("k_reduce_partials", s);
-  return PM_SUCCESS;
+  return bwd_weight(dz, false, x, cin, shape, dw_db, workspace, workspace_bytes, stream);
+}
+
+int pm_conv3d_bwd_weight_out1(const float* dz0, const void* x, const int32_t shape[3], float* dw_db, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+  return bwd_weight(dz0, true, x, 16, shape, dw_db, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

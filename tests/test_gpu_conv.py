@@ -168,3 +168,34 @@ def test_one_channel_output_layer_matches_torch(device, shape):
     ref = _ref_conv(x, w, b)[..., 0]
     scale = ref.abs().max().item()
     np.testing.assert_allclose(pre1[..., 0].cpu().numpy(), ref.numpy(), atol=1e-4 * scale)
+
+
+@pytest.mark.parametrize("cin,one", [(16, False), (8, False), (16, True)])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (24, 72, 16), (40, 64, 8), (8, 136, 24), (264, 64, 8)])
+def test_weight_gradient_tile_edges(device, cin, one, shape):
+    """y extents of one run of 8 rows, whole 64-row columns and ragged ones, x lines cut into
+    segments of 4 planes and up, one and many columns; 16-byte aligned and unaligned inputs (the
+    same bits); a one-channel dz equals the 16-channel one with channel 0 live.  Products of bf16
+    values are exact, so only the order of the float32 sums differs: 1e-4 of the output scale."""
+    g = torch.Generator().manual_seed(cin + sum(shape))
+    x = _bf(torch.randn(shape + (cin,), generator=g))
+    dz = _bf(torch.randn(shape + (16,), generator=g))
+    if one:
+        dz[..., 1:] = 0
+    xd, dd = x.to(device, torch.bfloat16), dz.to(device)
+    src = dd[..., 0].contiguous() if one else dd
+    dw, db = conv3d_bwd_weight(src, xd)
+    flat = dz.double().reshape(-1, 16)
+    offs = [(a, b, c) for a in (-1, 0, 1) for b in (-1, 0, 1) for c in (-1, 0, 1)]
+    ref = torch.stack([flat.T @ torch.roll(x.double(), tuple(-o for o in off), (0, 1, 2)).reshape(-1, cin)
+                       for off in offs])
+    scale = ref.abs().max().item()
+    np.testing.assert_allclose(dw.cpu().double().numpy(), ref.numpy(), atol=1e-4 * scale)
+    np.testing.assert_allclose(db.cpu().double().numpy(), flat.sum(0).numpy(), atol=1e-4 * scale)
+    # inputs that are not 16-byte aligned take element loads: the same sums bit for bit
+    ux = torch.empty(xd.numel() + 1, dtype=xd.dtype, device=device)[1:].view(xd.shape)
+    uz = torch.empty(src.numel() + 1, dtype=src.dtype, device=device)[1:].view(src.shape)
+    ux.copy_(xd)
+    uz.copy_(src)
+    dw2, db2 = conv3d_bwd_weight(uz, ux)
+    assert torch.equal(dw2, dw) and torch.equal(db2, db)
