@@ -50,7 +50,7 @@ def kernel_step_bytes(name, L, n_p, brick):
     R = real float32 mesh; S1 / S2 = the complex64 spectrum band the force passes keep
     (kz < nkz; all y rows / the packed |ky| band), pitch excluded; n_p particles of 18 B
     (int16 pmid + float32 disp).  The tiled scatter hands the upper x/y planes of each brick
-    column to the fold; tile reads of the gather count the mesh once.
+    column to the r2c pass, which adds them; tile reads of the gather count the mesh once.
     """
     R = 4 * L["nreal"]
     Ch = 8 * L["nx"] * L["ny"] * (L["nz"] // 2 + 1)
@@ -60,20 +60,17 @@ def kernel_step_bytes(name, L, n_p, brick):
     b0, b1, b2 = brick
     nb0, nb1 = L["nx"] // b0, L["ny"] // b1
     planes = 4 * nb0 * nb1 * (b1 + 1 + b0) * L["nz"]  # upper x/y planes of every brick column
-    fold = 8 * (nb0 * L["ny"] + (L["nx"] - nb0) * nb1) * L["nz"]  # lower x/y plane cells read + written
     table = {
-        "fft_z_r2c": R + S1,
+        "fft_z_r2c": R + planes + S1,
         "fft_cols_fwd": S1 + S2,
         "fft_cols_green": 3 * S2,
-        "fft_cols_inv2": S2 + 2 * S1,
-        "fft_cols_inv": S2 + S1,
+        "fft_cols_inv3": 2 * S2 + 3 * S1,
         "fft_z_c2r": 3 * (S1 + R),
         "k_bucket_count": 18 * n_p,
         "k_bucket_place": (18 + 4 + 18 + 1) * n_p,
         "k_zero_i32": 4 * (nb + 2),
         "scan": 8 * (nb + 2),
         "k_scatter_columns": 18 * n_p + R + planes,
-        "k_fold_xy": planes + fold,
         "k_gather_columns": (18 + 4 + 12) * n_p + 3 * R,
         "k_fill": R,
         "k_scatter_sorted": 19 * n_p + R,

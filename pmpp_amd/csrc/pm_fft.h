@@ -324,28 +324,42 @@ struct ColPass {
   // expand the band to full rows, the rows outside it are zero), 0 = output (forward passes).
   int keep = -1, compact_in = 0;
   int ky_split = 0x7fffffff, ky_shift = 0;
-  // kColAdj: the y and z components' spectra (in is the x component's)
+  // kColAdj: the y and z components' spectra (in is the x component's); kColInv3: the input of
+  // the third output
   const float2* in1 = nullptr;
   const float2* in2 = nullptr;
+  float2* out2 = nullptr;  // kColInv3: the third output
 };
 
 // kColAdj: the x pass of the force step's spectral adjoint: forward transforms of the three
 // cotangent spectra, out = mask * (-1/k^2) * sum_i conj(D_i) in_i, inverse transform
 // kColPot: x forward, mask * (-1/k^2), x inverse (the potential, one output)
-enum ColMode { kColFwd = 0, kColInv = 1, kColInv2 = 2, kColGreen = 3, kColAdj = 4, kColPot = 5 };
+// kColInv3: the y inverses of the three force components in one launch: out0 <- in, out1 <- D in,
+// out2 <- in1
+enum ColMode { kColFwd = 0, kColInv = 1, kColInv3 = 2, kColGreen = 3, kColAdj = 4, kColPot = 5 };
 
-// Line pass along the contiguous last axis (real <-> half spectrum, split main + Nyquist).
+// Upper x/y planes of the brick columns of a tiled scatter (pm_gravity.hip), which the R2C pass adds
+// to the lower planes of the neighbouring columns while it reads the mesh: extents of the
+// mesh's y axis and of a brick as log2, brick columns per axis.
+struct FoldPlanes {
+  const float* xs = nullptr;
+  const float* ys = nullptr;
+  int ny_log = 0, b0_log = 0, b1_log = 0, nb0 = 0, nb1 = 0;
+};
+
+// Line pass along the contiguous last axis (real <-> half spectrum).  C2R takes up to three
+// (spectrum, output) pairs in one launch; R2C reads rin into cmain[0].
 struct ZPass {
   const float* rin;    // R2C: real input rows (pitch_r floats)
-  float* rout;         // C2R: real output rows
-  float2* cmain;       // spectrum rows kz in [0, M) (pitch_c float2)
-  float2* cnyq;        // Nyquist kz = M, one float2 per row at stride nyq_stride
-  int64_t pitch_r, pitch_c, nyq_stride;
+  float* rout[3];      // C2R: real output rows
+  float2* cmain[3];    // spectrum rows kz in [0, M], the Nyquist column last (pitch_c float2)
+  int ncomp = 1;       // C2R: pairs
+  int64_t pitch_r, pitch_c;
   int64_t nlines;
   float src_shift;  // R2C pre-op: (x + src_shift) * src_scale
   float src_scale;
   float out_scale;  // C2R: output scale
-  int deriv;        // C2R pre-op: multiply by i*negk_z[k] when nonzero
+  int deriv;        // C2R pre-op: bit c set: pair c is multiplied by i*negk_z[k]
   // band of stored spectrum columns: R2C stores kz < kz_lim (and the Nyquist column only when
   // nyq != 0); C2R reads them and takes every other column, the Nyquist one included when
   // nyq == 0, as zero
@@ -353,6 +367,8 @@ struct ZPass {
   int nyq = 1;
   // R2C: optional second real input (same layout) added before the pre-op
   const float* rin_add = nullptr;
+  // R2C: optional plane buffers of a tiled scatter, folded into rin on load
+  FoldPlanes fold;
   // C2R: optional real mesh (same layout as rout, may alias it) added to the scaled output
   const float* rout_add = nullptr;
 };

@@ -1,5 +1,6 @@
 // FFT passes (real<->half-spectrum along z, complex along y/x) and the fused spectral
 // force passes of the PM step.  See pm_fft.h for the decomposition.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <mutex>
@@ -63,10 +64,10 @@ namespace fft {
 namespace {
 
 // ----------------------------------------------------------- column passes ----
-// T adjacent columns per workgroup.  The y inverse with two outputs (kColInv2) runs two
-// workgroups per tile (HALVES), each of which loads the same input tile (the second read is
-// served by L2: the pair runs on one XCD at nearly the same time) and inverts one of the two
-// outputs, so no thread keeps both spectra live.  The x Green pass (kColGreen) runs one
+// T adjacent columns per workgroup.  The y inverse of the three force components (kColInv3) runs
+// three workgroups per tile (HALVES), one per output; the first two load the same input tile (the
+// second read is served by L2: they run on one XCD at nearly the same time), so no thread
+// keeps two spectra live.  The x Green pass (kColGreen) runs one
 // workgroup per tile that parks its multiplied spectrum in its first output between the two
 // inverses.  Outputs of two-output passes must not alias the input or each other.
 template <int N, int T, int HALVES>
@@ -164,18 +165,19 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
     for (int s = 0; s < E; ++s) v[s] = io.in[ibase + (int64_t)(nrow<N>(p, s) - p) * io.s_row];
     forward_core<N>(v, my, p, idx, tw);
   } else {
+    const float2* src = MODE == kColInv3 && half == 2 ? io.in1 : io.in;  // uniform
     if (keep >= 0 && io.compact_in) {  // packed band in, zero outside it
 #pragma unroll
       for (int s = 0; s < E; ++s) {
         int k = xrow<N>(p, s);
-        v[s] = io.in[lbase + (int64_t)(in_band(k) ? packed(k) : 0) * io.s_row];
+        v[s] = src[lbase + (int64_t)(in_band(k) ? packed(k) : 0) * io.s_row];
       }
 #pragma unroll
       for (int s = 0; s < E; ++s)
         if (!in_band(xrow<N>(p, s))) v[s] = make_float2(0.f, 0.f);
     } else {
 #pragma unroll
-      for (int s = 0; s < E; ++s) v[s] = io.in[ibase + (int64_t)(xrow<N>(p, s) - p) * io.s_row];
+      for (int s = 0; s < E; ++s) v[s] = src[ibase + (int64_t)(xrow<N>(p, s) - p) * io.s_row];
     }
   }
 
@@ -233,7 +235,7 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
         for (int s = 0; s < E; ++s)
           v[s] = cok ? io.out0[obp + (int64_t)(nrow<N>(p, s) - p) * o_row] : make_float2(0.f, 0.f);
       }
-    } else if constexpr (MODE == kColInv2) {
+    } else if constexpr (MODE == kColInv3) {
       if (half == 1) {
 #pragma unroll
         for (int s = 0; s < E; ++s) v[s] = c_imul(tb.negk[dax][xrow<N>(p, s)], v[s]);
@@ -242,7 +244,7 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
     // after a forward transform in the same kernel (kColGreen, kColPot) the inverse's twiddles
     // are loaded afresh instead of kept live from the forward
     inverse_core<N>(v, my, p, idx, (MODE == kColGreen || MODE == kColPot) ? fresh_table(tw) : tw);
-    float2* out = (half == 1) ? io.out1 : io.out0;
+    float2* out = (half == 1) ? io.out1 : (half == 2 ? io.out2 : io.out0);
     if (cok) {
 #pragma unroll
       for (int s = 0; s < E; ++s) out[obp + (int64_t)(nrow<N>(p, s) - p) * o_row] = v[s];
@@ -272,8 +274,8 @@ struct ZCfg {
   static constexpr int LDS_FLOATS = LINES * LSTR;
 };
 
-// ADD (C2R only): the output is rout_add + the scaled line (a separate instantiation, so the
-// force step's c2r keeps its register budget)
+// ADD: C2R: the output is rout_add + the scaled line; R2C: rin's planes are folded on load
+// (ZPass::fold).  Separate instantiations, so the plain passes keep their register budget.
 template <int M, bool C2R, bool ADD = false>
 __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, SpecTables tb,
                                                                  const float2* __restrict__ tw) {
@@ -295,6 +297,52 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
     const float* src = zp.rin + lgl * zp.pitch_r;
 #pragma unroll
     for (int s = 0; s < E; ++s) v[s] = *reinterpret_cast<const float2*>(src + 2 * nrow<M>(p, s));
+    if constexpr (ADD) {
+      // a cell with lx = x mod b0 and ly = y mod b1 takes, from its neighbouring columns (periodic),
+      //   lx == 0: XS of column (cx-1, cy) row ly; and when ly == 0 also XS of (cx-1, cy-1) row b1
+      //            and YS of (cx, cy-1) row 0
+      //   ly == 0: YS of column (cx, cy-1) row lx
+      // summed in this order before they are added.  Reading them here saves the pass that
+      // would add them in place (1024^3: 1.67 + 0.54 ms for the two passes, 2.03 ms for this one;
+      // 512^3: 223 + 80 us, 253 us; 256^3: 37 + 11 us, 40 us).
+      const FoldPlanes& fp = zp.fold;
+      const int x = (int)(lgl >> fp.ny_log), y = (int)(lgl & ((1 << fp.ny_log) - 1));
+      const int lx = x & ((1 << fp.b0_log) - 1), ly = y & ((1 << fp.b1_log) - 1);
+      if (lx == 0 || ly == 0) {
+        const int cx = x >> fp.b0_log, cy = y >> fp.b1_log;
+        const int sx = cx == 0 ? fp.nb0 - 1 : cx - 1, sy = cy == 0 ? fp.nb1 - 1 : cy - 1;
+        const int64_t b0 = int64_t(1) << fp.b0_log, b1 = int64_t(1) << fp.b1_log;
+        auto xs_line = [&](int ccy, int64_t row) {
+          return fp.xs + (((int64_t)sx * fp.nb1 + ccy) * (b1 + 1) + row) * zp.pitch_r;
+        };
+        const float* ysl = fp.ys + (((int64_t)cx * fp.nb1 + sy) * b0 + lx) * zp.pitch_r;
+        const float* p0 = lx == 0 ? xs_line(cy, ly) : ysl;
+        float2 w[E];
+#pragma unroll
+        for (int s = 0; s < E; ++s) w[s] = *reinterpret_cast<const float2*>(p0 + 2 * nrow<M>(p, s));
+        if (lx == 0 && ly == 0) {
+          // four slots at a time: all at once, the loads would be issued one by one for want of
+          // registers, and the few corner lines would hold up the whole pass (35 % at 1024^3)
+          const float* p1 = xs_line(sy, b1);
+          constexpr int Q = E < 4 ? E : 4;
+#pragma unroll
+          for (int c = 0; c < E; c += Q) {
+            float2 a[Q], b[Q];
+#pragma unroll
+            for (int s = 0; s < Q; ++s) {
+              a[s] = *reinterpret_cast<const float2*>(p1 + 2 * nrow<M>(p, c + s));
+              b[s] = *reinterpret_cast<const float2*>(ysl + 2 * nrow<M>(p, c + s));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < Q; ++s) w[c + s] = c_add(c_add(w[c + s], a[s]), b[s]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < E; ++s) v[s] = c_add(v[s], w[s]);
+      }
+    }
     if (zp.rin_add) {  // uniform: the added field's loads join the same batch
       const float* src2 = zp.rin_add + lgl * zp.pitch_r;
 #pragma unroll
@@ -310,7 +358,7 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
 #pragma unroll
     for (int s = 0; s < E; ++s) nat[xrow<M>(p, s)] = v[s];
     __syncthreads();
-    float2* dst = zp.cmain + lg * zp.pitch_c;
+    float2* dst = zp.cmain[0] + lg * zp.pitch_c;
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       int k = p + P * j;
@@ -324,12 +372,13 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
     }
     if (ok && p == 0 && zp.nyq) {
       float2 z0 = nat[0];
-      zp.cnyq[lg * zp.nyq_stride] = make_float2(z0.x - z0.y, 0.f);
+      dst[M] = make_float2(z0.x - z0.y, 0.f);
     }
   } else {
     (void)nat;
-    const float2* srcm = zp.cmain + lgl * zp.pitch_c;
-    float2 xn = zp.cnyq[lgl * zp.nyq_stride];  // cnyq is a valid address even when nyq == 0
+    const int comp = blockIdx.y;
+    const float2* srcm = zp.cmain[comp] + lgl * zp.pitch_c;
+    float2 xn = srcm[zp.nyq ? M : 0];  // unconditional: column 0 stands in when there is none
     const int klim = zp.kz_lim < M ? zp.kz_lim : M;
 #pragma unroll
     for (int j = 0; j < E; ++j)  // P*j < klim is uniform: columns past the band cost no load
@@ -338,7 +387,7 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
     for (int j = 0; j < E; ++j)
       if (p + P * j >= klim) v[j] = make_float2(0.f, 0.f);
     if (!zp.nyq) xn = make_float2(0.f, 0.f);
-    if (zp.deriv) {
+    if ((zp.deriv >> comp) & 1) {
 #pragma unroll
       for (int j = 0; j < E; ++j) v[j] = c_imul(tb.negk[2][p + P * j], v[j]);
       xn = c_imul(tb.negk[2][M], xn);
@@ -376,7 +425,7 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
     __syncthreads();
     inverse_core<M>(v, lds, p, idx, tw);
     if (ok) {
-      float* dst = zp.rout + lg * zp.pitch_r;
+      float* dst = zp.rout[comp] + lg * zp.pitch_r;
       if constexpr (ADD) {
         const float* add = zp.rout_add + lg * zp.pitch_r;
 #pragma unroll
@@ -400,7 +449,11 @@ __global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, Spe
 // float (numerics/fft.py:30-41), the particle-Nyquist masks (core/utils.py:33-37) and
 // negk with the derivative zeroed at the mesh Nyquist (configuration.py:369-376), all
 // decided in float32 like the reference.
-__global__ void k_spec_tables(float* out, int n0, int n1, int n2, SpecTables sc) {
+// Also clears `zero` (counters of the step that follows on the stream: one launch less).
+__global__ void k_spec_tables(float* out, int n0, int n1, int n2, SpecTables sc, int32_t* __restrict__ zero,
+                              int64_t nzero) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nzero; i += (int64_t)gridDim.x * blockDim.x)
+    zero[i] = 0;
   int n[3] = {n0, n1, n2};
   int len[3] = {n0, n1, n2 / 2 + 1};
   int off = 0;
@@ -448,7 +501,10 @@ int launch_cols_cfg(const ColPass& cp, int batches, const SpecTables& tb, int da
   const int64_t tiles = (int64_t)gx * batches;
   const int64_t g = ceil_div(tiles * HALVES, 8) * 8;
   PM_RETURN_IF((HALVES > 1 || MODE == kColGreen) && (cp.in == cp.out0 || cp.in == cp.out1 || cp.out0 == cp.out1),
-               PM_ERROR_INVALID_ARGUMENT, "two-output FFT passes need outputs distinct from their input");
+               PM_ERROR_INVALID_ARGUMENT, "FFT passes with several outputs need them distinct from their input");
+  PM_RETURN_IF(MODE == kColInv3 && (cp.in1 == cp.out0 || cp.in1 == cp.out1 || cp.in1 == cp.out2 || cp.in == cp.out2 ||
+                                    cp.out0 == cp.out2 || cp.out1 == cp.out2),
+               PM_ERROR_INVALID_ARGUMENT, "FFT passes with several outputs need them distinct from their inputs");
   PM_RETURN_IF(g > INT32_MAX, PM_ERROR_UNSUPPORTED, "too many FFT column tiles");
   hipLaunchKernelGGL((k_cols<N, T, MODE, HALVES>), dim3((unsigned)g), dim3(CF::THREADS), 0, s, cp, tb, dax, tw,
                      gx, batches, (int)(g / 8));
@@ -461,11 +517,11 @@ template <int N>
 int launch_cols_n(int mode, const ColPass& cp, int batches, const SpecTables& tb, int dax,
                   hipStream_t s) {
   constexpr int T1 = (N >= 512) ? 8 : 16;  // one-output passes: 64 or 128-byte row segments
-  constexpr int T2 = (N >= 2048) ? 4 : 8;   // two-output passes: two workgroups of T2 columns per tile
+  constexpr int T2 = (N >= 2048) ? 4 : 8;   // passes with several outputs
   switch (mode) {
     case kColFwd: return launch_cols_cfg<N, T1, kColFwd, 1>(cp, batches, tb, dax, s, "fft_cols_fwd");
     case kColInv: return launch_cols_cfg<N, T1, kColInv, 1>(cp, batches, tb, dax, s, "fft_cols_inv");
-    case kColInv2: return launch_cols_cfg<N, T2, kColInv2, 2>(cp, batches, tb, dax, s, "fft_cols_inv2");
+    case kColInv3: return launch_cols_cfg<N, T2, kColInv3, 3>(cp, batches, tb, dax, s, "fft_cols_inv3");
     case kColGreen: return launch_cols_cfg<N, T2, kColGreen, 1>(cp, batches, tb, dax, s, "fft_cols_green");
     case kColAdj: return launch_cols_cfg<N, T1, kColAdj, 1>(cp, batches, tb, dax, s, "fft_cols_adjoint");
     case kColPot: return launch_cols_cfg<N, T2, kColPot, 1>(cp, batches, tb, dax, s, "fft_cols_potential");
@@ -481,7 +537,7 @@ int launch_z_n(bool c2r, const ZPass& zp, const SpecTables& tb, hipStream_t s) {
   PM_RETURN_IF(tw == nullptr, PM_ERROR_HIP, "twiddle table not initialised");
   if (zp.nlines == 0) return PM_SUCCESS;
   if (c2r) {
-    const dim3 grid((unsigned)ceil_div(zp.nlines, ZI::LINES));
+    const dim3 grid((unsigned)ceil_div(zp.nlines, ZI::LINES), (unsigned)zp.ncomp);
     if (zp.rout_add) {
       hipLaunchKernelGGL((k_zpass<M, true, true>), grid, dim3(ZI::THREADS), 0, s, zp, tb, tw);
       PM_LAUNCHED("fft_z_c2r_add", s);
@@ -491,7 +547,10 @@ int launch_z_n(bool c2r, const ZPass& zp, const SpecTables& tb, hipStream_t s) {
     }
   } else {
     const dim3 grid((unsigned)ceil_div(zp.nlines, ZF::LINES));
-    hipLaunchKernelGGL((k_zpass<M, false>), grid, dim3(ZF::THREADS), 0, s, zp, tb, tw);
+    if (zp.fold.xs)
+      hipLaunchKernelGGL((k_zpass<M, false, true>), grid, dim3(ZF::THREADS), 0, s, zp, tb, tw);
+    else
+      hipLaunchKernelGGL((k_zpass<M, false>), grid, dim3(ZF::THREADS), 0, s, zp, tb, tw);
     PM_LAUNCHED("fft_z_r2c", s);
   }
   return PM_SUCCESS;
@@ -563,8 +622,11 @@ SpecTables spec_tables_view(const float* base, const int32_t* shape, const SpecT
   return tb;
 }
 
-int launch_spec_tables(float* out, const int32_t* shape, const SpecTables& scalars, hipStream_t s) {
-  hipLaunchKernelGGL(k_spec_tables, dim3(8), dim3(256), 0, s, out, shape[0], shape[1], shape[2], scalars);
+int launch_spec_tables(float* out, const int32_t* shape, const SpecTables& scalars, int32_t* zero, int64_t nzero,
+                       hipStream_t s) {
+  const unsigned blocks = (unsigned)std::max<int64_t>(8, std::min<int64_t>(ceil_div(nzero, 1024), 512));
+  hipLaunchKernelGGL(k_spec_tables, dim3(blocks), dim3(256), 0, s, out, shape[0], shape[1], shape[2], scalars, zero,
+                     nzero);
   PM_LAUNCHED("k_spec_tables", s);
   return PM_SUCCESS;
 }
@@ -586,11 +648,9 @@ int rfft3d_pitched(const float* in, float2* spec, const int32_t* shape, int64_t 
   const int nx = shape[0], ny = shape[1], nz = shape[2], m = nz / 2;
   ZPass zp{};
   zp.rin = in;
-  zp.cmain = spec;
-  zp.cnyq = spec + m;
+  zp.cmain[0] = spec;
   zp.pitch_r = nz;
   zp.pitch_c = pitch;
-  zp.nyq_stride = pitch;
   zp.nlines = (int64_t)nx * ny;
   zp.src_shift = shift;
   zp.src_scale = scale;
@@ -614,12 +674,10 @@ int irfft3d_pitched(float2* spec, float* out, const int32_t* shape, int64_t pitc
   st = launch_cols(ny, kColInv, cy, nx, tb, 0, s);
   if (st) return st;
   ZPass zp{};
-  zp.rout = out;
-  zp.cmain = spec;
-  zp.cnyq = spec + m;
+  zp.rout[0] = out;
+  zp.cmain[0] = spec;
   zp.pitch_r = nz;
   zp.pitch_c = pitch;
-  zp.nyq_stride = pitch;
   zp.nlines = (int64_t)nx * ny;
   zp.out_scale = (float)(2.0 / ((double)nx * ny * nz));
   return launch_z(nz, true, zp, tb, s);

@@ -15,7 +15,8 @@ int launch_z(int nz, bool c2r, const ZPass& zp, const SpecTables& tb, hipStream_
 size_t spec_table_floats(const int32_t* shape);
 SpecTables spec_scalars(double cell_size, double ptcl_spacing, int mask_active);
 SpecTables spec_tables_view(const float* base, const int32_t* shape, const SpecTables& scalars);
-int launch_spec_tables(float* out, const int32_t* shape, const SpecTables& scalars, hipStream_t s);
+int launch_spec_tables(float* out, const int32_t* shape, const SpecTables& scalars, int32_t* zero, int64_t nzero,
+                       hipStream_t s);  // zero (nzero words, may be null with 0) is cleared too
 int launch_spectral_multiply(const float2* in, float2* out, const int32_t* shape, const SpecTables& tb,
                              int axis, int adjoint, hipStream_t s);
 

@@ -532,11 +532,24 @@ __device__ __forceinline__ void load_plane(float* plane, const float* __restrict
   }
 }
 
+// Invalid particles (binned last, past the last brick: sorted positions [first, n)) get zero rows,
+// a share per workgroup of the column walk that writes the others' (n = 0: nothing to do).
+__device__ __forceinline__ void zero_invalid(const int32_t* __restrict__ perm, int64_t first, int64_t n,
+                                             float* __restrict__ out) {
+  for (int64_t j = first + (int64_t)blockIdx.x * kTileThreads + threadIdx.x; j < n;
+       j += (int64_t)gridDim.x * kTileThreads) {
+    const int64_t i = perm[j];
+    out[i * 3 + 0] = 0.f;
+    out[i * 3 + 1] = 0.f;
+    out[i * 3 + 2] = 0.f;
+  }
+}
+
 template <int BX, int BY, int BZ>
 __global__ void __launch_bounds__(kTileThreads) k_gather_columns(
     const int16_t* __restrict__ pmid, const float* __restrict__ disp, const int32_t* __restrict__ bin_off,
     const int32_t* __restrict__ perm, Geom g, Bricks k, const float* __restrict__ f0,
-    const float* __restrict__ f1, const float* __restrict__ f2, float* __restrict__ acc) {
+    const float* __restrict__ f1, const float* __restrict__ f2, int64_t nzero, float* __restrict__ acc) {
   constexpr int kLds = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
   constexpr int kPl = BX ? (BX + 1) * (BY + 1) : kPlaneMax;
   __shared__ __align__(16) float tile[kLds];
@@ -606,6 +619,7 @@ __global__ void __launch_bounds__(kTileThreads) k_gather_columns(
       }
     }
   }
+  zero_invalid(perm, bin_off[(int64_t)k.nb[0] * k.nb[1] * nb2], nzero, acc);
 }
 
 // The displacement cotangent of the force step, tiled like k_gather_columns: for sorted
@@ -621,7 +635,7 @@ __global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
     const int16_t* __restrict__ pmid, const float* __restrict__ disp, const int32_t* __restrict__ bin_off,
     const int32_t* __restrict__ perm, Geom g, Bricks k, const float* __restrict__ f0, const float* __restrict__ f1,
     const float* __restrict__ f2, const float* __restrict__ dcot, const float* __restrict__ cot_s, int64_t n,
-    float val, float* __restrict__ disp_cot, int accum) {
+    float val, int64_t nzero, float* __restrict__ disp_cot, int accum) {
   constexpr int kLds = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
   constexpr int kPl = BX ? (BX + 1) * (BY + 1) : kPlaneMax;
   __shared__ __align__(16) float tile[kLds];
@@ -714,18 +728,7 @@ __global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
       }
     }
   }
-}
-
-// invalid particles (sorted last, past the last brick) get a zero acceleration
-__global__ void k_zero_invalid(const int32_t* __restrict__ perm, const int32_t* __restrict__ bin_off,
-                               int64_t nbins, int64_t n, float* __restrict__ acc) {
-  for (int64_t j = bin_off[nbins] + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n;
-       j += (int64_t)gridDim.x * blockDim.x) {
-    int64_t i = perm[j];
-    acc[i * 3 + 0] = 0.f;
-    acc[i * 3 + 1] = 0.f;
-    acc[i * 3 + 2] = 0.f;
-  }
+  zero_invalid(perm, bin_off[(int64_t)k.nb[0] * k.nb[1] * nb2], nzero, disp_cot);
 }
 
 // Reverse of the three gathers without brick tiling (gather^T = float-atomic scatter of
@@ -968,11 +971,14 @@ struct Buffers {
   float* r0;  // density, then F_x
   float* r1;  // F_y
   float* r2;  // F_z
-  float2* ca;
-  float2* cb;
+  float2* ca;  // s1-sized banded spectra: ca, cc, ce
+  float2* cb;  // s2-sized (packed y rows): cb, cd, cg
   float2* cc;
-  float2* cd;  // packed-y spectra (only when the y band is packed)
+  float2* cd;
   float2* ce;
+  float2* cg;
+  int32_t* count;    // the bucketing's counters and scan partials
+  int32_t* partial;
   // reverse only: F_x (the forward keeps rho in r0), three mesh cotangents
   float* g0;
   float* g1;
@@ -1007,13 +1013,17 @@ bool carve(Arena& ws, const Layout& L, int64_t n, const int32_t* shape, const in
   b.r0 = ws.take<float>(L.nreal);
   b.r1 = ws.take<float>(L.nreal);
   b.r2 = ws.take<float>(L.nreal);
-  // banded force pipeline (see force_mesh_stage and adjoint_spectral_stage): s1-sized ca,
-  // cc, ce and s2-sized cb, cd
+  // banded force pipeline (see force_mesh_stage and adjoint_spectral_stage)
+  // (the x Green pass's two outputs, cb and cg, side by side: 1.34 ms at 1024^3 against 1.47 with cg
+  // last, where the three streams of the pass start further apart)
   b.ca = ws.take<float2>(L.s1);
   b.cb = ws.take<float2>(L.s2);
+  b.cg = ws.take<float2>(L.s2);
   b.cc = ws.take<float2>(L.s1);
   b.cd = ws.take<float2>(L.s2);
   b.ce = ws.take<float2>(L.s1);
+  b.count = ws.take<int32_t>(nbins + 2);
+  b.partial = ws.take<int32_t>(sort::bucket_partials(nbins + 2));
   if (reverse) {
     b.g0 = ws.take<float>(L.nreal);
     b.g1 = ws.take<float>(L.nreal);
@@ -1032,8 +1042,7 @@ size_t workspace_bytes(const pm_gravity_desc* d, int64_t n, bool reverse) {
   Arena probe(reinterpret_cast<void*>(uintptr_t(256)), SIZE_MAX / 2);
   Buffers b;
   carve(probe, L, n, d->mesh_shape, d->brick, reverse, b);
-  // the sort's temporaries are carved after the step buffers
-  return probe.used + 256 + sort::bucket_workspace_bytes(d->mesh_shape, d->brick) + 256;
+  return probe.used + 256;
 }
 
 Geom step_geom(const pm_gravity_desc* d) {
@@ -1058,12 +1067,12 @@ int fill(float* p, int64_t n, hipStream_t s) {
   return PM_SUCCESS;
 }
 
-// Bucketing by brick (with the payload gathered into bucket order), density.  Leaves rho in b.r0.
 // Tiled CIC scatter of the bucketed particles into mesh (whose every cell it writes): the
 // constant particle value, or per-particle values vals (sorted order) with vscale[0] * |vals|
-// <= 1; then the fold of the neighbouring columns' upper x/y planes.
+// <= 1; then, with fold, the neighbouring columns' upper x/y planes (otherwise the R2C pass that
+// reads the mesh adds them: fold_planes).
 int scatter_tiled(const pm_gravity_desc* d, const Buffers& b, float* mesh, const float* vals, const float* vscale,
-                  hipStream_t s) {
+                  bool fold, hipStream_t s) {
   const Geom g = step_geom(d);
   Bricks k = make_bricks(d->mesh_shape, d->brick);
   const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
@@ -1074,6 +1083,7 @@ int scatter_tiled(const pm_gravity_desc* d, const Buffers& b, float* mesh, const
     hipLaunchKernelGGL((k_scatter_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
                        b.bins, d->particle_value, g, k, mesh, b.xs, b.ys, b.first, vals, vscale);
   PM_LAUNCHED("k_scatter_columns", s);
+  if (!fold) return PM_SUCCESS;
   const int64_t plane_cells = ((int64_t)k.nb[0] * k.n[1] + (int64_t)(k.n[0] - k.nb[0]) * k.nb[1]) * k.n[2];
   const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(plane_cells, kBlock), 8192));
   hipLaunchKernelGGL(k_fold_xy, dim3(blocks), dim3(kBlock), 0, s, k, b.xs, b.ys, mesh);
@@ -1081,10 +1091,24 @@ int scatter_tiled(const pm_gravity_desc* d, const Buffers& b, float* mesh, const
   return PM_SUCCESS;
 }
 
+// The plane buffers of an unfolded tiled scatter, for the R2C pass (mesh and brick extents are
+// powers of two: the brick divides the mesh).
+fft::FoldPlanes fold_planes(const pm_gravity_desc* d, const Buffers& b) {
+  fft::FoldPlanes f;
+  f.xs = b.xs;
+  f.ys = b.ys;
+  f.ny_log = fft::ilog2(d->mesh_shape[1]);
+  f.b0_log = fft::ilog2(d->brick[0]);
+  f.b1_log = fft::ilog2(d->brick[1]);
+  f.nb0 = d->mesh_shape[0] / d->brick[0];
+  f.nb1 = d->mesh_shape[1] / d->brick[1];
+  return f;
+}
+
 // The particles binned by brick into the workspace's sorted copies (b.perm, b.bins, b.pmid_s,
 // b.disp_s, b.valid_s).
 int bucket_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
-                 const pm_gravity_desc* d, Buffers& b, Arena& ws, hipStream_t s) {
+                 const pm_gravity_desc* d, Buffers& b, hipStream_t s) {
   // the Lagrangian grid the particle count implies (mesh * cell / spacing per axis)
   int32_t grid[3] = {0, 0, 0};
   if (d->ptcl_spacing > 0.f)
@@ -1093,14 +1117,16 @@ int bucket_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, i
       grid[a] = (v >= 1.0 && v < 1e9) ? (int32_t)lrint(v) : 0;
     }
   return sort::bucket_cells(pmid, disp, valid, n, d->mesh_shape, d->cell_size, d->brick, grid, b.perm, b.bins,
-                            b.pmid_s, b.disp_s, b.valid_s, ws, s);
+                            b.pmid_s, b.disp_s, b.valid_s, b.count, b.partial, true, s);
 }
 
+// Bucketing by brick (with the payload gathered into bucket order), then the density in b.r0; fold
+// as for scatter_tiled.
 int density_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
-                  const pm_gravity_desc* d, const Layout& L, Buffers& b, Arena& ws, hipStream_t s) {
+                  const pm_gravity_desc* d, const Layout& L, Buffers& b, bool fold, hipStream_t s) {
   const Geom g = step_geom(d);
-  PM_TRY(bucket_stage(pmid, disp, valid, n, d, b, ws, s));
-  if (b.tiled) return scatter_tiled(d, b, b.r0, nullptr, nullptr, s);
+  PM_TRY(bucket_stage(pmid, disp, valid, n, d, b, s));
+  if (b.tiled) return scatter_tiled(d, b, b.r0, nullptr, nullptr, fold, s);
   PM_TRY(fill(b.r0, L.nreal, s));
   if (n > 0) {
     hipLaunchKernelGGL(k_scatter_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, b.pmid_s, b.disp_s, b.valid_s,
@@ -1117,20 +1143,15 @@ int gather_stage(const int16_t* pmid_s, const float* disp_s, const uint8_t* vali
   const Geom g = step_geom(d);
   if (b.tiled) {
     Bricks k = make_bricks(d->mesh_shape, d->brick);
-    const int64_t nbins = (int64_t)k.nb[0] * k.nb[1] * k.nb[2];
     const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
+    const int64_t nzero = valid ? n : 0;
     if (is_brick(k, 16, 16, 32))
       hipLaunchKernelGGL((k_gather_columns<16, 16, 32>), dim3(ncols), dim3(kTileThreads), 0, s, pmid_s, disp_s,
-                         b.bins, b.perm, g, k, fx, fy, fz, acc);
+                         b.bins, b.perm, g, k, fx, fy, fz, nzero, acc);
     else
       hipLaunchKernelGGL((k_gather_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, pmid_s, disp_s,
-                         b.bins, b.perm, g, k, fx, fy, fz, acc);
+                         b.bins, b.perm, g, k, fx, fy, fz, nzero, acc);
     PM_LAUNCHED("k_gather_columns", s);
-    if (valid) {
-      unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kBlock), 4096);
-      hipLaunchKernelGGL(k_zero_invalid, dim3(blocks), dim3(kBlock), 0, s, b.perm, b.bins, nbins, n, acc);
-      PM_LAUNCHED("k_zero_invalid", s);
-    }
     return PM_SUCCESS;
   }
   hipLaunchKernelGGL(k_gather3_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, pmid_s, disp_s, valid_s, b.perm, n, g,
@@ -1146,54 +1167,51 @@ int disp_cot_tiled(const pm_gravity_desc* d, const Buffers& b, int64_t n, const 
                    hipStream_t s) {
   const Geom g = step_geom(d);
   Bricks k = make_bricks(d->mesh_shape, d->brick);
-  const int64_t nbins = (int64_t)k.nb[0] * k.nb[1] * k.nb[2];
   const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
   const float val = d->particle_value;
+  const int64_t nzero = valid ? n : 0;
   if (is_brick(k, 16, 16, 32))
     hipLaunchKernelGGL((k_disp_cot_columns<16, 16, 32>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, disp_cot, 0);
+                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, nzero, disp_cot, 0);
   else
     hipLaunchKernelGGL((k_disp_cot_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, disp_cot, 0);
+                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, nzero, disp_cot, 0);
   PM_LAUNCHED("k_disp_cot_columns", s);
-  if (valid) {
-    unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kBlock), 4096);
-    hipLaunchKernelGGL(k_zero_invalid, dim3(blocks), dim3(kBlock), 0, s, b.perm, b.bins, nbins, n, disp_cot);
-    PM_LAUNCHED("k_zero_invalid", s);
-  }
   return PM_SUCCESS;
 }
 
-// Density (b.r0) -> force meshes F_x (b.r0), F_y (b.r1), F_z (b.r2).
+// Density (b.r0) -> force meshes F_x (b.r0, or b.g0 when the density is kept), F_y (b.r1), F_z
+// (b.r2); unfolded: b.r0's plane buffers are still to be added (scatter_tiled).
 int force_mesh_stage(const pm_gravity_desc* d, const Layout& L, Buffers& b, const fft::SpecTables& tb,
-                     hipStream_t s, bool keep_density, const float* rho_add) {
+                     hipStream_t s, bool keep_density, bool unfolded, const float* rho_add) {
   using namespace fft;
   const float coef = 1.5f * d->omega_m;  // 1.5 * Omega_m in float32 (gravity.py:630)
   const bool zband = L.nkz <= L.m;      // Nyquist column not stored
   const bool ypack = L.ky_keep >= 0;
-  // every pass writes a buffer other than the one it reads (the two-output passes need it):
-  //   A (s1) z r2c output, later chi = y inverse of psi (D_z applied by the last z c2r)
+  // every pass writes buffers other than those it reads (the passes with several outputs need it):
+  //   A (s1) z r2c output, later chi = y inverse of psi (D_z applied by the z c2r)
   //   B (s2) y forward output (packed |ky| band)
-  //   G (s1) psi = x inverse of the Green-multiplied spectrum, later F_x's y inverse
+  //   G (s2) psi = x inverse of the Green-multiplied spectrum
   //   C (s2) D_x psi
   //   E (s1) D_y chi
+  //   H (s1) y inverse of D_x psi
   float2* A = b.ca;
   float2* B = b.cd;
-  float2* G = b.cc;
+  float2* G = b.cg;
   float2* C = b.cb;
   float2* E = b.ce;
+  float2* H = b.cc;
   const int64_t p1 = L.pitch1;
   ZPass z1{};
   z1.rin = b.r0;
-  z1.cmain = A;
-  z1.cnyq = zband ? A : A + L.m;
+  z1.cmain[0] = A;
   z1.pitch_r = L.nz;
   z1.pitch_c = p1;
-  z1.nyq_stride = p1;
   z1.nlines = (int64_t)L.nx * L.ny;
   z1.src_shift = -1.f;
   z1.src_scale = coef;
   z1.rin_add = rho_add;  // learned density correction (null: none)
+  if (unfolded && b.tiled) z1.fold = fold_planes(d, b);
   z1.kz_lim = L.nkz;
   z1.nyq = zband ? 0 : 1;
   PM_TRY(launch_z(L.nz, false, z1, tb, s));
@@ -1211,39 +1229,32 @@ int force_mesh_stage(const pm_gravity_desc* d, const Layout& L, Buffers& b, cons
     xg.ky_shift = L.ny - L.nky;
   }
   PM_TRY(launch_cols(L.nx, kColGreen, xg, L.nky, tb, 0, s));
-  // y inverses expand the band back to full rows
-  ColPass yi2{G, A, E, p1, 1, (int64_t)L.nky * p1, ncols, 0, 0, 0, 0, 0};
-  yi2.o_row = p1;
-  yi2.o_batch = (int64_t)L.ny * p1;
-  yi2.keep = L.ky_keep;
-  yi2.compact_in = 1;
-  PM_TRY(launch_cols(L.ny, kColInv2, yi2, L.nx, tb, 1, s));
-  ColPass yi{C, G, nullptr, p1, 1, (int64_t)L.nky * p1, ncols, 0, 0, 0, 0, 0};
+  // the three y inverses expand the band back to full rows, in one launch
+  ColPass yi{G, A, E, p1, 1, (int64_t)L.nky * p1, ncols, 0, 0, 0, 0, 0};
+  yi.in1 = C;
+  yi.out2 = H;
   yi.o_row = p1;
   yi.o_batch = (int64_t)L.ny * p1;
   yi.keep = L.ky_keep;
   yi.compact_in = 1;
-  PM_TRY(launch_cols(L.ny, kColInv, yi, L.nx, tb, 1, s));
-  const float norm = (float)(2.0 / ((double)L.nx * L.ny * L.nz));
+  PM_TRY(launch_cols(L.ny, kColInv3, yi, L.nx, tb, 1, s));
+  // the three c2r passes, in one launch
   ZPass zc{};
   zc.pitch_r = L.nz;
   zc.pitch_c = p1;
-  zc.nyq_stride = p1;
   zc.nlines = (int64_t)L.nx * L.ny;
-  zc.out_scale = norm;
+  zc.out_scale = (float)(2.0 / ((double)L.nx * L.ny * L.nz));
   zc.kz_lim = L.nkz;
   zc.nyq = zband ? 0 : 1;
-  float* fx = keep_density ? b.g0 : b.r0;  // reverse keeps rho for the Omega_m cotangent
-  const float2* srcs[3] = {G, E, A};
-  float* dsts[3] = {fx, b.r1, b.r2};
-  for (int c = 0; c < 3; ++c) {
-    zc.cmain = const_cast<float2*>(srcs[c]);
-    zc.cnyq = zband ? zc.cmain : zc.cmain + L.m;
-    zc.rout = dsts[c];
-    zc.deriv = c == 2;  // D_z on the last component
-    PM_TRY(launch_z(L.nz, true, zc, tb, s));
-  }
-  return PM_SUCCESS;
+  zc.ncomp = 3;
+  zc.cmain[0] = H;
+  zc.cmain[1] = E;
+  zc.cmain[2] = A;
+  zc.rout[0] = keep_density ? b.g0 : b.r0;  // reverse keeps rho for the Omega_m cotangent
+  zc.rout[1] = b.r1;
+  zc.rout[2] = b.r2;
+  zc.deriv = 1 << 2;  // D_z on the last component
+  return launch_z(L.nz, true, zc, tb, s);
 }
 
 // Spectral adjoint of the force meshes: src_cot (b.g1, real) = irfftn(G * sum_i conj(D_i) *
@@ -1252,34 +1263,37 @@ int force_mesh_stage(const pm_gravity_desc* d, const Layout& L, Buffers& b, cons
 // the particle-Nyquist band, so the passes are force_mesh_stage's in reverse on the same band:
 // three z r2c passes storing the kz band, three y passes packing the |ky| band, one x pass
 // that transforms the three spectra, combines them mode by mode and inverts (kColAdj), the y
-// inverse expanding the band and the z c2r.  Buffers: ca, cc, ce (s1) and cb, cd (s2).
-int adjoint_spectral_stage(const pm_gravity_desc* d, const Layout& L, Buffers& b, const fft::SpecTables& tb,
-                           hipStream_t s) {
+// inverse expanding the band and the z c2r.  Buffers: ca, cc, ce (s1) and cb, cd, cg (s2).
+// adjoint_z_pass is component c's z r2c, taken right after its scatter (whose plane buffers it
+// folds when unfolded).
+int adjoint_z_pass(const pm_gravity_desc* d, const Layout& L, Buffers& b, const fft::SpecTables& tb, int c,
+                   const float* mesh, bool unfolded, hipStream_t s) {
   using namespace fft;
   const bool zband = L.nkz <= L.m;
-  const bool ypack = L.ky_keep >= 0;
-  const int64_t p1 = L.pitch1;
-  const int ncols = L.nkz;
-  float* reals[3] = {b.g1, b.g2, b.g3};
-  float2* s1buf[3] = {b.ca, b.cc, b.ce};
+  float2* out[3] = {b.ca, b.cc, b.ce};
   ZPass zr{};
+  zr.rin = mesh;
+  zr.cmain[0] = out[c];
   zr.pitch_r = L.nz;
-  zr.pitch_c = p1;
-  zr.nyq_stride = p1;
+  zr.pitch_c = L.pitch1;
   zr.nlines = (int64_t)L.nx * L.ny;
   zr.src_shift = 0.f;
   zr.src_scale = 1.f;
   zr.kz_lim = L.nkz;
   zr.nyq = zband ? 0 : 1;
-  for (int c = 0; c < 3; ++c) {
-    zr.rin = reals[c];
-    zr.cmain = s1buf[c];
-    zr.cnyq = zband ? s1buf[c] : s1buf[c] + L.m;
-    PM_TRY(launch_z(L.nz, false, zr, tb, s));
-  }
-  // y forward, packed: ca -> cb, cc -> cd, then ce -> ca (ca is free again; s2 <= s1)
-  float2* s2buf[3] = {b.cb, b.cd, b.ca};
-  for (int c = 0; c < 3; ++c) {
+  if (unfolded) zr.fold = fold_planes(d, b);
+  return launch_z(L.nz, false, zr, tb, s);
+}
+
+int adjoint_spectral_stage(const Layout& L, Buffers& b, const fft::SpecTables& tb, hipStream_t s) {
+  using namespace fft;
+  const bool zband = L.nkz <= L.m;
+  const bool ypack = L.ky_keep >= 0;
+  const int64_t p1 = L.pitch1;
+  const int ncols = L.nkz;
+  float2* s1buf[3] = {b.ca, b.cc, b.ce};
+  float2* s2buf[3] = {b.cb, b.cd, b.cg};
+  for (int c = 0; c < 3; ++c) {  // y forward, packed
     ColPass yf{s1buf[c], s2buf[c], nullptr, p1, 1, (int64_t)L.ny * p1, ncols, 0, 0, 0, 0, 0};
     yf.o_row = p1;
     yf.o_batch = (int64_t)L.nky * p1;
@@ -1305,14 +1319,12 @@ int adjoint_spectral_stage(const pm_gravity_desc* d, const Layout& L, Buffers& b
   ZPass zc{};
   zc.pitch_r = L.nz;
   zc.pitch_c = p1;
-  zc.nyq_stride = p1;
   zc.nlines = (int64_t)L.nx * L.ny;
   zc.out_scale = (float)(2.0 / ((double)L.nx * L.ny * L.nz));
   zc.kz_lim = L.nkz;
   zc.nyq = zband ? 0 : 1;
-  zc.cmain = b.ce;
-  zc.cnyq = zband ? b.ce : b.ce + L.m;
-  zc.rout = b.g1;
+  zc.cmain[0] = b.ce;
+  zc.rout[0] = b.g1;
   zc.deriv = 0;
   return launch_z(L.nz, true, zc, tb, s);
 }
@@ -1333,11 +1345,9 @@ int potential_stage(const Layout& L, float2* A, float2* B, float2* G, const fft:
   const int ncols = L.nkz;
   ZPass zr{};
   zr.rin = in;
-  zr.cmain = A;
-  zr.cnyq = zband ? A : A + L.m;
+  zr.cmain[0] = A;
   zr.pitch_r = L.nz;
   zr.pitch_c = p1;
-  zr.nyq_stride = p1;
   zr.nlines = (int64_t)L.nx * L.ny;
   zr.src_shift = shift;
   zr.src_scale = scale;
@@ -1364,14 +1374,12 @@ int potential_stage(const Layout& L, float2* A, float2* B, float2* G, const fft:
   ZPass zc{};
   zc.pitch_r = L.nz;
   zc.pitch_c = p1;
-  zc.nyq_stride = p1;
   zc.nlines = (int64_t)L.nx * L.ny;
   zc.out_scale = (float)(2.0 / ((double)L.nx * L.ny * L.nz));
   zc.kz_lim = L.nkz;
   zc.nyq = zband ? 0 : 1;
-  zc.cmain = A;
-  zc.cnyq = zband ? A : A + L.m;
-  zc.rout = out;
+  zc.cmain[0] = A;
+  zc.rout[0] = out;
   zc.rout_add = add;
   zc.deriv = 0;
   return launch_z(L.nz, true, zc, tb, s);
@@ -1394,7 +1402,9 @@ int prepare(const pm_gravity_desc* d, int64_t n, void* workspace, size_t workspa
   PM_RETURN_IF(!carve(ws, L, n, d->mesh_shape, d->brick, reverse, b), PM_ERROR_WORKSPACE,
                "workspace carve failed");
   const fft::SpecTables sc = fft::spec_scalars(d->cell_size, d->ptcl_spacing, d->mask_active);
-  PM_TRY(fft::launch_spec_tables(b.tables, d->mesh_shape, sc, s));
+  // the bucketing's counters are cleared along (unused by the calls that resume)
+  PM_TRY(fft::launch_spec_tables(b.tables, d->mesh_shape, sc, b.count,
+                                 sort::bucket_count_len(d->mesh_shape, d->brick), s));
   tb = fft::spec_tables_view(b.tables, d->mesh_shape, sc);
   return PM_SUCCESS;
 }
@@ -1441,9 +1451,9 @@ int pm_gravity_corrected(const int16_t* pmid, const float* disp, const uint8_t* 
   if (st) return st;
   PM_RETURN_IF(n > 0 && (pmid == nullptr || disp == nullptr || acc == nullptr), PM_ERROR_INVALID_ARGUMENT,
                "pmid/disp/acc NULL");
-  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, ws, s);
+  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, false, s);
   if (st) return st;
-  st = grav::force_mesh_stage(desc, L, b, tb, s, false, rho_add);
+  st = grav::force_mesh_stage(desc, L, b, tb, s, false, true, rho_add);
   if (st) return st;
   return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
 }
@@ -1462,7 +1472,7 @@ int pm_gravity_corrected_resume(const int16_t* pmid, const float* disp, const ui
   if (st) return st;
   PM_RETURN_IF(n > 0 && (pmid == nullptr || disp == nullptr || acc == nullptr), PM_ERROR_INVALID_ARGUMENT,
                "pmid/disp/acc NULL");
-  st = grav::force_mesh_stage(desc, L, b, tb, s, false, rho_add);
+  st = grav::force_mesh_stage(desc, L, b, tb, s, false, false, rho_add);
   if (st) return st;
   return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
 }
@@ -1494,7 +1504,7 @@ int pm_gravity_density(const int16_t* pmid, const float* disp, const uint8_t* va
   if (st) return st;
   PM_RETURN_IF(rho == nullptr || (n > 0 && (pmid == nullptr || disp == nullptr)), PM_ERROR_INVALID_ARGUMENT,
                "pmid/disp/rho NULL");
-  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, ws, s);
+  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, true, s);
   if (st) return st;
   if (rho == b.r0) return PM_SUCCESS;  // the caller reads the density in place (pm_gravity_density_offset)
   if (((reinterpret_cast<uintptr_t>(rho) | reinterpret_cast<uintptr_t>(b.r0)) & 15) == 0) {
@@ -1532,9 +1542,9 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
   const Geom g = grav::step_geom(desc);
   // recompute the forward meshes: rho stays in r0, F_x goes to g0, F_y r1, F_z r2
   if (!resume) {
-    st = grav::density_stage(pmid, disp, valid, n, desc, L, b, ws, s);
+    st = grav::density_stage(pmid, disp, valid, n, desc, L, b, true, s);
     if (st) return st;
-    st = grav::force_mesh_stage(desc, L, b, tb, s, true, rho_add);
+    st = grav::force_mesh_stage(desc, L, b, tb, s, true, false, rho_add);
     if (st) return st;
   }
   // gather^T: acc_cot scattered into three cotangent meshes, displacement cotangent from F.
@@ -1551,7 +1561,9 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
     PM_LAUNCHED("k_cot_scale", s);
     float* gm[3] = {b.g1, b.g2, b.g3};
     for (int c = 0; c < 3; ++c) {
-      st = grav::scatter_tiled(desc, b, gm[c], b.cot_s + (int64_t)c * n, b.cot_pmax + grav::kCotBlocks, s);
+      st = grav::scatter_tiled(desc, b, gm[c], b.cot_s + (int64_t)c * n, b.cot_pmax + grav::kCotBlocks, false, s);
+      if (st) return st;
+      st = grav::adjoint_z_pass(desc, L, b, tb, c, gm[c], true, s);
       if (st) return st;
     }
   } else {
@@ -1567,9 +1579,11 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
                          b.disp_cot_s);
       PM_LAUNCHED("k_gather3_bwd_sorted", s);
     }
+    float* gm[3] = {b.g1, b.g2, b.g3};
+    for (int c = 0; c < 3; ++c) PM_TRY(grav::adjoint_z_pass(desc, L, b, tb, c, gm[c], false, s));
   }
   // spectral adjoint: src_cot (g1) = irfftn(G * sum_i conj(D_i) rfftn(g_i)) on the band
-  st = grav::adjoint_spectral_stage(desc, L, b, tb, s);
+  st = grav::adjoint_spectral_stage(L, b, tb, s);
   if (st) return st;
   {
     const float coef = 1.5f * desc->omega_m;
@@ -1610,9 +1624,9 @@ int pm_gravity_keep(const int16_t* pmid, const float* disp, const uint8_t* valid
   if (st) return st;
   PM_RETURN_IF(n > 0 && (pmid == nullptr || disp == nullptr || acc == nullptr), PM_ERROR_INVALID_ARGUMENT,
                "pmid/disp/acc NULL");
-  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, ws, s);
+  st = grav::density_stage(pmid, disp, valid, n, desc, L, b, true, s);
   if (st) return st;
-  st = grav::force_mesh_stage(desc, L, b, tb, s, true, nullptr);
+  st = grav::force_mesh_stage(desc, L, b, tb, s, true, false, nullptr);
   if (st) return st;
   return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.g0, b.r1, b.r2, acc, s);
 }
@@ -1637,7 +1651,7 @@ int pm_gravity_density_cot(const int16_t* pmid, const float* disp, const uint8_t
   PM_RETURN_IF(n > 0 && (pmid == nullptr || disp == nullptr || dens_cot == nullptr || disp_cot == nullptr),
                PM_ERROR_INVALID_ARGUMENT, "pmid/disp/dens_cot/disp_cot NULL");
   if (n == 0) return PM_SUCCESS;
-  PM_TRY(grav::bucket_stage(pmid, disp, valid, n, desc, b, ws, s));
+  PM_TRY(grav::bucket_stage(pmid, disp, valid, n, desc, b, s));
   const Geom g = grav::step_geom(desc);
   const float val = desc->particle_value;
   if (b.tiled) {  // invalid particles are in no bin: their disp_cot stays as it is
@@ -1646,11 +1660,11 @@ int pm_gravity_density_cot(const int16_t* pmid, const float* disp, const uint8_t
     if (grav::is_brick(k, 16, 16, 32))
       hipLaunchKernelGGL((grav::k_disp_cot_columns<16, 16, 32>), dim3(ncols), dim3(grav::kTileThreads), 0, s,
                          b.pmid_s, b.disp_s, b.bins, b.perm, g, k, nullptr, nullptr, nullptr, dens_cot, nullptr, n,
-                         val, disp_cot, 1);
+                         val, (int64_t)0, disp_cot, 1);
     else
       hipLaunchKernelGGL((grav::k_disp_cot_columns<0, 0, 0>), dim3(ncols), dim3(grav::kTileThreads), 0, s, b.pmid_s,
                          b.disp_s, b.bins, b.perm, g, k, nullptr, nullptr, nullptr, dens_cot, nullptr, n, val,
-                         disp_cot, 1);
+                         (int64_t)0, disp_cot, 1);
     PM_LAUNCHED("k_disp_cot_columns", s);
     return PM_SUCCESS;
   }
@@ -1684,7 +1698,7 @@ int pm_gravity_potential(const float* in, float shift, float scale, const float*
   float2* B = ws.take<float2>(L.s2);
   PM_RETURN_IF(!ws.ok(), PM_ERROR_WORKSPACE, "potential workspace carve failed");
   const fft::SpecTables sc = fft::spec_scalars(desc->cell_size, desc->ptcl_spacing, desc->mask_active);
-  PM_TRY(fft::launch_spec_tables(tables, desc->mesh_shape, sc, s));
+  PM_TRY(fft::launch_spec_tables(tables, desc->mesh_shape, sc, nullptr, 0, s));
   const fft::SpecTables tb = fft::spec_tables_view(tables, desc->mesh_shape, sc);
   return grav::potential_stage(L, A, B, G, tb, in, shift, scale, add, out, s);
 }
@@ -1714,7 +1728,7 @@ int pm_spectral_force_multiply(const float* in_complex, float* out_complex, cons
   hipStream_t s = as_stream(stream);
   float* tables = static_cast<float*>(workspace);
   const fft::SpecTables sc = fft::spec_scalars(desc->cell_size, desc->ptcl_spacing, desc->mask_active);
-  st = fft::launch_spec_tables(tables, desc->mesh_shape, sc, s);
+  st = fft::launch_spec_tables(tables, desc->mesh_shape, sc, nullptr, 0, s);
   if (st) return st;
   fft::SpecTables tb = fft::spec_tables_view(tables, desc->mesh_shape, sc);
   return fft::launch_spectral_multiply(reinterpret_cast<const float2*>(in_complex),

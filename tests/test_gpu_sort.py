@@ -135,3 +135,25 @@ def test_force_step_bucketing_bins_every_particle(device, grid, hint, valid_frac
     np.testing.assert_array_equal(pm_s, pmid[perm])
     np.testing.assert_array_equal(dp_s.view(np.uint32), disp[perm].view(np.uint32))
     np.testing.assert_array_equal(v_s, np.ones(n, np.uint8) if valid is None else valid[perm].astype(np.uint8))
+
+
+@pytest.mark.parametrize("mesh", [(1, 1, 1), (2, 23, 89), (9, 5, 91), (64, 8, 8), (89, 23, 4), (68, 15, 257),
+                                  (27, 133, 73), (64, 64, 65)])
+def test_bin_offsets_at_the_edges_of_the_scan(device, mesh):
+    """Bin counts just below, at and above the scan's chunk of 4096 counters (4094, 4095, 4096
+    bins), several chunks, the last size of the single-launch scan (262,140 bins) and the first of
+    the three-launch one (262,143, 266,240): integers, so equal to numpy's."""
+    rng = np.random.default_rng(sum(mesh))
+    n = 30011
+    pmid = np.stack([rng.integers(0, m, n) for m in mesh], 1).astype(np.int16)
+    pmid[: n // 4] = [m - 1 for m in mesh]  # a quarter in the last bin
+    disp = np.zeros((n, 3), np.float32)
+    valid = rng.random(n) < 0.9
+    perm, offs, pm_s, _, _ = hip_bucket(pmid, disp, valid, mesh, 1.0, (1, 1, 1), None, device)
+    key = np.where(valid, (pmid[:, 0].astype(np.int64) * mesh[1] + pmid[:, 1]) * mesh[2] + pmid[:, 2],
+                   int(np.prod(mesh)))
+    count = np.bincount(key, minlength=int(np.prod(mesh)) + 1)
+    np.testing.assert_array_equal(offs, np.concatenate([[0], np.cumsum(count)]))
+    np.testing.assert_array_equal(key[perm], np.sort(key))
+    assert np.array_equal(np.sort(perm), np.arange(n))
+    np.testing.assert_array_equal(pm_s, pmid[perm])
