@@ -67,11 +67,10 @@ def kernel_step_bytes(name, L, n_p, brick):
         "fft_cols_inv3": 2 * S2 + 3 * S1,
         "fft_z_c2r": 3 * (S1 + R),
         "k_bucket_count": 18 * n_p,
-        "k_bucket_place": (18 + 4 + 18 + 1) * n_p,
-        "k_zero_i32": 4 * (nb + 2),
+        "k_bucket_place": (18 + 4 + 16) * n_p,
         "scan": 8 * (nb + 2),
-        "k_scatter_columns": 18 * n_p + R + planes,
-        "k_gather_columns": (18 + 4 + 12) * n_p + 3 * R,
+        "k_scatter_columns": 16 * n_p + R + planes,
+        "k_gather_columns": (16 + 4 + 12) * n_p + 3 * R,
         "k_fill": R,
         "k_scatter_sorted": 19 * n_p + R,
         "k_gather3_sorted": (19 + 4 + 12) * n_p + 3 * R,

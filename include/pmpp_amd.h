@@ -137,8 +137,8 @@ int pm_sort_cells(const int16_t* pmid, const float* disp, const uint8_t* valid, 
  * unspecified (atomic arrival order), which the step's order-independent tile kernels allow.
  * perm, pmid_sorted (n,3), disp_sorted (n,3) and valid_sorted (n) are all written.
  * ptcl_grid (optional) names the Lagrangian grid the particles were generated on in C order;
- * when its product is n and it is a multiple of (4, 8, 64), particles are read in blocks of
- * that grid (speed only; any value gives a valid binning).  No counterpart in the reference,
+ * when its product is n (and its extents leave few slots of such blocks empty), particles are read
+ * in blocks of 64 along z of that grid (speed only; any value gives a valid binning).  No counterpart in the reference,
  * whose single-device path does not order particles (nbody/gravity.py:813). */
 int pm_bucket_cells_workspace(int64_t n, const int32_t mesh_shape[3], const int32_t brick[3],
                               size_t* bytes);

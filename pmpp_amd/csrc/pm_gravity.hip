@@ -104,16 +104,23 @@ __global__ void __launch_bounds__(kBlock) k_gather3_sorted(const int16_t* __rest
 // particle touches lies in its brick's tile extended by one cell on the upper side.  One
 // workgroup walks a column of bricks (fixed x and y brick coordinates) along z.
 //
-// Scatter (owner computes): the column's bricks are accumulated one after the other into an
+// Particles come as 16-byte records (pm_sort.h): the fractions and the tile offset of the base cell,
+// one vector load instead of six scalar ones and no division per particle (512^3 particles on a 1024^3
+// mesh: scatter 2.26 -> 1.54 ms, gather 4.95 -> 4.71 ms).
+//
+// Scatter (owner computes): a run of a column's bricks is accumulated one after the other into an
 // LDS tile of (BX+1)(BY+1)(BZ+1) int64 fixed-point cells with LDS atomics.  The tile's upper z
-// plane belongs to the next brick of the column and is carried to it inside LDS (the first
-// brick's lower plane waits for the last brick's carry), so the z halo never leaves the CU.
-// Owned cells are stored once with plain stores (no zero fill, no global atomics); the upper
-// x and y planes go to z-contiguous plane buffers (XS, YS) that k_fold_xy adds into the lower
-// x/y planes of the neighbouring columns (pull, fixed order: deterministic).
-// Gather: the column is walked downward in z.  Each force component's tile rows z in [0, BZ)
+// plane belongs to the next brick of the column and is carried to it inside LDS; the lower plane
+// of the run's first brick gets the carry of the brick below (the one above the periodic
+// wrap for the first) from that brick's own particles in its last z plane, read a second time.
+// So every owned cell is complete when it is stored, once, with plain stores (no zero fill, no
+// global atomics), and a column can be cut into runs for different workgroups: with whole
+// columns a 128^3 mesh has 64 of them.  The upper x and y planes go to z-contiguous plane buffers
+// (XS, YS), which are added to the lower x/y planes of the neighbouring columns later (pull,
+// fixed order: deterministic).
+// Gather: a run is walked downward in z.  Each force component's tile rows z in [0, BZ)
 // are read as aligned rows; the z = BZ plane is the lower plane of the brick above, kept in
-// LDS from the previous step, so no row costs a second cache line.
+// LDS from the previous step (read directly for the first), so no row costs a second cache line.
 constexpr int kTileMaxFloats = 19100;  // gather f32 tile: (32+1)*(16+1)*(32+2) = 19074 fits
 constexpr int kTileMaxWords = 9900;    // scatter int64 tile: (16+1)*(16+1)*(32+2) = 9826 (78.6 KB: 2 WG/CU)
 constexpr int kPlaneMax = 1100;        // (b0+1)*(b1+1) cells of one z plane of a tile
@@ -183,7 +190,6 @@ __device__ __forceinline__ int patch_column_of(int L, int G, int nb0, int nb1) {
   return cx * nb1 + cy;
 }
 
-constexpr int kTileThreads = 512;
 constexpr int kBatch = 8;  // independent loads kept in flight per thread in the runtime-shape tile loops
 
 // Compile-time brick shape when BX > 0 (integer divisions by the tile extents become
@@ -197,6 +203,17 @@ template <int BX, int BY, int BZ>
 struct BrickShape {
   int b0, b1, b2;
   static constexpr bool kVec = BX > 0 && BZ % 4 == 0;
+  // 8 x 8 x 16 bricks (small meshes) on 256 threads, the others on 512
+  static constexpr int NT = BX == 8 ? 256 : 512;
+  // particles of one brick processed per tile staging by the gathers: their results wait in LDS,
+  // so each tile is read once per brick unless the brick holds more (~2x the mean occupancy at
+  // 1/8 particle per cell)
+  static constexpr int CAP = BX == 8 ? 512 : 2048;
+  static constexpr int PPT = CAP / NT;
+  // LDS tile sizes: gather (float), scatter (int64) and one z plane
+  static constexpr int TF = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
+  static constexpr int TW = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxWords;
+  static constexpr int PL = BX ? (BX + 1) * (BY + 1) : kPlaneMax;
   __device__ __forceinline__ explicit BrickShape(const Bricks& k)
       : b0(BX ? BX : k.b[0]), b1(BY ? BY : k.b[1]), b2(BZ ? BZ : k.b[2]) {}
   __device__ __forceinline__ int t0() const { return b0 + 1; }
@@ -212,65 +229,6 @@ struct BrickShape {
   }
 };
 
-// Base cell and fractional offset of a particle for the offset-0, same-cell-size CIC of the
-// force step: bit-identical to axis_cic_same_cell with offset 0 (rem = 0 there).
-__device__ __forceinline__ void base_frac(const int16_t* __restrict__ pmid, const float* __restrict__ disp,
-                                          int64_t j, float a1, const int n[3], int base[3], float f[3]) {
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    float t = disp[j * 3 + a] / a1;
-    float lf = floorf(t);
-    base[a] = pos_mod((int)pmid[j * 3 + a] + (int)lf, n[a]);
-    f[a] = t - lf;
-  }
-}
-
-// Raw particle record (int16 anchor, float32 displacement) held in registers.
-struct PRaw {
-  int p[3];
-  float d[3];
-};
-
-// Loads particles start + threadIdx.x + q * kTileThreads (q < PPT), clamped to end - 1 so every
-// load is unconditional (callers make sure end > start of the particle range).
-template <int PPT>
-__device__ __forceinline__ void load_raw(PRaw* raw, const int16_t* __restrict__ pmid, const float* __restrict__ disp,
-                                         int64_t start, int64_t end) {
-#pragma unroll
-  for (int q = 0; q < PPT; ++q) {
-    int64_t j = start + threadIdx.x + (int64_t)q * kTileThreads;
-    j = j < end ? j : end - 1;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      raw[q].p[a] = pmid[j * 3 + a];
-      raw[q].d[a] = disp[j * 3 + a];
-    }
-  }
-}
-
-// base_frac on a raw record (same arithmetic)
-__device__ __forceinline__ void raw_base_frac(const PRaw& r, float a1, const int n[3], int base[3], float f[3]) {
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    float t = r.d[a] / a1;
-    float lf = floorf(t);
-    base[a] = pos_mod(r.p[a] + (int)lf, n[a]);
-    f[a] = t - lf;
-  }
-}
-
-// Tile cell of a particle's base (corner 0) cell.  The particle was binned by the sort with
-// the brick of this same base cell (pm_sort.hip cell_key: the same float32 division, floor and
-// periodic wrap), so the local index lies inside the brick; the clamp only keeps the LDS
-// access in bounds should that invariant ever be broken.
-template <int BX, int BY, int BZ>
-__device__ __forceinline__ int local_cell(const BrickShape<BX, BY, BZ>& B, const int bs[3], const int o[3]) {
-  int l0 = min(max(bs[0] - o[0], 0), B.b0 - 1);
-  int l1 = min(max(bs[1] - o[1], 0), B.b1 - 1);
-  int l2 = min(max(bs[2] - o[2], 0), B.b2 - 1);
-  return B.cell(l0, l1, l2);
-}
-
 // CIC weight of corner c from the fractional offsets, in the reference's product order
 __device__ __forceinline__ float frac_weight(const float f[3], int c) {
   float wx = (c & 1) ? 1.f - fabsf(f[0] - 1.f) : 1.f - fabsf(f[0]);
@@ -279,73 +237,96 @@ __device__ __forceinline__ float frac_weight(const float f[3], int c) {
   return wx * wy * wz;
 }
 
-__device__ __forceinline__ float unfix(unsigned long long v) { return (float)(long long)v * kUnfix; }
-
 template <int BX, int BY, int BZ>
-__global__ void __launch_bounds__(kTileThreads) k_scatter_columns(
-    const int16_t* __restrict__ pmid, const float* __restrict__ disp, const int32_t* __restrict__ bin_off,
-    float val, Geom g, Bricks k, float* __restrict__ mesh, float* __restrict__ xs, float* __restrict__ ys,
-    unsigned long long* __restrict__ first, const float* __restrict__ vals, const float* __restrict__ vscale) {
-  __shared__ __align__(16) unsigned long long tile[kTileMaxWords];
+__global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_columns(
+    const float4* __restrict__ rec, const int32_t* __restrict__ bin_off, float val, Bricks k, int run,
+    float* __restrict__ mesh, float* __restrict__ xs, float* __restrict__ ys, const float* __restrict__ vals,
+    const float* __restrict__ vscale) {
+  using B_ = BrickShape<BX, BY, BZ>;
+  constexpr int NT = B_::NT;
+  __shared__ __align__(16) unsigned long long tile[B_::TW];
   // per-particle values (sorted order) are brought to |v| <= 1 by vscale[0] before the fixed
   // point and scaled back on output; a constant value is used as it is
   const float vs = vals ? vscale[0] : 1.f;
   const float us = vals ? kUnfix / vs : kUnfix;
-  auto unfix_s = [&](unsigned long long x) { return (float)(long long)x * us; };
-  const BrickShape<BX, BY, BZ> B(k);
+  auto unfix = [&](unsigned long long x) { return (float)(long long)x * us; };
+  const B_ B(k);
   const int col = column_of(blockIdx.x, gridDim.x);
   const int cx = col / k.nb[1], cy = col - cx * k.nb[1];
   const int P = B.pitch(), rows = B.rows(), carry = B.b2 + 1, tf = B.tfloats();
   const int64_t n1 = k.n[1], n2 = k.n[2];
-  for (int i = threadIdx.x; i < tf; i += kTileThreads) tile[i] = 0ull;
-  // Particles stream through the column in chunks of kTileThreads * PPT in index order (the
-  // bricks' bins are contiguous).  The raw loads of the next chunk are issued before the
-  // current one is accumulated, so they are in flight across the flush between bricks.
+  const int bz0 = blockIdx.y * run, bz1 = min(k.nb[2], bz0 + run);
+  const int32_t* off = bin_off + (int64_t)col * k.nb[2];
+  for (int i = threadIdx.x; i < tf; i += NT) tile[i] = 0ull;
+  // Particles stream in chunks of NT * PPT in index order (the bricks' bins are contiguous).  The
+  // loads of the next chunk are issued before the current one is accumulated, so they are in
+  // flight across the flush between bricks.
   constexpr int PPT = 4;
-  constexpr int64_t CH = (int64_t)kTileThreads * PPT;
-  const int64_t col_begin = bin_off[(int64_t)col * k.nb[2]], col_end = bin_off[(int64_t)(col + 1) * k.nb[2]];
-  const bool any = col_end > col_begin;
-  PRaw raw[PPT];
-  if (any) load_raw<PPT>(raw, pmid, disp, col_begin, col_end);
-  __syncthreads();
-  for (int bz = 0; bz < k.nb[2]; ++bz) {
-    const int o[3] = {cx * B.b0, cy * B.b1, bz * B.b2};
-    const int64_t bid = (int64_t)col * k.nb[2] + bz;
-    const int64_t j0 = bin_off[bid], j1 = bin_off[bid + 1];
-    for (int64_t c0 = j0; c0 < j1; c0 += CH) {
-      PRaw cur[PPT];
+  constexpr int64_t CH = (int64_t)NT * PPT;
+  auto load = [&](float4* r, int64_t start, int64_t end) {  // clamped: unconditional (end > start somewhere)
 #pragma unroll
-      for (int q = 0; q < PPT; ++q) cur[q] = raw[q];
-      load_raw<PPT>(raw, pmid, disp, c0 + CH < j1 ? c0 + CH : j1, col_end);  // next chunk
+    for (int q = 0; q < PPT; ++q) {
+      const int64_t j = start + threadIdx.x + (int64_t)q * NT;
+      r[q] = rec[j < end ? j : end - 1];
+    }
+  };
+  auto add = [&](const float4& r, int64_t j, int c0, int c_begin) {  // corners c_begin .. 7 (4: the upper z plane)
+    const float fr[3] = {r.x, r.y, r.z};
+    const float v = vals ? vals[j] * vs : val;
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (c >= c_begin)
+        atomicAdd(&tile[c0 + B.corner_off(c)], (unsigned long long)__float2ll_rn(v * frac_weight(fr, c) * kFix));
+  };
+  const int64_t run0 = off[bz0], run1 = off[bz1];
+  float4 raw[PPT];
+  if (run1 > run0) load(raw, run0, run1);
+  __syncthreads();
+  {
+    // the brick below the run: its last z plane's upper corners are the first brick's z = 0 plane
+    const int bb = bz0 == 0 ? k.nb[2] - 1 : bz0 - 1;
+    const int64_t h0 = off[bb], h1 = off[bb + 1];
+    for (int64_t c0 = h0; c0 < h1; c0 += CH) {
+      float4 h[PPT];
+      load(h, c0, h1);
 #pragma unroll
       for (int q = 0; q < PPT; ++q) {
-        int64_t j = c0 + threadIdx.x + (int64_t)q * kTileThreads;
-        if (j >= j1) continue;
-        int bs[3];
-        float fr[3];
-        raw_base_frac(cur[q], g.a1, k.n, bs, fr);
-        const int c0i = local_cell(B, bs, o);
-        const float v = vals ? vals[j] * vs : val;
+        const int64_t j = c0 + threadIdx.x + (int64_t)q * NT;
+        const uint32_t bits = __float_as_uint(h[q].w);
+        if (j < h1 && sort::rec_top(bits)) add(h[q], j, sort::rec_cell(bits) - B.b2, 4);
+      }
+    }
+  }
+  for (int bz = bz0; bz < bz1; ++bz) {
+    const int o[3] = {cx * B.b0, cy * B.b1, bz * B.b2};
+    const int64_t j0 = off[bz], j1 = off[bz + 1];
+    for (int64_t c0 = j0; c0 < j1; c0 += CH) {
+      float4 cur[PPT];
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-          atomicAdd(&tile[c0i + B.corner_off(c)], (unsigned long long)__float2ll_rn(v * frac_weight(fr, c) * kFix));
+      for (int q = 0; q < PPT; ++q) cur[q] = raw[q];
+      load(raw, c0 + CH < j1 ? c0 + CH : j1, run1);  // next chunk
+#pragma unroll
+      for (int q = 0; q < PPT; ++q) {
+        const int64_t j = c0 + threadIdx.x + (int64_t)q * NT;
+        if (j < j1) add(cur[q], j, sort::rec_cell(__float_as_uint(cur[q].w)), 0);
       }
     }
     __syncthreads();
     // z carry: the plane z = b2 is the next brick's z = 0 plane
-    for (int r = threadIdx.x; r < rows; r += kTileThreads) {
+    for (int r = threadIdx.x; r < rows; r += NT) {
       unsigned long long* row = tile + r * P;
       const unsigned long long cin = row[carry];
       row[carry] = row[B.b2];
+      row[B.b2] = 0ull;
       row[0] += cin;
-      if (bz == 0) first[(int64_t)col * rows + r] = row[0];  // completed after the last brick
     }
     __syncthreads();
-    // owned cells x < b0, y < b1, z < b2, then the x == b0 and y == b1 planes (z < b2)
-    if constexpr (BrickShape<BX, BY, BZ>::kVec) {
+    // owned cells x < b0, y < b1, z < b2, then the x == b0 and y == b1 planes (z < b2); each cell is
+    // cleared for the next brick as it is read
+    if constexpr (B_::kVec) {
       constexpr int C4 = BZ / 4;
       constexpr int OWN = BX * BY * C4, XP = (BY + 1) * C4, YP = BX * C4;
-      for (int it = threadIdx.x; it < OWN + XP + YP; it += kTileThreads) {
+      for (int it = threadIdx.x; it < OWN + XP + YP; it += NT) {
         int x, y, c4;
         float* dst;
         if (it < OWN) {
@@ -367,42 +348,36 @@ __global__ void __launch_bounds__(kTileThreads) k_scatter_columns(
           y = BY;
           dst = &ys[((int64_t)col * BX + x) * n2 + o[2] + 4 * c4];
         }
-        const unsigned long long* src = &tile[B.cell(x, y, 4 * c4)];
-        longlong2 lo = *reinterpret_cast<const longlong2*>(src), hi = *reinterpret_cast<const longlong2*>(src + 2);
+        longlong2* src = reinterpret_cast<longlong2*>(&tile[B.cell(x, y, 4 * c4)]);
+        const longlong2 lo = src[0], hi = src[1];
+        src[0] = src[1] = make_longlong2(0, 0);
         *reinterpret_cast<float4*>(dst) =
             make_float4((float)lo.x * us, (float)lo.y * us, (float)hi.x * us, (float)hi.y * us);
       }
     } else {
       const int own = B.b0 * B.b1 * B.b2, xp = B.t1() * B.b2, yp = B.b0 * B.b2;
-      for (int i = threadIdx.x; i < own + xp + yp; i += kTileThreads) {
+      for (int i = threadIdx.x; i < own + xp + yp; i += NT) {
+        unsigned long long* src;
+        float* dst;
         if (i < own) {
           int r = i / B.b2, z = i - r * B.b2;
           int x = r / B.b1, y = r - x * B.b1;
-          mesh[((int64_t)(o[0] + x) * n1 + (o[1] + y)) * n2 + (o[2] + z)] = unfix_s(tile[B.cell(x, y, z)]);
+          dst = &mesh[((int64_t)(o[0] + x) * n1 + (o[1] + y)) * n2 + (o[2] + z)];
+          src = &tile[B.cell(x, y, z)];
         } else if (i < own + xp) {
           int r = (i - own) / B.b2, z = (i - own) - r * B.b2;
-          xs[((int64_t)col * B.t1() + r) * n2 + o[2] + z] = unfix_s(tile[B.cell(B.b0, r, z)]);
+          dst = &xs[((int64_t)col * B.t1() + r) * n2 + o[2] + z];
+          src = &tile[B.cell(B.b0, r, z)];
         } else {
           int r = (i - own - xp) / B.b2, z = (i - own - xp) - r * B.b2;
-          ys[((int64_t)col * B.b0 + r) * n2 + o[2] + z] = unfix_s(tile[B.cell(r, B.b1, z)]);
+          dst = &ys[((int64_t)col * B.b0 + r) * n2 + o[2] + z];
+          src = &tile[B.cell(r, B.b1, z)];
         }
+        *dst = unfix(*src);
+        *src = 0ull;
       }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < tf; i += kTileThreads)
-      if (i % P != carry) tile[i] = 0ull;
-    __syncthreads();
-  }
-  // the first brick's z = 0 plane: its own part plus the carry of the last brick (periodic)
-  for (int r = threadIdx.x; r < rows; r += kTileThreads) {
-    const int x = r / B.t1(), y = r - x * B.t1();
-    const float v = unfix_s(first[(int64_t)col * rows + r] + tile[r * P + carry]);
-    if (x < B.b0 && y < B.b1)
-      mesh[((int64_t)(cx * B.b0 + x) * n1 + (cy * B.b1 + y)) * n2] = v;
-    else if (x == B.b0)
-      xs[((int64_t)col * B.t1() + y) * n2] = v;
-    else
-      ys[((int64_t)col * B.b0 + x) * n2] = v;
   }
 }
 
@@ -453,28 +428,23 @@ __global__ void __launch_bounds__(kBlock) k_fold_xy(Bricks k, const float* __res
   }
 }
 
-// Particles of one brick processed per tile staging: their three interpolated components
-// wait in LDS, so each component tile is read from HBM once per brick unless the brick holds
-// more than kGatherCap particles (rare: ~2x the mean occupancy at 1/8 particle per cell).
-constexpr int kGatherCap = 2048;
-constexpr int kGatherPPT = kGatherCap / kTileThreads;
-
 // Stage rows z in [0, b2) of one component's tile for brick (cx, cy, bz) (rows wrap in x, y).
 template <int BX, int BY, int BZ>
 __device__ __forceinline__ void stage_rows(float* tile, const float* __restrict__ F, const BrickShape<BX, BY, BZ>& B,
                                            const Bricks& k, int cx, int cy, int bz) {
+  constexpr int NT = BrickShape<BX, BY, BZ>::NT;
   const int ox = cx * B.b0, oy = cy * B.b1, oz = bz * B.b2;
   if constexpr (BrickShape<BX, BY, BZ>::kVec) {
     constexpr int C4 = BZ / 4;
     constexpr int ITEMS = (BX + 1) * (BY + 1) * C4;
-    constexpr int ONE = (ITEMS + kTileThreads - 1) / kTileThreads;
+    constexpr int ONE = (ITEMS + NT - 1) / NT;
     constexpr int ROUND = ONE <= 6 ? ONE : 4;
 #pragma unroll 1
-    for (int base = 0; base < ITEMS; base += ROUND * kTileThreads) {
+    for (int base = 0; base < ITEMS; base += ROUND * NT) {
       float4 v[ROUND];
 #pragma unroll
       for (int u = 0; u < ROUND; ++u) {  // unconditional (clamped) loads: the round stays in flight
-        int it = min(base + (int)threadIdx.x + u * kTileThreads, ITEMS - 1);
+        int it = min(base + (int)threadIdx.x + u * NT, ITEMS - 1);
         int r = it / C4, c4 = it - r * C4;
         int x = r / (BY + 1), y = r - x * (BY + 1);
         int gx = ox + x, gy = oy + y;
@@ -484,7 +454,7 @@ __device__ __forceinline__ void stage_rows(float* tile, const float* __restrict_
       }
 #pragma unroll
       for (int u = 0; u < ROUND; ++u) {
-        int it = base + threadIdx.x + u * kTileThreads;
+        int it = base + threadIdx.x + u * NT;
         if (it < ITEMS) {
           int r = it / C4, c4 = it - r * C4;
           float* dst = &tile[r * (BZ + 2) + 4 * c4];
@@ -496,12 +466,12 @@ __device__ __forceinline__ void stage_rows(float* tile, const float* __restrict_
   } else {
     const int t1 = B.t1(), b2 = B.b2, P = B.pitch();
     const int items = B.rows() * b2;
-    for (int i0 = 0; i0 < items; i0 += kTileThreads * kBatch) {
+    for (int i0 = 0; i0 < items; i0 += NT * kBatch) {
       float v[kBatch];
       int dst[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        int iu = i0 + u * kTileThreads + (int)threadIdx.x;
+        int iu = i0 + u * NT + (int)threadIdx.x;
         int i = min(iu, items - 1);
         int r = i / b2, z = i - r * b2;
         int x = r / t1, y = r - x * t1;
@@ -522,8 +492,9 @@ __device__ __forceinline__ void stage_rows(float* tile, const float* __restrict_
 template <int BX, int BY, int BZ>
 __device__ __forceinline__ void load_plane(float* plane, const float* __restrict__ F, const BrickShape<BX, BY, BZ>& B,
                                            const Bricks& k, int cx, int cy, int bz) {
+  constexpr int NT = BrickShape<BX, BY, BZ>::NT;
   const int t1 = B.t1();
-  for (int r = threadIdx.x; r < B.rows(); r += kTileThreads) {
+  for (int r = threadIdx.x; r < B.rows(); r += NT) {
     int x = r / t1, y = r - x * t1;
     int gx = cx * B.b0 + x, gy = cy * B.b1 + y;
     gx -= gx >= k.n[0] ? k.n[0] : 0;
@@ -536,8 +507,9 @@ __device__ __forceinline__ void load_plane(float* plane, const float* __restrict
 // a share per workgroup of the column walk that writes the others' (n = 0: nothing to do).
 __device__ __forceinline__ void zero_invalid(const int32_t* __restrict__ perm, int64_t first, int64_t n,
                                              float* __restrict__ out) {
-  for (int64_t j = first + (int64_t)blockIdx.x * kTileThreads + threadIdx.x; j < n;
-       j += (int64_t)gridDim.x * kTileThreads) {
+  const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  for (int64_t j = first + wg * blockDim.x + threadIdx.x; j < n;
+       j += (int64_t)gridDim.x * gridDim.y * blockDim.x) {
     const int64_t i = perm[j];
     out[i * 3 + 0] = 0.f;
     out[i * 3 + 1] = 0.f;
@@ -546,25 +518,26 @@ __device__ __forceinline__ void zero_invalid(const int32_t* __restrict__ perm, i
 }
 
 template <int BX, int BY, int BZ>
-__global__ void __launch_bounds__(kTileThreads) k_gather_columns(
-    const int16_t* __restrict__ pmid, const float* __restrict__ disp, const int32_t* __restrict__ bin_off,
-    const int32_t* __restrict__ perm, Geom g, Bricks k, const float* __restrict__ f0,
-    const float* __restrict__ f1, const float* __restrict__ f2, int64_t nzero, float* __restrict__ acc) {
-  constexpr int kLds = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
-  constexpr int kPl = BX ? (BX + 1) * (BY + 1) : kPlaneMax;
-  __shared__ __align__(16) float tile[kLds];
-  __shared__ float res[3][kGatherCap];
-  __shared__ float plane[2][3][kPl];  // [parity of bz][component]: lower z plane of brick bz
-  const BrickShape<BX, BY, BZ> B(k);
+__global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_gather_columns(
+    const float4* __restrict__ rec, const int32_t* __restrict__ bin_off, const int32_t* __restrict__ perm, Bricks k,
+    int run, const float* __restrict__ f0, const float* __restrict__ f1, const float* __restrict__ f2, int64_t nzero,
+    float* __restrict__ acc) {
+  using B_ = BrickShape<BX, BY, BZ>;
+  constexpr int NT = B_::NT, CAP = B_::CAP, PPT = B_::PPT;
+  __shared__ __align__(16) float tile[B_::TF];
+  __shared__ float res[3][CAP];
+  __shared__ float plane[2][3][B_::PL];  // [parity of bz][component]: lower z plane of brick bz
+  const B_ B(k);
   const int col = patch_column_of(blockIdx.x, gridDim.x, k.nb[0], k.nb[1]);
   const int cx = col / k.nb[1], cy = col - cx * k.nb[1];
   const int rows = B.rows(), P = B.pitch(), nb2 = k.nb[2];
-  // the brick above the top one is brick 0 (periodic)
-  load_plane(plane[nb2 & 1][0], f0, B, k, cx, cy, 0);
-  load_plane(plane[nb2 & 1][1], f1, B, k, cx, cy, 0);
-  load_plane(plane[nb2 & 1][2], f2, B, k, cx, cy, 0);
-  for (int bz = nb2 - 1; bz >= 0; --bz) {
-    const int o[3] = {cx * B.b0, cy * B.b1, bz * B.b2};
+  const int bz0 = blockIdx.y * run, bz1 = min(nb2, bz0 + run);
+  // the brick above the run (above the top one: brick 0, periodic)
+  const int above = bz1 == nb2 ? 0 : bz1;
+  load_plane(plane[bz1 & 1][0], f0, B, k, cx, cy, above);
+  load_plane(plane[bz1 & 1][1], f1, B, k, cx, cy, above);
+  load_plane(plane[bz1 & 1][2], f2, B, k, cx, cy, above);
+  for (int bz = bz1 - 1; bz >= bz0; --bz) {
     const int64_t bid = (int64_t)col * nb2 + bz;
     const int64_t j0 = bin_off[bid], j1 = bin_off[bid + 1];
     const int up = (bz + 1) & 1, me = bz & 1;
@@ -575,41 +548,40 @@ __global__ void __launch_bounds__(kTileThreads) k_gather_columns(
       load_plane(plane[me][2], f2, B, k, cx, cy, bz);
       continue;
     }
-    for (int64_t s0 = j0; s0 < j1; s0 += kGatherCap) {
-      const int64_t s1 = s0 + kGatherCap < j1 ? s0 + kGatherCap : j1;
-      // each particle's tile cell and fractions, once for the three components (clamped
-      // loads; their latency overlaps the first tile's staging)
-      int c0[kGatherPPT];
-      float fr[kGatherPPT][3];
+    for (int64_t s0 = j0; s0 < j1; s0 += CAP) {
+      const int64_t s1 = s0 + CAP < j1 ? s0 + CAP : j1;
+      // each particle's record, once for the three components (clamped loads; their latency
+      // overlaps the first tile's staging)
+      float4 r[PPT];
 #pragma unroll
-      for (int q = 0; q < kGatherPPT; ++q) {
-        int64_t j = s0 + threadIdx.x + (int64_t)q * kTileThreads;
-        int bs[3];
-        base_frac(pmid, disp, j < s1 ? j : s1 - 1, g.a1, k.n, bs, fr[q]);
-        c0[q] = local_cell(B, bs, o);
+      for (int q = 0; q < PPT; ++q) {
+        const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
+        r[q] = rec[j < s1 ? j : s1 - 1];
       }
 #pragma unroll 1
       for (int comp = 0; comp < 3; ++comp) {
         const float* __restrict__ F = comp == 0 ? f0 : (comp == 1 ? f1 : f2);
         __syncthreads();  // the previous component's interpolation is done with the tile
         stage_rows<BX, BY, BZ>(tile, F, B, k, cx, cy, bz);
-        for (int r = threadIdx.x; r < rows; r += kTileThreads) tile[r * P + B.b2] = plane[up][comp][r];
+        for (int i = threadIdx.x; i < rows; i += NT) tile[i * P + B.b2] = plane[up][comp][i];
         __syncthreads();
-        for (int r = threadIdx.x; r < rows; r += kTileThreads) plane[me][comp][r] = tile[r * P];
+        for (int i = threadIdx.x; i < rows; i += NT) plane[me][comp][i] = tile[i * P];
 #pragma unroll
-        for (int q = 0; q < kGatherPPT; ++q) {
-          const int jl = threadIdx.x + q * kTileThreads;
+        for (int q = 0; q < PPT; ++q) {
+          const int jl = threadIdx.x + q * NT;
           if (s0 + jl >= s1) continue;
+          const float fr[3] = {r[q].x, r[q].y, r[q].z};
+          const int c0 = sort::rec_cell(__float_as_uint(r[q].w));
           float sum = 0.f;
 #pragma unroll
-          for (int c = 0; c < 8; ++c) sum = sum + tile[c0[q] + B.corner_off(c)] * frac_weight(fr[q], c);
+          for (int c = 0; c < 8; ++c) sum = sum + tile[c0 + B.corner_off(c)] * frac_weight(fr, c);
           res[comp][jl] = sum;
         }
       }
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < kGatherPPT; ++q) {
-        const int jl = threadIdx.x + q * kTileThreads;
+      for (int q = 0; q < PPT; ++q) {
+        const int jl = threadIdx.x + q * NT;
         if (s0 + jl < s1) {
           int64_t i = perm[s0 + jl];
           acc[i * 3 + 0] = res[0][jl];
@@ -631,27 +603,28 @@ __global__ void __launch_bounds__(kTileThreads) k_gather_columns(
 // 0 (the corner_grad convention).  Each mesh's tile is staged in turn; a particle's partial sums
 // wait in its thread's own LDS slots.  With a zero particle value the density term is skipped.
 template <int BX, int BY, int BZ>
-__global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
-    const int16_t* __restrict__ pmid, const float* __restrict__ disp, const int32_t* __restrict__ bin_off,
-    const int32_t* __restrict__ perm, Geom g, Bricks k, const float* __restrict__ f0, const float* __restrict__ f1,
-    const float* __restrict__ f2, const float* __restrict__ dcot, const float* __restrict__ cot_s, int64_t n,
-    float val, int64_t nzero, float* __restrict__ disp_cot, int accum) {
-  constexpr int kLds = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
-  constexpr int kPl = BX ? (BX + 1) * (BY + 1) : kPlaneMax;
-  __shared__ __align__(16) float tile[kLds];
-  __shared__ float res[3][kGatherCap];
-  __shared__ float plane[2][4][kPl];  // [parity of bz][mesh]: lower z plane of brick bz
-  const BrickShape<BX, BY, BZ> B(k);
+__global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_columns(
+    const float4* __restrict__ rec, const int32_t* __restrict__ bin_off, const int32_t* __restrict__ perm, float cell,
+    Bricks k, int run, const float* __restrict__ f0, const float* __restrict__ f1, const float* __restrict__ f2,
+    const float* __restrict__ dcot, const float* __restrict__ cot_s, int64_t n, float val, int64_t nzero,
+    float* __restrict__ disp_cot, int accum) {
+  using B_ = BrickShape<BX, BY, BZ>;
+  constexpr int NT = B_::NT, CAP = B_::CAP, PPT = B_::PPT;
+  __shared__ __align__(16) float tile[B_::TF];
+  __shared__ float res[3][CAP];
+  __shared__ float plane[2][4][B_::PL];  // [parity of bz][mesh]: lower z plane of brick bz
+  const B_ B(k);
   const int col = patch_column_of(blockIdx.x, gridDim.x, k.nb[0], k.nb[1]);
   const int cx = col / k.nb[1], cy = col - cx * k.nb[1];
   const int rows = B.rows(), P = B.pitch(), nb2 = k.nb[2];
   const int nm = val != 0.f ? 4 : 3;
   const int m0 = f0 ? 0 : 3;  // the first mesh: the force components, or the density cotangent alone
-  // the brick above the top one is brick 0 (periodic)
+  const int bz0 = blockIdx.y * run, bz1 = min(nb2, bz0 + run);
+  // the brick above the run (above the top one: brick 0, periodic)
+  const int above = bz1 == nb2 ? 0 : bz1;
   for (int m = m0; m < nm; ++m)
-    load_plane(plane[nb2 & 1][m], m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot)), B, k, cx, cy, 0);
-  for (int bz = nb2 - 1; bz >= 0; --bz) {
-    const int o[3] = {cx * B.b0, cy * B.b1, bz * B.b2};
+    load_plane(plane[bz1 & 1][m], m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot)), B, k, cx, cy, above);
+  for (int bz = bz1 - 1; bz >= bz0; --bz) {
     const int64_t bid = (int64_t)col * nb2 + bz;
     const int64_t j0 = bin_off[bid], j1 = bin_off[bid + 1];
     const int up = (bz + 1) & 1, me = bz & 1;
@@ -661,40 +634,39 @@ __global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
         load_plane(plane[me][m], m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot)), B, k, cx, cy, bz);
       continue;
     }
-    for (int64_t s0 = j0; s0 < j1; s0 += kGatherCap) {
-      const int64_t s1 = s0 + kGatherCap < j1 ? s0 + kGatherCap : j1;
-      // each particle's tile cell and fractions, once for every mesh
-      int c0[kGatherPPT];
-      float fr[kGatherPPT][3];
+    for (int64_t s0 = j0; s0 < j1; s0 += CAP) {
+      const int64_t s1 = s0 + CAP < j1 ? s0 + CAP : j1;
+      // each particle's record, once for every mesh
+      float4 r[PPT];
 #pragma unroll
-      for (int q = 0; q < kGatherPPT; ++q) {
-        int64_t j = s0 + threadIdx.x + (int64_t)q * kTileThreads;
-        int bs[3];
-        base_frac(pmid, disp, j < s1 ? j : s1 - 1, g.a1, k.n, bs, fr[q]);
-        c0[q] = local_cell(B, bs, o);
+      for (int q = 0; q < PPT; ++q) {
+        const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
+        r[q] = rec[j < s1 ? j : s1 - 1];
       }
 #pragma unroll 1
       for (int m = m0; m < nm; ++m) {
         const float* __restrict__ F = m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot));
         __syncthreads();  // the previous mesh's pass is done with the tile
         stage_rows<BX, BY, BZ>(tile, F, B, k, cx, cy, bz);
-        for (int r = threadIdx.x; r < rows; r += kTileThreads) tile[r * P + B.b2] = plane[up][m][r];
+        for (int i = threadIdx.x; i < rows; i += NT) tile[i * P + B.b2] = plane[up][m][i];
         __syncthreads();
-        for (int r = threadIdx.x; r < rows; r += kTileThreads) plane[me][m][r] = tile[r * P];
-        float cf[kGatherPPT];
+        for (int i = threadIdx.x; i < rows; i += NT) plane[me][m][i] = tile[i * P];
+        float cf[PPT];
 #pragma unroll
-        for (int q = 0; q < kGatherPPT; ++q) {  // this mesh's coefficients (clamped loads)
-          const int64_t j = s0 + threadIdx.x + (int64_t)q * kTileThreads;
+        for (int q = 0; q < PPT; ++q) {  // this mesh's coefficients (clamped loads)
+          const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
           cf[q] = m < 3 ? cot_s[(int64_t)m * n + (j < s1 ? j : s1 - 1)] : val;
         }
 #pragma unroll
-        for (int q = 0; q < kGatherPPT; ++q) {
-          const int jl = threadIdx.x + q * kTileThreads;
+        for (int q = 0; q < PPT; ++q) {
+          const int jl = threadIdx.x + q * NT;
           if (s0 + jl >= s1) continue;
+          const float fr[3] = {r[q].x, r[q].y, r[q].z};
+          const int c0 = sort::rec_cell(__float_as_uint(r[q].w));
           float w[3][2], sg[3][2];
 #pragma unroll
           for (int a = 0; a < 3; ++a) {
-            float f = fr[q][a];
+            float f = fr[a];
             asm volatile("" : "+v"(f));  // weights per mesh pass: kept out of registers between passes
 #pragma unroll
             for (int bb = 0; bb < 2; ++bb) {
@@ -707,7 +679,7 @@ __global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
             const int bx = c & 1, by = (c >> 1) & 1, bzz = (c >> 2) & 1;
-            const float v = tile[c0[q] + B.corner_off(c)];
+            const float v = tile[c0 + B.corner_off(c)];
             gs[0] = gs[0] + v * (sg[0][bx] * w[1][by] * w[2][bzz]);
             gs[1] = gs[1] + v * (w[0][bx] * sg[1][by] * w[2][bzz]);
             gs[2] = gs[2] + v * (w[0][bx] * w[1][by] * sg[2][bzz]);
@@ -718,12 +690,12 @@ __global__ void __launch_bounds__(kTileThreads) k_disp_cot_columns(
       }
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < kGatherPPT; ++q) {
-        const int jl = threadIdx.x + q * kTileThreads;
+      for (int q = 0; q < PPT; ++q) {
+        const int jl = threadIdx.x + q * NT;
         if (s0 + jl < s1) {
           const int64_t i = perm[s0 + jl];
 #pragma unroll
-          for (int a = 0; a < 3; ++a) disp_cot[i * 3 + a] = (accum ? disp_cot[i * 3 + a] : 0.f) + res[a][jl] / g.a1;
+          for (int a = 0; a < 3; ++a) disp_cot[i * 3 + a] = (accum ? disp_cot[i * 3 + a] : 0.f) + res[a][jl] / cell;
         }
       }
     }
@@ -958,16 +930,11 @@ int check_desc(const pm_gravity_desc* d, int64_t n) {
 constexpr int kCotBlocks = 1024;  // blocks of k_cot_sorted (and slots of their maxima)
 
 struct Buffers {
-  int32_t* perm;
-  int16_t* pmid_s;
-  float* disp_s;
-  uint8_t* valid_s;
+  sort::Sorted srt;  // the bucketed particles: records when tiled, else the sorted payload
   float* tables;
-  int32_t* bins;   // brick offsets of the bucketed particles
   bool tiled;      // brick-tiled scatter/gather (the brick divides the mesh and fits LDS)
   float* xs;       // upper x / y planes of every brick column (tiled scatter)
   float* ys;
-  unsigned long long* first;  // first brick's lower z plane per column (tiled scatter)
   float* r0;  // density, then F_x
   float* r1;  // F_y
   float* r2;  // F_z
@@ -993,22 +960,24 @@ struct Buffers {
 bool carve(Arena& ws, const Layout& L, int64_t n, const int32_t* shape, const int32_t* brick, bool reverse,
            Buffers& b) {
   b.xs = b.ys = nullptr;
-  b.first = nullptr;
   int64_t nbins = 1;
   for (int a = 0; a < 3; ++a) nbins *= ceil_div(shape[a], brick[a]);
-  b.bins = ws.take<int32_t>(nbins + 2);
+  b.srt = sort::Sorted();
+  b.srt.bins = ws.take<int32_t>(nbins + 2);
   b.tiled = tiled_ok(shape, brick);
   if (b.tiled) {
     Bricks k = make_bricks(shape, brick);
-    int64_t ncols = (int64_t)k.nb[0] * k.nb[1];
     b.xs = ws.take<float>(xs_floats(k));
     b.ys = ws.take<float>(ys_floats(k));
-    b.first = ws.take<unsigned long long>(ncols * (k.b[0] + 1) * (k.b[1] + 1));
   }
-  b.perm = ws.take<int32_t>(n);
-  b.pmid_s = ws.take<int16_t>(3 * n);
-  b.disp_s = ws.take<float>(3 * n);
-  b.valid_s = ws.take<uint8_t>(n);
+  b.srt.perm = ws.take<int32_t>(n);
+  if (b.tiled) {
+    b.srt.rec = ws.take<float4>(n);
+  } else {
+    b.srt.pmid = ws.take<int16_t>(3 * n);
+    b.srt.disp = ws.take<float>(3 * n);
+    b.srt.valid = ws.take<uint8_t>(n);
+  }
   b.tables = ws.take<float>(fft::spec_table_floats(shape));
   b.r0 = ws.take<float>(L.nreal);
   b.r1 = ws.take<float>(L.nreal);
@@ -1022,8 +991,9 @@ bool carve(Arena& ws, const Layout& L, int64_t n, const int32_t* shape, const in
   b.cc = ws.take<float2>(L.s1);
   b.cd = ws.take<float2>(L.s2);
   b.ce = ws.take<float2>(L.s1);
-  b.count = ws.take<int32_t>(nbins + 2);
-  b.partial = ws.take<int32_t>(sort::bucket_partials(nbins + 2));
+  const int64_t counters = sort::bucket_count_len(shape, brick);
+  b.count = ws.take<int32_t>(counters);
+  b.partial = ws.take<int32_t>(sort::bucket_partials(counters));
   if (reverse) {
     b.g0 = ws.take<float>(L.nreal);
     b.g1 = ws.take<float>(L.nreal);
@@ -1067,21 +1037,61 @@ int fill(float* p, int64_t n, hipStream_t s) {
   return PM_SUCCESS;
 }
 
+// How the column walks cut their columns: `run` bricks per workgroup.  A cut costs the scatter a
+// second read of a brick's particles and the gathers a strided plane per component, so columns stay
+// whole when there are enough of them for the workgroups the chip holds at once (two per CU of
+// 16 x 16 x 32 bricks; 8 x 8 x 16 ones fit more) and are halved until there are otherwise.  256^3
+// mesh, 128^3 particles, scatter / gather with 256, 512, 1024 and 2048 workgroups wanted: 37 / 91,
+// 33 / 69, 36 / 77, 39 / 83 us; 128^3 mesh in 8 x 8 x 16 bricks with 512, 1024, 2048: 14 / 19, 12 / 17,
+// 13 / 15 us.
+struct Walk {
+  dim3 grid;
+  int run;
+};
+Walk column_walk(const Bricks& k) {
+  const int64_t ncols = (int64_t)k.nb[0] * k.nb[1];
+  const int64_t want = k.b[0] == 8 ? 1024 : 512;
+  int run = k.nb[2];
+  while (run > 1 && ncols * ceil_div(k.nb[2], run) < want) run = (run + 1) / 2;
+  return {dim3((unsigned)ncols, (unsigned)ceil_div(k.nb[2], run)), run};
+}
+
+// The bricks the step uses: the caller's, but 8 x 8 x 16 ones in place of larger ones they divide on
+// meshes of up to kSmallMesh cells, where 16 x 16 x 32 columns are too few workgroups (a 64^3
+// mesh, 32^3 particles: scatter 16 -> 5, gather 17 -> 6 us; 128^3: 28 -> 11, 36 -> 13 us; at 256^3 their
+// additional plane cells cost more, 33 -> 45 and 69 -> 91 us).  The results do not depend on it beyond
+// the rounding of the cells that neighbouring columns share.
+constexpr int64_t kSmallMesh = int64_t(1) << 21;
+int effective_desc(const pm_gravity_desc* d, int64_t n, pm_gravity_desc* out) {
+  PM_TRY(check_desc(d, n));
+  *out = *d;
+  constexpr int small[3] = {8, 8, 16};
+  const int64_t cells = (int64_t)d->mesh_shape[0] * d->mesh_shape[1] * d->mesh_shape[2];
+  bool use = cells <= kSmallMesh && tiled_ok(d->mesh_shape, d->brick);
+  for (int a = 0; a < 3; ++a) use = use && d->brick[a] % small[a] == 0;
+  if (use)
+    for (int a = 0; a < 3; ++a) out->brick[a] = small[a];
+  return PM_SUCCESS;
+}
+
 // Tiled CIC scatter of the bucketed particles into mesh (whose every cell it writes): the
 // constant particle value, or per-particle values vals (sorted order) with vscale[0] * |vals|
 // <= 1; then, with fold, the neighbouring columns' upper x/y planes (otherwise the R2C pass that
 // reads the mesh adds them: fold_planes).
 int scatter_tiled(const pm_gravity_desc* d, const Buffers& b, float* mesh, const float* vals, const float* vscale,
                   bool fold, hipStream_t s) {
-  const Geom g = step_geom(d);
   Bricks k = make_bricks(d->mesh_shape, d->brick);
-  const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
+  const Walk w = column_walk(k);
+  auto launch = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, w.grid, dim3(threads), 0, s, b.srt.rec, b.srt.bins, d->particle_value, k, w.run, mesh,
+                       b.xs, b.ys, vals, vscale);
+  };
   if (is_brick(k, 16, 16, 32))
-    hipLaunchKernelGGL((k_scatter_columns<16, 16, 32>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, d->particle_value, g, k, mesh, b.xs, b.ys, b.first, vals, vscale);
+    launch(k_scatter_columns<16, 16, 32>, BrickShape<16, 16, 32>::NT);
+  else if (is_brick(k, 8, 8, 16))
+    launch(k_scatter_columns<8, 8, 16>, BrickShape<8, 8, 16>::NT);
   else
-    hipLaunchKernelGGL((k_scatter_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, d->particle_value, g, k, mesh, b.xs, b.ys, b.first, vals, vscale);
+    launch(k_scatter_columns<0, 0, 0>, BrickShape<0, 0, 0>::NT);
   PM_LAUNCHED("k_scatter_columns", s);
   if (!fold) return PM_SUCCESS;
   const int64_t plane_cells = ((int64_t)k.nb[0] * k.n[1] + (int64_t)(k.n[0] - k.nb[0]) * k.nb[1]) * k.n[2];
@@ -1105,8 +1115,7 @@ fft::FoldPlanes fold_planes(const pm_gravity_desc* d, const Buffers& b) {
   return f;
 }
 
-// The particles binned by brick into the workspace's sorted copies (b.perm, b.bins, b.pmid_s,
-// b.disp_s, b.valid_s).
+// The particles binned by brick into the workspace's sorted copies (b.srt).
 int bucket_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
                  const pm_gravity_desc* d, Buffers& b, hipStream_t s) {
   // the Lagrangian grid the particle count implies (mesh * cell / spacing per axis)
@@ -1116,8 +1125,8 @@ int bucket_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, i
       const double v = (double)d->mesh_shape[a] * d->cell_size / d->ptcl_spacing;
       grid[a] = (v >= 1.0 && v < 1e9) ? (int32_t)lrint(v) : 0;
     }
-  return sort::bucket_cells(pmid, disp, valid, n, d->mesh_shape, d->cell_size, d->brick, grid, b.perm, b.bins,
-                            b.pmid_s, b.disp_s, b.valid_s, b.count, b.partial, true, s);
+  return sort::bucket_cells(pmid, disp, valid, n, d->mesh_shape, d->cell_size, d->brick, grid, b.srt,
+                            b.count, b.partial, true, s);
 }
 
 // Bucketing by brick (with the payload gathered into bucket order), then the density in b.r0; fold
@@ -1129,53 +1138,56 @@ int density_stage(const int16_t* pmid, const float* disp, const uint8_t* valid, 
   if (b.tiled) return scatter_tiled(d, b, b.r0, nullptr, nullptr, fold, s);
   PM_TRY(fill(b.r0, L.nreal, s));
   if (n > 0) {
-    hipLaunchKernelGGL(k_scatter_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, b.pmid_s, b.disp_s, b.valid_s,
+    hipLaunchKernelGGL(k_scatter_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, b.srt.pmid, b.srt.disp, b.srt.valid,
                        n, d->particle_value, g, b.r0);
     PM_LAUNCHED("k_scatter_sorted", s);
   }
   return PM_SUCCESS;
 }
 
-int gather_stage(const int16_t* pmid_s, const float* disp_s, const uint8_t* valid_s, const uint8_t* valid,
-                 int64_t n, const pm_gravity_desc* d, const Buffers& b, const float* fx, const float* fy,
-                 const float* fz, float* acc, hipStream_t s) {
+int gather_stage(const uint8_t* valid, int64_t n, const pm_gravity_desc* d, const Buffers& b, const float* fx,
+                 const float* fy, const float* fz, float* acc, hipStream_t s) {
   if (n == 0) return PM_SUCCESS;
-  const Geom g = step_geom(d);
   if (b.tiled) {
     Bricks k = make_bricks(d->mesh_shape, d->brick);
-    const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
+    const Walk w = column_walk(k);
     const int64_t nzero = valid ? n : 0;
+    auto launch = [&](auto kern, int threads) {
+      hipLaunchKernelGGL(kern, w.grid, dim3(threads), 0, s, b.srt.rec, b.srt.bins, b.srt.perm, k, w.run, fx, fy, fz,
+                         nzero, acc);
+    };
     if (is_brick(k, 16, 16, 32))
-      hipLaunchKernelGGL((k_gather_columns<16, 16, 32>), dim3(ncols), dim3(kTileThreads), 0, s, pmid_s, disp_s,
-                         b.bins, b.perm, g, k, fx, fy, fz, nzero, acc);
+      launch(k_gather_columns<16, 16, 32>, BrickShape<16, 16, 32>::NT);
+    else if (is_brick(k, 8, 8, 16))
+      launch(k_gather_columns<8, 8, 16>, BrickShape<8, 8, 16>::NT);
     else
-      hipLaunchKernelGGL((k_gather_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, pmid_s, disp_s,
-                         b.bins, b.perm, g, k, fx, fy, fz, nzero, acc);
+      launch(k_gather_columns<0, 0, 0>, BrickShape<0, 0, 0>::NT);
     PM_LAUNCHED("k_gather_columns", s);
     return PM_SUCCESS;
   }
-  hipLaunchKernelGGL(k_gather3_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, pmid_s, disp_s, valid_s, b.perm, n, g,
-                     fx, fy, fz, acc);
+  hipLaunchKernelGGL(k_gather3_sorted, dim3(grid_for(n)), dim3(kBlock), 0, s, b.srt.pmid, b.srt.disp, b.srt.valid,
+                     b.srt.perm, n, step_geom(d), fx, fy, fz, acc);
   PM_LAUNCHED("k_gather3_sorted", s);
   return PM_SUCCESS;
 }
 
-// Tiled displacement cotangent of the reverse pass: F = (b.g0, b.r1, b.r2), the density
-// cotangent in b.g1, the sorted acc_cot copies in b.cot_s; particles outside every brick (the
-// invalid ones) get zero.
-int disp_cot_tiled(const pm_gravity_desc* d, const Buffers& b, int64_t n, const uint8_t* valid, float* disp_cot,
-                   hipStream_t s) {
-  const Geom g = step_geom(d);
+// Tiled displacement cotangent of the reverse pass from the meshes f0, f1, f2 (null: none) and the
+// density cotangent dcot, with the sorted acc_cot copies in b.cot_s; nzero = n: particles outside
+// every brick (the invalid ones) get zero.  accum: added to disp_cot.
+int disp_cot_tiled(const pm_gravity_desc* d, const Buffers& b, int64_t n, const float* f0, const float* f1,
+                   const float* f2, const float* dcot, int64_t nzero, int accum, float* disp_cot, hipStream_t s) {
   Bricks k = make_bricks(d->mesh_shape, d->brick);
-  const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
-  const float val = d->particle_value;
-  const int64_t nzero = valid ? n : 0;
+  const Walk w = column_walk(k);
+  auto launch = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, w.grid, dim3(threads), 0, s, b.srt.rec, b.srt.bins, b.srt.perm, d->cell_size, k, w.run,
+                       f0, f1, f2, dcot, f0 ? b.cot_s : nullptr, n, d->particle_value, nzero, disp_cot, accum);
+  };
   if (is_brick(k, 16, 16, 32))
-    hipLaunchKernelGGL((k_disp_cot_columns<16, 16, 32>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, nzero, disp_cot, 0);
+    launch(k_disp_cot_columns<16, 16, 32>, BrickShape<16, 16, 32>::NT);
+  else if (is_brick(k, 8, 8, 16))
+    launch(k_disp_cot_columns<8, 8, 16>, BrickShape<8, 8, 16>::NT);
   else
-    hipLaunchKernelGGL((k_disp_cot_columns<0, 0, 0>), dim3(ncols), dim3(kTileThreads), 0, s, b.pmid_s, b.disp_s,
-                       b.bins, b.perm, g, k, b.g0, b.r1, b.r2, b.g1, b.cot_s, n, val, nzero, disp_cot, 0);
+    launch(k_disp_cot_columns<0, 0, 0>, BrickShape<0, 0, 0>::NT);
   PM_LAUNCHED("k_disp_cot_columns", s);
   return PM_SUCCESS;
 }
@@ -1418,18 +1430,18 @@ using namespace pm;
 extern "C" {
 
 int pm_gravity_workspace(const pm_gravity_desc* desc, int64_t n, size_t* bytes) {
-  int st = grav::check_desc(desc, n);
-  if (st) return st;
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
   PM_RETURN_IF(bytes == nullptr, PM_ERROR_INVALID_ARGUMENT, "bytes is NULL");
-  *bytes = grav::workspace_bytes(desc, n, false);
+  *bytes = grav::workspace_bytes(&eff, n, false);
   return PM_SUCCESS;
 }
 
 int pm_gravity_vjp_workspace(const pm_gravity_desc* desc, int64_t n, size_t* bytes) {
-  int st = grav::check_desc(desc, n);
-  if (st) return st;
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
   PM_RETURN_IF(bytes == nullptr, PM_ERROR_INVALID_ARGUMENT, "bytes is NULL");
-  *bytes = grav::workspace_bytes(desc, n, true);
+  *bytes = grav::workspace_bytes(&eff, n, true);
   return PM_SUCCESS;
 }
 
@@ -1443,6 +1455,9 @@ int pm_gravity_corrected(const int16_t* pmid, const float* disp, const uint8_t* 
                          const pm_gravity_desc* desc, const float* rho_add, float* acc, void* workspace,
                          size_t workspace_bytes, void* stream) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1455,13 +1470,16 @@ int pm_gravity_corrected(const int16_t* pmid, const float* disp, const uint8_t* 
   if (st) return st;
   st = grav::force_mesh_stage(desc, L, b, tb, s, false, true, rho_add);
   if (st) return st;
-  return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
+  return grav::gather_stage(valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
 }
 
 int pm_gravity_corrected_resume(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
                                 const pm_gravity_desc* desc, const float* rho_add, float* acc, void* workspace,
                                 size_t workspace_bytes, void* stream) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1474,11 +1492,13 @@ int pm_gravity_corrected_resume(const int16_t* pmid, const float* disp, const ui
                "pmid/disp/acc NULL");
   st = grav::force_mesh_stage(desc, L, b, tb, s, false, false, rho_add);
   if (st) return st;
-  return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
+  return grav::gather_stage(valid, n, desc, b, b.r0, b.r1, b.r2, acc, s);
 }
 
 int pm_gravity_density_offset(const pm_gravity_desc* desc, int64_t n, size_t* offset) {
-  PM_TRY(grav::check_desc(desc, n));
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   PM_RETURN_IF(offset == nullptr, PM_ERROR_INVALID_ARGUMENT, "offset is NULL");
   // the forward carve on a stand-in base (never dereferenced): prepare() carves from the
   // workspace start in the same order, so the density's offset is the same there
@@ -1496,6 +1516,9 @@ int pm_gravity_density(const int16_t* pmid, const float* disp, const uint8_t* va
                        const pm_gravity_desc* desc, float* rho, void* workspace, size_t workspace_bytes,
                        void* stream) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1530,6 +1553,9 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
                     float* omega_cot, float* rho_cot, void* workspace, size_t workspace_bytes, void* stream,
                     bool resume) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1554,7 +1580,7 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
   // over F and the density cotangent.
   if (b.tiled) {
     const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, grav::kBlock), grav::kCotBlocks));
-    hipLaunchKernelGGL(grav::k_cot_sorted, dim3(nb), dim3(grav::kBlock), 0, s, b.perm, acc_cot, n, b.cot_s,
+    hipLaunchKernelGGL(grav::k_cot_sorted, dim3(nb), dim3(grav::kBlock), 0, s, b.srt.perm, acc_cot, n, b.cot_s,
                        b.cot_pmax);
     PM_LAUNCHED("k_cot_sorted", s);
     hipLaunchKernelGGL(grav::k_cot_scale, dim3(1), dim3(64), 0, s, b.cot_pmax, (int)nb, b.cot_pmax + grav::kCotBlocks);
@@ -1575,7 +1601,7 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
     if (st) return st;
     if (n > 0) {
       hipLaunchKernelGGL(grav::k_gather3_bwd_sorted, dim3(grav::grid_for(n)), dim3(grav::kBlock), 0, s,
-                         b.pmid_s, b.disp_s, b.valid_s, b.perm, n, g, b.g0, b.r1, b.r2, acc_cot, b.g1, b.g2, b.g3,
+                         b.srt.pmid, b.srt.disp, b.srt.valid, b.srt.perm, n, g, b.g0, b.r1, b.r2, acc_cot, b.g1, b.g2, b.g3,
                          b.disp_cot_s);
       PM_LAUNCHED("k_gather3_bwd_sorted", s);
     }
@@ -1595,10 +1621,11 @@ static int vjp_impl(const int16_t* pmid, const float* disp, const uint8_t* valid
     hipLaunchKernelGGL(grav::k_source_bwd_sum, dim3(1), dim3(64), 0, s, b.src_part, (int)blocks, omega_cot);
     PM_LAUNCHED("k_source_bwd_sum", s);
   }
-  if (n > 0 && b.tiled) return grav::disp_cot_tiled(desc, b, n, valid, disp_cot, s);
+  if (n > 0 && b.tiled)
+    return grav::disp_cot_tiled(desc, b, n, b.g0, b.r1, b.r2, b.g1, valid ? n : 0, 0, disp_cot, s);
   if (n > 0) {
-    hipLaunchKernelGGL(grav::k_scatter_bwd_sorted, dim3(grav::grid_for(n)), dim3(grav::kBlock), 0, s, b.pmid_s,
-                       b.disp_s, b.valid_s, b.perm, n, g, desc->particle_value, b.g1, b.disp_cot_s, disp_cot);
+    hipLaunchKernelGGL(grav::k_scatter_bwd_sorted, dim3(grav::grid_for(n)), dim3(grav::kBlock), 0, s, b.srt.pmid,
+                       b.srt.disp, b.srt.valid, b.srt.perm, n, g, desc->particle_value, b.g1, b.disp_cot_s, disp_cot);
     PM_LAUNCHED("k_scatter_bwd_sorted", s);
   }
   return PM_SUCCESS;
@@ -1615,6 +1642,9 @@ int pm_gravity_corrected_vjp(const int16_t* pmid, const float* disp, const uint8
 int pm_gravity_keep(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
                     const pm_gravity_desc* desc, float* acc, void* workspace, size_t workspace_bytes, void* stream) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1628,7 +1658,7 @@ int pm_gravity_keep(const int16_t* pmid, const float* disp, const uint8_t* valid
   if (st) return st;
   st = grav::force_mesh_stage(desc, L, b, tb, s, true, false, nullptr);
   if (st) return st;
-  return grav::gather_stage(b.pmid_s, b.disp_s, b.valid_s, valid, n, desc, b, b.g0, b.r1, b.r2, acc, s);
+  return grav::gather_stage(valid, n, desc, b, b.g0, b.r1, b.r2, acc, s);
 }
 
 int pm_gravity_vjp_resume(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
@@ -1642,6 +1672,9 @@ int pm_gravity_density_cot(const int16_t* pmid, const float* disp, const uint8_t
                            const pm_gravity_desc* desc, const float* dens_cot, float* disp_cot, void* workspace,
                            size_t workspace_bytes, void* stream) {
   hipStream_t s = as_stream(stream);
+  pm_gravity_desc eff;
+  PM_TRY(grav::effective_desc(desc, n, &eff));
+  desc = &eff;
   grav::Layout L;
   grav::Buffers b{};
   Arena ws(workspace, workspace_bytes);
@@ -1653,23 +1686,10 @@ int pm_gravity_density_cot(const int16_t* pmid, const float* disp, const uint8_t
   if (n == 0) return PM_SUCCESS;
   PM_TRY(grav::bucket_stage(pmid, disp, valid, n, desc, b, s));
   const Geom g = grav::step_geom(desc);
-  const float val = desc->particle_value;
-  if (b.tiled) {  // invalid particles are in no bin: their disp_cot stays as it is
-    grav::Bricks k = grav::make_bricks(desc->mesh_shape, desc->brick);
-    const unsigned ncols = (unsigned)((int64_t)k.nb[0] * k.nb[1]);
-    if (grav::is_brick(k, 16, 16, 32))
-      hipLaunchKernelGGL((grav::k_disp_cot_columns<16, 16, 32>), dim3(ncols), dim3(grav::kTileThreads), 0, s,
-                         b.pmid_s, b.disp_s, b.bins, b.perm, g, k, nullptr, nullptr, nullptr, dens_cot, nullptr, n,
-                         val, (int64_t)0, disp_cot, 1);
-    else
-      hipLaunchKernelGGL((grav::k_disp_cot_columns<0, 0, 0>), dim3(ncols), dim3(grav::kTileThreads), 0, s, b.pmid_s,
-                         b.disp_s, b.bins, b.perm, g, k, nullptr, nullptr, nullptr, dens_cot, nullptr, n, val,
-                         (int64_t)0, disp_cot, 1);
-    PM_LAUNCHED("k_disp_cot_columns", s);
-    return PM_SUCCESS;
-  }
-  hipLaunchKernelGGL(grav::k_scatter_bwd_sorted, dim3(grav::grid_for(n)), dim3(grav::kBlock), 0, s, b.pmid_s,
-                     b.disp_s, b.valid_s, b.perm, n, g, val, dens_cot, nullptr, disp_cot);
+  if (b.tiled)  // invalid particles are in no bin: their disp_cot stays as it is
+    return grav::disp_cot_tiled(desc, b, n, nullptr, nullptr, nullptr, dens_cot, 0, 1, disp_cot, s);
+  hipLaunchKernelGGL(grav::k_scatter_bwd_sorted, dim3(grav::grid_for(n)), dim3(grav::kBlock), 0, s, b.srt.pmid,
+                     b.srt.disp, b.srt.valid, b.srt.perm, n, g, desc->particle_value, dens_cot, nullptr, disp_cot);
   PM_LAUNCHED("k_scatter_bwd_sorted", s);
   return PM_SUCCESS;
 }

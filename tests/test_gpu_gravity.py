@@ -294,3 +294,52 @@ def test_particle_subsets_empty_sets_and_all_invalid(device):
     assert tuple(gravity(1.0, empty, 0.3, conf).shape) == (0, 3)
     dead = full.replace(unused_index=torch.ones(len(full), dtype=torch.bool, device=device))
     assert torch.all(gravity(1.0, dead, 0.3, conf) == 0)
+
+
+@pytest.mark.parametrize("mesh,grid,clustered,valid_frac", [
+    ((64, 64, 64), (32, 32, 32), False, None),      # 8 x 8 x 16 bricks, columns cut into runs of one brick
+    ((128, 64, 256), (64, 32, 128), True, 0.9),     # the largest mesh that takes them, more than one round a brick
+    ((16, 16, 32), (16, 16, 32), False, 0.8),       # one caller's brick of 16 x 16 x 32: 2 x 2 x 2 of them
+    ((128, 128, 256), (32, 32, 64), False, 0.9),    # 16 x 16 x 32 bricks, columns of 8 cut into runs
+    ((256, 32, 512), (64, 8, 128), True, None),     # the same, 2 columns along y, clustered
+    ((512, 256, 64), (64, 32, 8), False, 0.5),      # 512 columns of two bricks: whole columns
+])
+def test_column_runs_and_brick_sizes_match_oracle(device, mesh, grid, clustered, valid_frac):
+    """Force and VJP where the column walks take each brick size and cut their columns into runs
+    (the lower plane of a run's first brick comes from the brick below, periodically): 1e-5 and 1e-3
+    of the float64 oracle as everywhere, and the order of the particles changes no bit."""
+    from pmpp_amd.nbody.gravity import gravity_vjp
+
+    conf = Configuration(2.0, grid, mesh_shape=mesh)
+    rng = np.random.default_rng(sum(mesh))
+    base = Particles.gen_grid(conf, device=device)
+    disp = base.disp.cpu().numpy() + (rng.normal(size=base.disp.shape) * 1.3 * conf.cell_size).astype(np.float32)
+    pm = base.pmid.cpu().numpy()
+    if clustered:  # a third of the particles in a few cells across a brick corner and the wrap
+        k = len(pm) // 3
+        pm = pm.copy()
+        pm[:k] = rng.integers(-1, 2, size=(k, 3)) + np.array(mesh) // 2
+        pm[: k // 4] = rng.integers(-1, 1, size=(k // 4, 3)) % np.array(mesh)
+    unused = None if valid_frac is None else torch.as_tensor(rng.random(len(pm)) > valid_frac, device=device)
+    ptcl = base.replace(pmid=torch.as_tensor(pm.astype(np.int16), device=device),
+                        disp=torch.as_tensor(disp.astype(np.float32), device=device), unused_index=unused)
+    valid = None if unused is None else ~unused.cpu().numpy()
+    masks = spectral.particle_nyquist_masks(conf.mesh_shape, conf.ptcl_grid_shape, conf.ptcl_spacing, conf.cell_size)
+    p64, d64 = pm.astype(np.int64), disp.astype(np.float32).astype(np.float64)
+    acc = gravity(1.0, ptcl, 0.3, conf)
+    ref = spectral.gravity(p64, d64, 0.3, conf.mesh_shape, conf.cell_size, conf.ptcl_num, masks, valid=valid)
+    got = acc.cpu().numpy()
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 1e-5
+    if valid is not None:
+        assert np.all(got[~valid] == 0)
+    cot = rng.normal(size=got.shape).astype(np.float32)
+    cosmo = type("C", (), {"Omega_m": 0.3})()
+    d_gpu, o_gpu = gravity_vjp(ptcl, cosmo, conf, torch.as_tensor(cot, device=device))
+    dref, oref = spectral.gravity_vjp(p64, d64, 0.3, cot, conf.mesh_shape, conf.cell_size, conf.ptcl_num, masks,
+                                      valid=valid)
+    assert np.linalg.norm(d_gpu.cpu().numpy() - dref) / np.linalg.norm(dref) < 1e-3
+    assert o_gpu == pytest.approx(oref, rel=1e-3)
+    order = torch.as_tensor(rng.permutation(len(pm)), device=device)
+    shuffled = ptcl.replace(pmid=ptcl.pmid[order].contiguous(), disp=ptcl.disp[order].contiguous(),
+                            unused_index=None if unused is None else unused[order].contiguous())
+    assert torch.equal(gravity(1.0, shuffled, 0.3, conf), acc[order])

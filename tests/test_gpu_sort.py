@@ -105,6 +105,38 @@ def hip_bucket(pmid, disp, valid, mesh_shape, cell, brick, grid, dev):
     return perm.cpu().numpy(), offs.cpu().numpy(), pm_s.cpu().numpy(), dp_s.cpu().numpy(), v_s.cpu().numpy()
 
 
+@pytest.mark.parametrize("grid", [(96, 96, 64), (100, 101, 60), (130, 129, 128), (120, 120, 121), (17, 300, 40)])
+@pytest.mark.parametrize("valid_frac,shift", [(None, 0), (0.7, 0), (0.02, 1)])
+def test_bucketing_at_every_chunk_level(device, grid, valid_frac, shift):
+    """Sizes of all three chunk levels, grids whose blocks divide, whose blocks are partly empty
+    (rows of 60 and 121) and that count as index ranges (rows of 40); few and many invalid particles
+    over the counters they share; arrays off 16-byte alignment (shift) and rows that start off it."""
+    mesh, brick, cell = tuple(2 * g for g in grid), (16, 16, 32), 0.5
+    rng = np.random.default_rng(sum(grid))
+    n = int(np.prod(grid))
+    pm = np.stack(np.meshgrid(*[2 * np.arange(g) for g in grid], indexing="ij"), -1).reshape(-1, 3)
+    P = torch.empty((n + 1) * 3, dtype=torch.int16, device=device)[3 * shift:3 * (n + shift)].view(n, 3)
+    D = torch.empty((n + 1) * 3, dtype=torch.float32, device=device)[3 * shift:3 * (n + shift)].view(n, 3)
+    P.copy_(torch.as_tensor(pm.astype(np.int16)))
+    disp = (rng.normal(size=(n, 3)) * 0.8).astype(np.float32)
+    D.copy_(torch.as_tensor(disp))
+    valid = None if valid_frac is None else rng.random(n) < valid_frac
+    perm, offs, pm_s, dp_s, v_s = hip_bucket(P, D, valid, mesh, cell, brick, grid, device)
+    cells = np.mod(pm + np.floor(disp / np.float32(cell)).astype(np.int64), mesh)
+    nb = [-(-m // b) for m, b in zip(mesh, brick)]
+    key = ((cells[:, 0] // brick[0]) * nb[1] + cells[:, 1] // brick[1]) * nb[2] + cells[:, 2] // brick[2]
+    if valid is not None:
+        key = np.where(valid, key, int(np.prod(nb)))
+    count = np.bincount(key, minlength=int(np.prod(nb)) + 1)
+    np.testing.assert_array_equal(offs, np.concatenate([[0], np.cumsum(count)]))
+    np.testing.assert_array_equal(key[perm], np.sort(key))
+    assert np.array_equal(np.sort(perm), np.arange(n))
+    np.testing.assert_array_equal(pm_s, pm[perm])
+    np.testing.assert_array_equal(dp_s.view(np.uint32), disp[perm].view(np.uint32))
+    if valid is not None:
+        np.testing.assert_array_equal(v_s, valid[perm].astype(np.uint8))
+
+
 @pytest.mark.parametrize("grid,hint,valid_frac", [
     ((8, 8, 64), True, None),     # particle-grid chunks (4 x 8 x 64 blocks)
     ((8, 8, 64), False, 0.9),     # contiguous index chunks, invalid particles
@@ -137,12 +169,13 @@ def test_force_step_bucketing_bins_every_particle(device, grid, hint, valid_frac
     np.testing.assert_array_equal(v_s, np.ones(n, np.uint8) if valid is None else valid[perm].astype(np.uint8))
 
 
-@pytest.mark.parametrize("mesh", [(1, 1, 1), (2, 23, 89), (9, 5, 91), (64, 8, 8), (89, 23, 4), (68, 15, 257),
-                                  (27, 133, 73), (64, 64, 65)])
+@pytest.mark.parametrize("mesh", [(1, 1, 1), (29, 139, 1), (52, 31, 5), (37, 109, 1), (64, 8, 8), (89, 23, 4),
+                                  (68, 15, 257), (97, 52, 52), (64, 64, 65)])
 def test_bin_offsets_at_the_edges_of_the_scan(device, mesh):
-    """Bin counts just below, at and above the scan's chunk of 4096 counters (4094, 4095, 4096
-    bins), several chunks, the last size of the single-launch scan (262,140 bins) and the first of
-    the three-launch one (262,143, 266,240): integers, so equal to numpy's."""
+    """Bin counts (plus 65 counters of invalid particles and the end) around the scan's chunk of
+    4096 counters (4031 and 4033 bins on either side), several chunks, a size of the single-launch
+    scan (262,140 bins) and two of the three-launch one (262,288, 266,240): integers, so equal to
+    numpy's."""
     rng = np.random.default_rng(sum(mesh))
     n = 30011
     pmid = np.stack([rng.integers(0, m, n) for m in mesh], 1).astype(np.int16)
