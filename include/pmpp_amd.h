@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PM_ABI_VERSION 10
+#define PM_ABI_VERSION 11
 
 enum pm_status {
   PM_SUCCESS = 0,
@@ -171,6 +171,12 @@ int pm_rfft3d(const float* in, float* out_complex, const int32_t shape[3], void*
               size_t workspace_bytes, void* stream);
 int pm_irfft3d(float* in_complex, float* out, const int32_t shape[3], void* workspace,
                size_t workspace_bytes, void* stream);
+
+/* pm_irfft3d_keep  pm_irfft3d that only reads its input spectrum (a workspace of the size its query
+ *                  gives takes the place of it as scratch). */
+int pm_irfft3d_keep_workspace(const int32_t shape[3], size_t* bytes);
+int pm_irfft3d_keep(const float* in_complex, float* out, const int32_t shape[3], void* workspace,
+                    size_t workspace_bytes, void* stream);
 
 /* Fused spectral force multiplier on a standard-layout spectrum:
  *   out = D_axis(k) * mask(k) * (-1/k^2) * in,  D_axis = -i k_axis (Nyquist derivative 0)
@@ -445,6 +451,17 @@ int pm_to_bf16(const float* src, int64_t n, void* dst, void* stream);
  *                      wavenumber zeroed for i != j (_strain, lpt.py:17-43); 3 -i k_i with the
  *                      Nyquist zeroed (neg_grad, gravity.py:355-391).  A wavenumber is the
  *                      Nyquist when | |k| - nyquist[a] | <= tol[a].
+ *                      op 4: op 0 then op 1.
+ * pm_ic_symbol_inverse out[c] = irfftn(symbol_c(k) in), three real meshes one after the other, in only
+ *                      read: kind 0 the strains -k_i k_i, 1 the strains -k_0 k_1, -k_0 k_2, -k_1 k_2, 2
+ *                      the gradient -i k_i (the Nyquist rules of ops 2 and 3); workspace from the
+ *                      query.  FFT axes as pm_irfft3d.
+ * pm_ic_lpt2_source    the 2LPT source (_L, lpt.py:239-302) of six strain meshes of n cells one after
+ *                      the other, kind 0's then kind 1's.
+ * pm_ic_lpt_particles  particles on the Lagrangian grid of a mesh (nbody/particles.py:615-727): pmid,
+ *                      and disp = the lattice's own + D1 grad1 + D2 grad2, vel = V1 grad1 + V2 grad2
+ *                      (lpt.py:419-436) for gradients of kind 2 on that grid (NULL: no such term); vel
+ *                      may be NULL.
  * pm_ic_product_acc    acc = (init ? 0 : acc) + coef a b elementwise (b = NULL: + coef a); the
  *                      2LPT source (_L, lpt.py:239-302) and the sums of its adjoint
  * pm_ic_lpt_accumulate disp[:, axis] += D grad, vel[:, axis] += V grad (vel may be NULL) for
@@ -457,6 +474,14 @@ int pm_ic_spectral_op(const float* in, float* out, const int32_t shape[3], const
                       void* stream);
 int pm_ic_product_acc(float* acc, const float* a, const float* b, int64_t n, float coef, int32_t init,
                       void* stream);
+int pm_ic_symbol_inverse_workspace(const int32_t shape[3], size_t* bytes);
+int pm_ic_symbol_inverse(const float* in, float* out, const int32_t shape[3], const float* const ktab[3], int32_t kind,
+                         const float nyquist[3], const float tol[3], void* workspace, size_t workspace_bytes,
+                         void* stream);
+int pm_ic_lpt2_source(const float* strains, int64_t n, float* out, void* stream);
+int pm_ic_lpt_particles(const int32_t grid[3], const int32_t mesh[3], double cell_size, const float* grad1,
+                        const float* grad2, float D1, float V1, float D2, float V2, int16_t* pmid, float* disp,
+                        float* vel, void* stream);
 int pm_ic_lpt_accumulate(float* disp, float* vel, const float* grad, int64_t n, int32_t axis, float D, float V,
                          void* stream);
 

@@ -14,7 +14,7 @@ import ctypes
 import os
 from pathlib import Path
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 PM_SUCCESS = 0
 PM_ERROR_INVALID_ARGUMENT = 1
@@ -29,7 +29,7 @@ EXPORTED_SYMBOLS = (
     "pm_cic_scatter", "pm_cic_gather", "pm_cic_gather_bwd", "pm_cic_scatter_bwd",
     "pm_sort_cells_workspace", "pm_sort_cells", "pm_bucket_cells_workspace", "pm_bucket_cells",
     "pm_bucket_cells_noalloc",
-    "pm_fft_workspace", "pm_rfft3d", "pm_irfft3d",
+    "pm_fft_workspace", "pm_rfft3d", "pm_irfft3d", "pm_irfft3d_keep_workspace", "pm_irfft3d_keep",
     "pm_spectral_workspace", "pm_spectral_force_multiply",
     "pm_gravity_workspace", "pm_gravity_vjp_workspace", "pm_gravity", "pm_gravity_vjp",
     "pm_gravity_keep", "pm_gravity_vjp_resume",
@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "pm_correction_workspace", "pm_correction_features", "pm_correction_residual", "pm_correction_residual_bwd",
     "pm_correction_input_bwd", "pm_force_loss", "pm_adamax_step", "pm_to_bf16",
     "pm_ic_linear_modes", "pm_ic_spectral_op", "pm_ic_product_acc", "pm_ic_lpt_accumulate",
+    "pm_ic_symbol_inverse_workspace", "pm_ic_symbol_inverse", "pm_ic_lpt2_source", "pm_ic_lpt_particles",
 )
 
 
@@ -103,6 +104,8 @@ _SIGNATURES = {
                                 ctypes.c_int),
     "pm_fft_workspace": ([_i32x3, _sz_p], ctypes.c_int),
     "pm_rfft3d": ([_vp, _vp, _i32x3, _vp, ctypes.c_size_t, _vp], ctypes.c_int),
+    "pm_irfft3d_keep_workspace": ([_i32x3, _sz_p], ctypes.c_int),
+    "pm_irfft3d_keep": ([_vp, _vp, _i32x3, _vp, ctypes.c_size_t, _vp], ctypes.c_int),
     "pm_irfft3d": ([_vp, _vp, _i32x3, _vp, ctypes.c_size_t, _vp], ctypes.c_int),
     "pm_spectral_workspace": ([ctypes.POINTER(GravityDesc), _sz_p], ctypes.c_int),
     "pm_spectral_force_multiply": ([_vp, _vp, ctypes.POINTER(GravityDesc), _i32, _i32, _vp, ctypes.c_size_t, _vp],
@@ -163,6 +166,11 @@ _SIGNATURES = {
     "pm_ic_linear_modes": ([_vp, _i32x3, _vp, _vp, _vp, _i32, _f32, _f32, _f32, _f32, _vp], ctypes.c_int),
     "pm_ic_spectral_op": ([_vp, _vp, _i32x3, _vp, _i32, _i32, _i32, _f32, _vp, _vp, _vp], ctypes.c_int),
     "pm_ic_product_acc": ([_vp, _vp, _vp, _i64, _f32, _i32, _vp], ctypes.c_int),
+    "pm_ic_symbol_inverse_workspace": ([_i32x3, _sz_p], ctypes.c_int),
+    "pm_ic_symbol_inverse": ([_vp, _vp, _i32x3, _vp, _i32, _vp, _vp, _vp, ctypes.c_size_t, _vp], ctypes.c_int),
+    "pm_ic_lpt2_source": ([_vp, _i64, _vp, _vp], ctypes.c_int),
+    "pm_ic_lpt_particles": ([_i32x3, _i32x3, ctypes.c_double, _vp, _vp, _f32, _f32, _f32, _f32, _vp, _vp, _vp, _vp],
+                            ctypes.c_int),
     "pm_ic_lpt_accumulate": ([_vp, _vp, _vp, _i64, _i32, _f32, _f32, _vp], ctypes.c_int),
 }
 

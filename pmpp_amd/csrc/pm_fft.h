@@ -305,6 +305,12 @@ __device__ __forceinline__ float spec_negk(float k, const SpecTables& tb) {
   return (fabsf(fabsf(k) - tb.nyq) <= tb.nyq_eps) ? 0.f : -k;
 }
 
+// A component of kColSym: the strain symbol -k_i k_j (a Nyquist wavenumber zeroed when i != j), or,
+// with j < 0, the gradient's -i k_i (a Nyquist wavenumber zeroed).
+struct ColSymbol {
+  int i, j;
+};
+
 // Column pass: FFT along a strided axis over tiles of T adjacent columns (unit stride).
 // element (row r, column c, batch b) lives at base[b*s_batch + r*s_row + c*s_col].
 struct ColPass {
@@ -329,6 +335,8 @@ struct ColPass {
   const float2* in1 = nullptr;
   const float2* in2 = nullptr;
   float2* out2 = nullptr;  // kColInv3: the third output
+  ColSymbol sym[3] = {};   // kColSym: the three components' symbols
+  float sym_nyq[3] = {}, sym_tol[3] = {};  // a wavenumber k is the Nyquist of axis a when ||k| - nyq[a]| <= tol[a]
 };
 
 // kColAdj: the x pass of the force step's spectral adjoint: forward transforms of the three
@@ -336,7 +344,9 @@ struct ColPass {
 // kColPot: x forward, mask * (-1/k^2), x inverse (the potential, one output)
 // kColInv3: the y inverses of the three force components in one launch: out0 <- in, out1 <- D in,
 // out2 <- in1
-enum ColMode { kColFwd = 0, kColInv = 1, kColInv3 = 2, kColGreen = 3, kColAdj = 4, kColPot = 5 };
+// kColSym: x inverses of three symbols times one spectrum (batches ky, columns kz): out0, out1, out2 <-
+// IFFT_x(sym[c](k) in), with the wavenumbers of tb.k
+enum ColMode { kColFwd = 0, kColInv = 1, kColInv3 = 2, kColGreen = 3, kColAdj = 4, kColPot = 5, kColSym = 6 };
 
 // Upper x/y planes of the brick columns of a tiled scatter (pm_gravity.hip), which the R2C pass adds
 // to the lower planes of the neighbouring columns while it reads the mesh: extents of the

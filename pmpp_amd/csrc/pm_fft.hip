@@ -235,6 +235,25 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
         for (int s = 0; s < E; ++s)
           v[s] = cok ? io.out0[obp + (int64_t)(nrow<N>(p, s) - p) * o_row] : make_float2(0.f, 0.f);
       }
+    } else if constexpr (MODE == kColSym) {
+      const ColSymbol sy = half == 0 ? io.sym[0] : (half == 1 ? io.sym[1] : io.sym[2]);  // uniform
+      const float ky = tb.k[1][b], kz = tb.k[2][cgl];
+      // a wavenumber of axis a with the Nyquist zeroed
+      auto live = [&](int a, float k) { return fabsf(fabsf(k) - io.sym_nyq[a]) <= io.sym_tol[a] ? 0.f : k; };
+      const bool cross = sy.j != sy.i;  // strains of two axes and gradients zero the Nyquist
+#pragma unroll
+      for (int s = 0; s < E; ++s) {
+        const float kx = tb.k[0][xrow<N>(p, s)];
+        float ki = sy.i == 0 ? kx : (sy.i == 1 ? ky : kz);
+        if (cross) ki = live(sy.i, ki);
+        if (sy.j < 0) {
+          v[s] = make_float2(ki * v[s].y, -ki * v[s].x);  // -i k v
+        } else {
+          float kj = sy.j == 0 ? kx : (sy.j == 1 ? ky : kz);
+          if (cross) kj = live(sy.j, kj);
+          v[s] = c_scale(v[s], -ki * kj);
+        }
+      }
     } else if constexpr (MODE == kColInv3) {
       if (half == 1) {
 #pragma unroll
@@ -523,6 +542,7 @@ int launch_cols_n(int mode, const ColPass& cp, int batches, const SpecTables& tb
     case kColInv: return launch_cols_cfg<N, T1, kColInv, 1>(cp, batches, tb, dax, s, "fft_cols_inv");
     case kColInv3: return launch_cols_cfg<N, T2, kColInv3, 3>(cp, batches, tb, dax, s, "fft_cols_inv3");
     case kColGreen: return launch_cols_cfg<N, T2, kColGreen, 1>(cp, batches, tb, dax, s, "fft_cols_green");
+    case kColSym: return launch_cols_cfg<N, T2, kColSym, 3>(cp, batches, tb, dax, s, "fft_cols_symbol");
     case kColAdj: return launch_cols_cfg<N, T1, kColAdj, 1>(cp, batches, tb, dax, s, "fft_cols_adjoint");
     case kColPot: return launch_cols_cfg<N, T2, kColPot, 1>(cp, batches, tb, dax, s, "fft_cols_potential");
     default: return fail(PM_ERROR_INVALID_ARGUMENT, "bad column mode");
@@ -663,24 +683,73 @@ int rfft3d_pitched(const float* in, float2* spec, const int32_t* shape, int64_t 
   return launch_cols(nx, kColFwd, cx, ny, tb, 0, s);
 }
 
-// Inverse 3D c2r (1/N normalised); the spectrum is used as scratch.
-int irfft3d_pitched(float2* spec, float* out, const int32_t* shape, int64_t pitch, const SpecTables& tb,
-                    hipStream_t s) {
+// Row pitch of a scratch half spectrum: rows start on cache lines.
+int64_t scratch_pitch(const int32_t* shape) { return (int64_t)align_up((size_t)shape[2] / 2 + 1, 16); }
+
+// The y and z passes of ncomp inverse transforms whose x inverses lie one after the other in
+// `spec` (pitched rows), into ncomp meshes one after the other (1/N normalised).
+static int inverse_yz(float2* spec, float* out, const int32_t* shape, int64_t pitch, int ncomp, const SpecTables& tb,
+                      hipStream_t s) {
   const int nx = shape[0], ny = shape[1], nz = shape[2], m = nz / 2;
-  ColPass cx{spec, spec, nullptr, (int64_t)ny * pitch, 1, pitch, m + 1, 0, 0, 0, 0, 0};
-  int st = launch_cols(nx, kColInv, cx, ny, tb, 0, s);
-  if (st) return st;
   ColPass cy{spec, spec, nullptr, pitch, 1, (int64_t)ny * pitch, m + 1, 0, 0, 0, 0, 0};
-  st = launch_cols(ny, kColInv, cy, nx, tb, 0, s);
-  if (st) return st;
+  PM_TRY(launch_cols(ny, kColInv, cy, ncomp * nx, tb, 0, s));
   ZPass zp{};
   zp.rout[0] = out;
   zp.cmain[0] = spec;
   zp.pitch_r = nz;
   zp.pitch_c = pitch;
-  zp.nlines = (int64_t)nx * ny;
+  zp.nlines = (int64_t)ncomp * nx * ny;
   zp.out_scale = (float)(2.0 / ((double)nx * ny * nz));
   return launch_z(nz, true, zp, tb, s);
+}
+
+size_t symbol_inverse_bytes(const int32_t* shape) {
+  return sizeof(float2) * 3 * (size_t)shape[0] * shape[1] * scratch_pitch(shape);
+}
+
+// out[c] = irfftn(symbol_c(k) spec), c = 0..2, for a standard-layout spectrum that is only read: the
+// symbols are applied by the x pass, which writes the three components to scratch; the y and z
+// passes run over the three in one launch each (nine launches and three passes over a
+// spectrum each before: the multiply, its scratch copy, and the transform's three).
+int symbol_inverse3(const float2* spec, float* out, const int32_t* shape, const float* const ktab[3],
+                    const ColSymbol sym[3], const float nyquist[3], const float tol[3], float2* scratch,
+                    hipStream_t s) {
+  const int nx = shape[0], ny = shape[1], m = shape[2] / 2;
+  const int64_t pitch = scratch_pitch(shape), comp = (int64_t)nx * ny * pitch;
+  SpecTables tb{};
+  for (int a = 0; a < 3; ++a) tb.k[a] = ktab[a];
+  ColPass cx{const_cast<float2*>(spec), scratch, scratch + comp, (int64_t)ny * (m + 1), 1, m + 1, m + 1, 0, 0, 0, 0, 0};
+  cx.out2 = scratch + 2 * comp;
+  cx.o_row = (int64_t)ny * pitch;
+  cx.o_batch = pitch;
+  for (int c = 0; c < 3; ++c) {
+    cx.sym[c] = sym[c];
+    cx.sym_nyq[c] = nyquist[c];
+    cx.sym_tol[c] = tol[c];
+  }
+  PM_TRY(launch_cols(nx, kColSym, cx, ny, tb, 0, s));
+  return inverse_yz(scratch, out, shape, pitch, 3, tb, s);
+}
+
+// Inverse 3D c2r of a standard-layout spectrum that is only read: the x pass writes the scratch.
+int irfft3d_keep(const float2* spec, float* out, const int32_t* shape, float2* scratch, hipStream_t s) {
+  const int nx = shape[0], ny = shape[1], m = shape[2] / 2;
+  const int64_t pitch = scratch_pitch(shape);
+  SpecTables tb{};
+  ColPass cx{const_cast<float2*>(spec), scratch, nullptr, (int64_t)ny * (m + 1), 1, m + 1, m + 1, 0, 0, 0, 0, 0};
+  cx.o_row = (int64_t)ny * pitch;
+  cx.o_batch = pitch;
+  PM_TRY(launch_cols(nx, kColInv, cx, ny, tb, 0, s));
+  return inverse_yz(scratch, out, shape, pitch, 1, tb, s);
+}
+
+// Inverse 3D c2r (1/N normalised); the spectrum is used as scratch.
+int irfft3d_pitched(float2* spec, float* out, const int32_t* shape, int64_t pitch, const SpecTables& tb,
+                    hipStream_t s) {
+  const int nx = shape[0], ny = shape[1], m = shape[2] / 2;
+  ColPass cx{spec, spec, nullptr, (int64_t)ny * pitch, 1, pitch, m + 1, 0, 0, 0, 0, 0};
+  PM_TRY(launch_cols(nx, kColInv, cx, ny, tb, 0, s));
+  return inverse_yz(spec, out, shape, pitch, 1, tb, s);
 }
 
 }  // namespace fft
@@ -730,6 +799,26 @@ int pm_irfft3d(float* in_complex, float* out, const int32_t shape[3], void* work
   fft::SpecTables tb{};
   return fft::irfft3d_pitched(reinterpret_cast<float2*>(in_complex), out, shape, shape[2] / 2 + 1, tb,
                               as_stream(stream));
+}
+
+int pm_irfft3d_keep_workspace(const int32_t shape[3], size_t* bytes) {
+  PM_RETURN_IF(shape == nullptr || bytes == nullptr, PM_ERROR_INVALID_ARGUMENT, "NULL argument");
+  PM_RETURN_IF(!fft::supported_shape(shape), PM_ERROR_UNSUPPORTED,
+               "FFT axes must be powers of two in [2, 2048]");
+  *bytes = sizeof(float2) * (size_t)shape[0] * shape[1] * fft::scratch_pitch(shape);
+  return PM_SUCCESS;
+}
+
+int pm_irfft3d_keep(const float* in_complex, float* out, const int32_t shape[3], void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  size_t need = 0;
+  PM_TRY(pm_irfft3d_keep_workspace(shape, &need));
+  PM_RETURN_IF(in_complex == nullptr || out == nullptr, PM_ERROR_INVALID_ARGUMENT, "NULL argument");
+  PM_TRY(require_device_tables());
+  PM_RETURN_IF(workspace == nullptr || workspace_bytes < need, PM_ERROR_WORKSPACE,
+               "inverse FFT workspace too small: need " + std::to_string(need) + " bytes");
+  return fft::irfft3d_keep(reinterpret_cast<const float2*>(in_complex), out, shape, static_cast<float2*>(workspace),
+                           as_stream(stream));
 }
 
 }  // extern "C"

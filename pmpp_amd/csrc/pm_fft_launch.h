@@ -22,6 +22,10 @@ int launch_spectral_multiply(const float2* in, float2* out, const int32_t* shape
 
 int rfft3d_pitched(const float* in, float2* spec, const int32_t* shape, int64_t pitch, float shift,
                    float scale, const SpecTables& tb, hipStream_t s);
+size_t symbol_inverse_bytes(const int32_t* shape);
+int symbol_inverse3(const float2* spec, float* out, const int32_t* shape, const float* const ktab[3],
+                    const ColSymbol sym[3], const float nyquist[3], const float tol[3], float2* scratch,
+                    hipStream_t s);
 int irfft3d_pitched(float2* spec, float* out, const int32_t* shape, int64_t pitch, const SpecTables& tb,
                     hipStream_t s);
 

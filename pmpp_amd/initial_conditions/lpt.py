@@ -9,10 +9,10 @@ displacements and canonical velocities to ``conf.lpt_order`` (0, 1 or 2):
   disp += D_m(a) grad_m,   vel += a^2 H(a) dD_m/dln a grad_m,   grad_m = irfftn(-i k phi_m)
 
 with the strain and gradient symbols zeroing the Nyquist wavenumber where the reference does
-(``_strain`` :17-43 for i != j, ``neg_grad`` gravity.py:355-391).  Every spectral product is
-one ``pm_ic_spectral_op`` launch and every transform the library's own rFFT; the growth
-factors are the host float64 table's, cast to float32 as the reference casts them.
-Particles come from ``Particles.gen_grid``, so particle n samples grid point n (the
+(``_strain`` :17-43 for i != j, ``neg_grad`` gravity.py:355-391).  The strains and gradients are
+``pm_ic_symbol_inverse`` calls (three symbols of one potential each) and every transform the
+library's own rFFT; the growth factors are the host float64 table's, cast to float32 as the
+reference casts them.  Particles come from ``Particles.gen_grid``, so particle n samples grid point n (the
 single-device branch of ``_sample_lpt_field`` :55-81).
 """
 
@@ -29,7 +29,7 @@ from ..cosmology.background import E2
 from ..nbody.integrator import growth_table
 from ..nbody.particles import Particles
 from ..numerics import irfftn, rfftn
-from .modes import KGrid, LAPLACE, NEG_GRAD, SCALE, STRAIN
+from .modes import GRADIENT, KGrid, LAPLACE, NEG_GRAD, POTENTIAL, SCALE, STRAIN, STRAINS_CROSS, STRAINS_DIAG
 
 
 def _acc_product(acc, a, b, coef, init):
@@ -39,25 +39,14 @@ def _acc_product(acc, a, b, coef, init):
 
 def second_order_source(kg, pot):
     """L = sum_{i<j} phi_ii phi_jj - phi_ij^2 of a potential spectrum (lpt.py:239-302, one
-    potential, diagonal strains cached), accumulated in the reference's order."""
+    potential): the six strains from two batched inverse transforms, then one pass over them,
+    accumulated in the reference's order."""
     shape = kg.shape
-    scratch = torch.empty_like(pot)
-    diag = []
-    for i in range(3):
-        kg.op(pot, STRAIN, i, i, out=scratch)
-        diag.append(irfftn(scratch, s=shape))
+    strains = torch.empty((6,) + shape, dtype=torch.float32, device=pot.device)
+    kg.inverse3(pot, STRAINS_DIAG, out=strains[:3])
+    kg.inverse3(pot, STRAINS_CROSS, out=strains[3:])
     L = torch.empty(shape, dtype=torch.float32, device=pot.device)
-    first = True
-    for i in range(3):
-        for j in range(2, i, -1):
-            _acc_product(L, diag[i], diag[j], 1.0, first)
-            first = False
-    del diag
-    for i in range(2):
-        for j in range(i + 1, 3):
-            kg.op(pot, STRAIN, i, j, out=scratch)
-            t = irfftn(scratch, s=shape)
-            _acc_product(L, t, t, -1.0, False)
+    _lib.call("pm_ic_lpt2_source", ptr(strains), L.numel(), ptr(L), stream_handle(pot.device))
     return L
 
 
@@ -79,31 +68,21 @@ def lpt(modes, cosmo, conf):
     cell_vol = conf.ptcl_spacing ** 3
     pots = []
     if conf.lpt_order > 0:
-        src = kg.op(modes.to(torch.complex64).contiguous(), SCALE, scale=1.0 / cell_vol)
-        pots.append(kg.op(src, LAPLACE))
-        del src
+        pots.append(kg.op(modes.to(torch.complex64).contiguous(), POTENTIAL, scale=1.0 / cell_vol))
     if conf.lpt_order > 1:
         L = second_order_source(kg, pots[0])
         src2 = rfftn(L)
         del L
-        pots.append(kg.op(src2, LAPLACE))
-        del src2
-    ptcl = Particles.gen_grid(conf, vel=True, device=dev)
-    disp = ptcl.disp.contiguous().clone()
-    vel = ptcl.vel.contiguous().clone()
+        pots.append(kg.op(src2, LAPLACE, out=src2))
     a = float(conf.a_start)
     tab = growth_table(cosmo, conf)
-    scratch = torch.empty_like(pots[0]) if pots else None
-    n = len(ptcl)
-    for order, pot in enumerate(pots, start=1):
-        D = np.float32(tab.growth(a, order))
-        a2HDp = np.float32(a ** 2 * math.sqrt(float(E2(a, tab.cosmo))) * float(tab.growth(a, order, 1)))
-        for i in range(3):
-            kg.op(pot, NEG_GRAD, i, out=scratch)
-            g = irfftn(scratch, s=shape)
-            _lib.call("pm_ic_lpt_accumulate", ptr(disp), ptr(vel), ptr(g), n, i, float(D), float(a2HDp),
-                      stream_handle(dev))
-    return ptcl.replace(disp=disp, vel=vel, acc=None)
+    grads, D, V = [], [0.0, 0.0], [0.0, 0.0]
+    for m, pot in enumerate(pots):
+        D[m] = float(np.float32(tab.growth(a, m + 1)))
+        V[m] = float(np.float32(a ** 2 * math.sqrt(float(E2(a, tab.cosmo))) * float(tab.growth(a, m + 1, 1))))
+        grads.append(kg.inverse3(pot, GRADIENT))
+    grads += [None] * (2 - len(grads))
+    return Particles.gen_grid(conf, vel=True, device=dev, lpt=(*grads, D[0], V[0], D[1], V[1]))
 
 
 def particles_2lpt(conf, cosmo, seed=0, jitter_seed=None, device="cuda", a=None):

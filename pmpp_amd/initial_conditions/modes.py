@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from .. import _lib
-from .._torch import ensure_init, ptr, require_device, stream_handle
+from .._torch import ensure_init, ptr, require_device, stream_handle, workspace
 from ..cosmology import boltzmann
 from ..nbody.integrator import growth_table
 from ..numerics import irfftn, rfftn
@@ -39,7 +39,8 @@ class KGrid:
         self.tol = (ctypes.c_float * 3)(*([float(nyq * np.finfo(np.float32).eps)] * 3))
 
     def op(self, spec, op, i=0, j=0, scale=1.0, out=None):
-        """symbol(k) * spec: 0 scale, 1 Laplace inverse, 2 strain -k_i k_j, 3 -i k_i."""
+        """symbol(k) * spec: 0 scale, 1 Laplace inverse, 2 strain -k_i k_j, 3 -i k_i, 4 scale then
+        Laplace inverse."""
         if out is None:
             out = torch.empty_like(spec)
         _lib.call("pm_ic_spectral_op", ptr(spec), ptr(out), _lib.int3(self.shape), self.ptrs, int(op), int(i), int(j),
@@ -47,7 +48,23 @@ class KGrid:
         return out
 
 
-SCALE, LAPLACE, STRAIN, NEG_GRAD = 0, 1, 2, 3
+    def inverse3(self, spec, kind, out=None):
+        """Three real meshes (3, *shape): the inverse transforms of symbol(k) * spec for the strains
+        -k_i k_i (kind 0), -k_0 k_1, -k_0 k_2, -k_1 k_2 (1) or the gradient -i k_i (2), in one call
+        (``pm_ic_symbol_inverse``)."""
+        dev = spec.device
+        if out is None:
+            out = torch.empty((3,) + self.shape, dtype=torch.float32, device=dev)
+        shape = _lib.int3(self.shape)
+        nbytes = _lib.size_query("pm_ic_symbol_inverse_workspace", shape)
+        ws = workspace(nbytes, dev)
+        _lib.call("pm_ic_symbol_inverse", ptr(spec), ptr(out), shape, self.ptrs, int(kind), self.nyquist, self.tol,
+                  ptr(ws), nbytes, stream_handle(dev))
+        return out
+
+
+SCALE, LAPLACE, STRAIN, NEG_GRAD, POTENTIAL = 0, 1, 2, 3, 4
+STRAINS_DIAG, STRAINS_CROSS, GRADIENT = 0, 1, 2  # kinds of KGrid.inverse3
 
 
 def white_noise(seed, conf, real=False, device="cuda"):

@@ -44,8 +44,27 @@ class Particles:
         return None if self.unused_index is None else ~self.unused_index
 
     @classmethod
-    def gen_grid(cls, conf, vel=False, acc=False, device="cuda"):
-        """Particles on the uniform Lagrangian grid with exact integer anchors (:615-727)."""
+    def gen_grid(cls, conf, vel=False, acc=False, device="cuda", lpt=None):
+        """Particles on the uniform Lagrangian grid with exact integer anchors (:615-727).
+
+        On a GPU they are made there (``pm_ic_lpt_particles``), the same values bit for bit.
+        ``lpt`` (GPU only) adds LPT terms: (grad1, grad2, D1, V1, D2, V2), the displacements D1 grad1 +
+        D2 grad2 and the velocities V1 grad1 + V2 grad2 of (3, *grid) gradient meshes (None: none)."""
+        dev = torch.device(device)
+        if dev.type == "cuda" and conf.dim == 3:
+            from .. import _lib
+            from .._torch import ptr, stream_handle
+
+            n = conf.ptcl_num
+            pm_t = torch.empty((n, 3), dtype=torch.int16, device=dev)
+            dp_t = torch.empty((n, 3), dtype=torch.float32, device=dev)
+            v = torch.empty_like(dp_t) if vel else None
+            g1, g2, *factors = lpt if lpt is not None else (None, None, 0.0, 0.0, 0.0, 0.0)
+            _lib.call("pm_ic_lpt_particles", _lib.int3(conf.ptcl_grid_shape), _lib.int3(conf.mesh_shape),
+                      float(conf.cell_size), ptr(g1), ptr(g2), *factors, ptr(pm_t), ptr(dp_t), ptr(v),
+                      stream_handle(dev))
+            unused = torch.zeros(n, dtype=torch.bool, device=dev)
+            return cls(conf, pm_t, dp_t, vel=v, acc=torch.zeros_like(dp_t) if acc else None, unused_index=unused)
         pmid, disp = [], []
         for sp, sm in zip(conf.ptcl_grid_shape, conf.mesh_shape):
             p = np.rint(np.linspace(0, sm, num=sp, endpoint=False)).astype(np.int64)

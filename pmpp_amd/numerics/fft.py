@@ -31,10 +31,13 @@ def irfftn(xk: torch.Tensor, s=None) -> torch.Tensor:
         s = (xk.shape[0], xk.shape[1], 2 * (xk.shape[2] - 1))
     if tuple(xk.shape) != (s[0], s[1], s[2] // 2 + 1):
         raise ValueError(f"spectrum shape {tuple(xk.shape)} does not match real shape {tuple(s)}")
-    scratch = as_contig(xk, torch.complex64, "xk").clone()  # the inverse uses its input as scratch
+    xin = as_contig(xk, torch.complex64, "xk")
     ensure_init(xk.device)
+    shape = _lib.int3(s)
     out = torch.empty(tuple(s), dtype=torch.float32, device=xk.device)
-    _lib.call("pm_irfft3d", ptr(scratch), ptr(out), _lib.int3(s), None, 0, stream_handle(xk.device))
+    nbytes = _lib.size_query("pm_irfft3d_keep_workspace", shape)
+    ws = workspace(nbytes, xk.device)
+    _lib.call("pm_irfft3d_keep", ptr(xin), ptr(out), shape, ptr(ws), nbytes, stream_handle(xk.device))
     return out
 
 

@@ -213,3 +213,45 @@ def test_pk_loss_gradient_wrt_white_noise_matches_oracle_finite_differences(devi
     fds = np.array(fds)
     print("gradient vs FD:", np.c_[got, fds])
     np.testing.assert_allclose(got, fds, rtol=1e-3, atol=1e-3 * np.abs(fds).max())
+
+
+@pytest.mark.parametrize("grid,mesh,spacing", [((16, 16, 16), (16, 16, 16), 1.0), ((45, 45, 45), (64, 64, 64), 1.25),
+                                               ((3, 5, 7), (6, 10, 14), 1000 / 512), ((1, 1, 1), (2, 2, 2), 0.3),
+                                               ((180, 180, 180), (256, 256, 256), 0.977), ((64, 8, 32), (128, 16, 64), 2.0)])
+def test_particle_lattice_on_the_device_equals_the_host_one(device, grid, mesh, spacing):
+    """Whole groups of four particles, ragged ends (45^3, 105, 1) and anchors that are not multiples
+    of the ratio: the same float64 formulas, so the same bits."""
+    conf = Configuration(spacing, grid, mesh_shape=mesh)
+    a, b = Particles.gen_grid(conf, vel=True, acc=True, device=device), Particles.gen_grid(conf, vel=True, acc=True,
+                                                                                          device="cpu")
+    for name in ("pmid", "disp", "vel", "acc", "unused_index"):
+        x, y = getattr(a, name), getattr(b, name)
+        assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
+
+
+@pytest.mark.parametrize("grid", [(2, 2, 2), (8, 8, 8), (64, 4, 16), (4, 128, 32), (32, 16, 256), (512, 4, 4)])
+def test_symbol_inverses_match_multiply_then_transform(device, grid):
+    """The three strains, cross strains and gradient components of one call against the symbol
+    applied on its own and numpy's float64 inverse: 2e-6 log2 N of the rms as the transforms; the
+    input spectrum is only read."""
+    from pmpp_amd.initial_conditions.modes import GRADIENT, KGrid, NEG_GRAD, STRAIN, STRAINS_CROSS, STRAINS_DIAG
+    from pmpp_amd.numerics import irfftn
+
+    rng = np.random.default_rng(sum(grid))
+    spec = torch.as_tensor(np.fft.rfftn(rng.normal(size=grid)).astype(np.complex64), device=device)
+    keep = spec.clone()
+    kg = KGrid(grid, 1.7, device)
+    tol = 2e-6 * math.log2(max(2, math.prod(grid)))
+    for kind, parts in ((STRAINS_DIAG, [(STRAIN, 0, 0), (STRAIN, 1, 1), (STRAIN, 2, 2)]),
+                        (STRAINS_CROSS, [(STRAIN, 0, 1), (STRAIN, 0, 2), (STRAIN, 1, 2)]),
+                        (GRADIENT, [(NEG_GRAD, 0, 0), (NEG_GRAD, 1, 0), (NEG_GRAD, 2, 0)])):
+        got = kg.inverse3(spec, kind).cpu().numpy()
+        for c, (op, i, j) in enumerate(parts):
+            part = kg.op(spec, op, i, j)
+            ref = np.fft.irfftn(part.cpu().numpy().astype(np.complex128), s=grid, axes=(0, 1, 2))
+            rms = max(np.sqrt(np.mean(ref ** 2)), 1e-30)
+            assert np.abs(got[c] - ref).max() <= tol * rms * 8 + 1e-30, (kind, c)
+            one = irfftn(part, s=grid)
+            assert np.abs(one.cpu().numpy() - ref).max() <= tol * rms * 8 + 1e-30
+            assert torch.equal(part, kg.op(spec, op, i, j))  # the transform left it as it was
+    assert torch.equal(spec, keep)
