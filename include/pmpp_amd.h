@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PM_ABI_VERSION 11
+#define PM_ABI_VERSION 12
 
 enum pm_status {
   PM_SUCCESS = 0,
@@ -116,6 +116,22 @@ int pm_cic_scatter_bwd(const int16_t* pmid, const float* disp, const uint8_t* va
                        const float* val, float val_scalar, int64_t n, int32_t channels,
                        const pm_cic_geom* geom, const float* mesh_cot, float* disp_cot,
                        float* val_cot, void* stream);
+
+/* pm_cic_scatter_tiled     pm_cic_scatter into a mesh of its own: mesh = base + sum val W (base NULL: 0;
+ *                          not in place), by binning the particles and adding each brick up on chip.
+ * pm_cic_gather_bwd_tiled  pm_cic_gather_bwd with mesh_cot overwritten, the same way.
+ * Both take one-channel meshes without offset, corner drops or a cell size of their own, whose axes
+ * are whole bricks, and enough particles; pm_cic_tiled_workspace gives the workspace they need, or 0
+ * for a call that only the plain entry points take (PM_ERROR_UNSUPPORTED here).  Values too far below
+ * the largest for the fixed point, and all when a value or a position is not finite, go
+ * through the plain entry points' float atomics, decided on the device. */
+int pm_cic_tiled_workspace(int64_t n, int32_t channels, const pm_cic_geom* geom, size_t* bytes);
+int pm_cic_scatter_tiled(const int16_t* pmid, const float* disp, const uint8_t* valid, const float* val,
+                         float val_scalar, int64_t n, const pm_cic_geom* geom, const float* base, float* mesh,
+                         void* workspace, size_t workspace_bytes, void* stream);
+int pm_cic_gather_bwd_tiled(const int16_t* pmid, const float* disp, const uint8_t* valid, int64_t n,
+                            const pm_cic_geom* geom, const float* mesh, const float* val_cot, float* disp_cot,
+                            float* mesh_cot, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------- cell sort ----
  * Stable counting sort of particles by the raveled brick key of their containing

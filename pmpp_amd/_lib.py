@@ -14,7 +14,7 @@ import ctypes
 import os
 from pathlib import Path
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 PM_SUCCESS = 0
 PM_ERROR_INVALID_ARGUMENT = 1
@@ -27,6 +27,7 @@ EXPORTED_SYMBOLS = (
     "pm_last_error", "pm_abi_version", "pm_init",
     "pm_timing_enable", "pm_timing_mark", "pm_timing_read",
     "pm_cic_scatter", "pm_cic_gather", "pm_cic_gather_bwd", "pm_cic_scatter_bwd",
+    "pm_cic_tiled_workspace", "pm_cic_scatter_tiled", "pm_cic_gather_bwd_tiled",
     "pm_sort_cells_workspace", "pm_sort_cells", "pm_bucket_cells_workspace", "pm_bucket_cells",
     "pm_bucket_cells_noalloc",
     "pm_fft_workspace", "pm_rfft3d", "pm_irfft3d", "pm_irfft3d_keep_workspace", "pm_irfft3d_keep",
@@ -89,6 +90,11 @@ _SIGNATURES = {
     "pm_timing_read": ([ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_char_p), _i32,
                         ctypes.POINTER(ctypes.c_int32)], ctypes.c_int),
     "pm_cic_scatter": ([_vp, _vp, _vp, _vp, _f32, _i64, _i32, ctypes.POINTER(CicGeom), _vp, _vp], ctypes.c_int),
+    "pm_cic_tiled_workspace": ([_i64, _i32, ctypes.POINTER(CicGeom), _sz_p], ctypes.c_int),
+    "pm_cic_scatter_tiled": ([_vp, _vp, _vp, _vp, _f32, _i64, ctypes.POINTER(CicGeom), _vp, _vp, _vp,
+                              ctypes.c_size_t, _vp], ctypes.c_int),
+    "pm_cic_gather_bwd_tiled": ([_vp, _vp, _vp, _i64, ctypes.POINTER(CicGeom), _vp, _vp, _vp, _vp, _vp,
+                                 ctypes.c_size_t, _vp], ctypes.c_int),
     "pm_cic_gather": ([_vp, _vp, _vp, _i64, _i32, ctypes.POINTER(CicGeom), _vp, _vp, _vp], ctypes.c_int),
     "pm_cic_gather_bwd": ([_vp, _vp, _vp, _i64, _i32, ctypes.POINTER(CicGeom), _vp, _vp, _vp, _vp, _vp],
                           ctypes.c_int),

@@ -16,7 +16,7 @@ import math
 import torch
 
 from .. import _lib
-from .._torch import as_contig, ensure_init, ptr, require_device, stream_handle
+from .._torch import as_contig, ensure_init, ptr, require_device, stream_handle, workspace
 
 
 def _check(pmid, disp, mesh):
@@ -73,7 +73,6 @@ def hip_scatter(pmid, disp, val, mesh, *, offset, particle_cell_size, cell_size=
     n = pmid.shape[0]
     chan_shape = tuple(mesh.shape[3:])
     C = math.prod(chan_shape) if chan_shape else 1
-    out = as_contig(mesh, torch.float32, "mesh").clone()
     pm = as_contig(pmid, torch.int16, "pmid")
     dp = as_contig(disp, torch.float32, "disp")
     if _is_scalar(val):
@@ -85,9 +84,42 @@ def hip_scatter(pmid, disp, val, mesh, *, offset, particle_cell_size, cell_size=
         vs = 0.0
     valid = _valid(valid_mask, n, mesh.device)
     g = _geom(mesh.shape[:3], global_shape, offset, particle_cell_size, cell_size)
+    base = as_contig(mesh, torch.float32, "mesh")
+    nbytes = 0 if base.data_ptr() % 16 else _lib.size_query("pm_cic_tiled_workspace", n, C, g)
+    if nbytes:
+        return _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, nbytes)
+    out = base.clone()
     _lib.call("pm_cic_scatter", ptr(pm), ptr(dp), ptr(valid), ptr(vt), vs, n, C, g, ptr(out),
               stream_handle(mesh.device))
     return out
+
+
+def _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, nbytes):
+    """base (None: 0) + sum val W through ``pm_cic_scatter_tiled``, on checked arguments."""
+    dev = dp.device
+    out = torch.empty(tuple(g.local_shape) if base is None else base.shape, dtype=torch.float32, device=dev)
+    ws = workspace(nbytes, dev)
+    _lib.call("pm_cic_scatter_tiled", ptr(pm), ptr(dp), ptr(valid), ptr(vt), vs, n, g, ptr(base), ptr(out), ptr(ws),
+              nbytes, stream_handle(dev))
+    return out
+
+
+def hip_scatter_new(pmid, disp, val, shape, *, offset, particle_cell_size, cell_size=None, global_shape,
+                    valid_mask=None):
+    """``hip_scatter`` onto a mesh of zeros of ``shape`` (spatial and channel axes)."""
+    n = pmid.shape[0]
+    if n and disp.is_cuda and len(shape) == 3 and tuple(pmid.shape) == (n, 3) == tuple(disp.shape):
+        ensure_init(disp.device)
+        g = _geom(shape, global_shape, offset, particle_cell_size, cell_size)
+        nbytes = _lib.size_query("pm_cic_tiled_workspace", n, 1, g)
+        if nbytes and (_is_scalar(val) or tuple(val.shape) == (n,)):
+            vt = None if _is_scalar(val) else as_contig(val, torch.float32, "val")
+            return _scatter_tiled(as_contig(pmid, torch.int16, "pmid"), as_contig(disp, torch.float32, "disp"),
+                                  _valid(valid_mask, n, disp.device), vt, float(val) if vt is None else 0.0, n, g, None,
+                                  nbytes)
+    mesh = torch.zeros(tuple(shape), dtype=torch.float32, device=disp.device)
+    return hip_scatter(pmid, disp, val, mesh, offset=offset, particle_cell_size=particle_cell_size,
+                       cell_size=cell_size, global_shape=global_shape, valid_mask=valid_mask)
 
 
 def hip_gather(pmid, disp, mesh, *, offset, particle_cell_size, cell_size=None, global_shape,
@@ -122,9 +154,16 @@ def hip_gather_bwd(pmid, disp, mesh, val_cot, *, offset, particle_cell_size, cel
     pm = as_contig(pmid, torch.int16, "pmid")
     dp = as_contig(disp, torch.float32, "disp")
     disp_cot = torch.empty((n, 3), dtype=torch.float32, device=mesh.device)
-    mesh_cot = torch.zeros_like(m)
     valid = _valid(valid_mask, n, mesh.device)
     g = _geom(mesh.shape[:3], global_shape, offset, particle_cell_size, cell_size)
+    nbytes = 0 if m.data_ptr() % 16 or vc.numel() != n else _lib.size_query("pm_cic_tiled_workspace", n, C, g)
+    if nbytes:
+        mesh_cot = torch.empty_like(m)
+        ws = workspace(nbytes, mesh.device)
+        _lib.call("pm_cic_gather_bwd_tiled", ptr(pm), ptr(dp), ptr(valid), n, g, ptr(m), ptr(vc), ptr(disp_cot),
+                  ptr(mesh_cot), ptr(ws), nbytes, stream_handle(mesh.device))
+        return disp_cot, mesh_cot
+    mesh_cot = torch.zeros_like(m)
     _lib.call("pm_cic_gather_bwd", ptr(pm), ptr(dp), ptr(valid), n, C, g, ptr(m), ptr(vc), ptr(disp_cot),
               ptr(mesh_cot), stream_handle(mesh.device))
     return disp_cot, mesh_cot

@@ -9,15 +9,21 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import hip_scatter, hip_scatter_bwd
+from .kernels import hip_scatter, hip_scatter_bwd, hip_scatter_new
 
 
 class _ScatterFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, disp, mesh, val_t, pmid, val_scalar, offset, particle_cell, cell_size, global_shape, valid):
         val = val_scalar if val_t is None else val_t
-        out = hip_scatter(pmid, disp, val, mesh, offset=offset, particle_cell_size=particle_cell,
-                          cell_size=cell_size, global_shape=global_shape, valid_mask=valid)
+        kw = dict(offset=offset, particle_cell_size=particle_cell, cell_size=cell_size, global_shape=global_shape,
+                  valid_mask=valid)
+        if mesh is None:  # a mesh of zeros of the global shape
+            chan = () if val_t is None else tuple(val_t.shape[1:])
+            out = hip_scatter_new(pmid, disp, val, tuple(global_shape) + chan, **kw)
+        else:
+            out = hip_scatter(pmid, disp, val, mesh, **kw)
+        ctx.has_mesh = mesh is not None
         ctx.save_for_backward(disp, pmid, val_t, valid)
         ctx.meta = (val_scalar, offset, particle_cell, cell_size, global_shape)
         return out
@@ -33,7 +39,7 @@ class _ScatterFn(torch.autograd.Function):
         val_grad = None
         if val_t is not None and ctx.needs_input_grad[2]:
             val_grad = val_cot.reshape(val_t.shape)
-        return disp_cot, mesh_cot, val_grad, None, None, None, None, None, None, None
+        return disp_cot, mesh_cot if ctx.has_mesh else None, val_grad, None, None, None, None, None, None, None
 
 
 def _scatter(pmid, disp, conf, mesh, val, offset, cell_size, valid_mask=None):
@@ -43,9 +49,7 @@ def _scatter(pmid, disp, conf, mesh, val, offset, cell_size, valid_mask=None):
     val_t = val if isinstance(val, torch.Tensor) and val.ndim > 0 else None
     val_scalar = 0.0 if val_t is not None else float(val)
     chan = () if val_t is None else tuple(val_t.shape[1:])
-    if mesh is None:
-        mesh = torch.zeros(tuple(conf.mesh_shape) + chan, dtype=torch.float32, device=disp.device)
-    if tuple(mesh.shape[3:]) != chan:
+    if mesh is not None and tuple(mesh.shape[3:]) != chan:
         raise ValueError(f"channel shape mismatch: {tuple(mesh.shape[3:])} != {chan}")
     valid = None if valid_mask is None else valid_mask.detach()
     if valid is not None and val_t is not None:

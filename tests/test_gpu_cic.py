@@ -112,3 +112,121 @@ def test_bad_arguments_raise(device):
     with pytest.raises(ValueError, match="channel shape mismatch"):
         hip_scatter(P, D, torch.ones((3, 2), device=device), torch.zeros((4, 4, 4, 3), device=device), offset=0,
                     particle_cell_size=1.0, global_shape=(4, 4, 4))
+
+
+# the tiled path: (mesh, n, spread in cells, invalid share, value kind); small bricks (8, 8, 16) up to
+# 2^21 cells, (16, 16, 32) above; axes that are and are not powers of two; the smallest n
+TILED = [
+    ((48, 32, 64), 1 << 18, 0.4, 0.0, "normal"),
+    ((8, 8, 16), (1 << 18) + 5, 3.0, 0.3, "normal"),
+    ((24, 16, 48), (1 << 18) + 77, 9.0, 0.2, "scalar"),
+    ((144, 128, 128), (1 << 18) + 1, 1.5, 0.1, "normal"),
+    ((64, 32, 32), 1 << 18, 1.5, 0.0, "wide"),  # values 10^12 apart: the smaller ones take the atomics
+    ((64, 32, 32), 1 << 18, 1.5, 0.1, "zero"),
+]
+
+
+@pytest.mark.parametrize("mesh_shape,n,spread,invalid,kind", TILED)
+def test_tiled_scatter_and_gather_adjoint_match_oracle(device, mesh_shape, n, spread, invalid, kind):
+    rng = np.random.default_rng(n + mesh_shape[0])
+    cell = 0.75
+    pmid = np.stack([rng.integers(-3, m + 3, n) for m in mesh_shape], 1).astype(np.int16)
+    disp = (rng.uniform(-spread, spread, (n, 3)) * cell).astype(np.float32)
+    val = (rng.choice([-1.0, 1.0], n) * rng.uniform(0.01, 2.0, n)).astype(np.float32)
+    if kind == "wide":
+        val[::1000] *= 1e12
+    if kind == "zero":
+        val[:] = 0
+        val[::3] = 0.5
+    valid = (rng.random(n) >= invalid) if invalid else None
+    if valid is not None:
+        val[~valid] = np.nan  # never read
+    mesh = rng.normal(size=mesh_shape).astype(np.float32)
+    v = 1.7 if kind == "scalar" else val
+    okw = dict(cell_size=cell, mesh_shape=mesh_shape, valid=valid)
+    kw = dict(offset=0.0, particle_cell_size=cell, global_shape=mesh_shape,
+              valid_mask=None if valid is None else _t(valid, device, torch.bool))
+    P, D, M = _t(pmid, device, torch.int16), _t(disp, device), _t(mesh, device)
+    V = v if kind == "scalar" else _t(v, device)
+    from pmpp_amd import _lib
+    from pmpp_amd.cic.kernels import _geom, hip_scatter_new
+
+    g = _geom(mesh_shape, mesh_shape, 0.0, cell, None)
+    assert _lib.size_query("pm_cic_tiled_workspace", n, 1, g) > 0
+
+    # a deposit's error: 3 axes x (fraction: 2^-24 (1 + |t|), weight and products: 2^-23) of |v|, atomics
+    # another 2^-24 of the partial sum each; bounded through the sum of |v| over the touching particles
+    ok = np.ones(n, bool) if valid is None else valid
+    av = np.where(ok, np.abs(np.nan_to_num(v) if kind != "scalar" else np.full(n, v)), 0.0)
+    t = disp.astype(np.float64) / cell
+    base = pmid.astype(np.int64) + np.floor(disp / np.float32(cell)).astype(np.int64)
+    touch = np.zeros(mesh_shape)
+    cnt = np.zeros(mesh_shape)
+    for c in range(8):
+        ix = tuple((base[:, a] + ((c >> a) & 1)) % mesh_shape[a] for a in range(3))
+        np.add.at(touch, ix, av)
+        np.add.at(cnt, ix, av > 0)
+    per = 3 * (2.0 ** -24 * (1 + spread) + 2.0 ** -23)
+    bound = touch * (per + (cnt * 2.0 ** -24 if kind == "wide" else 0)) + 1e-30
+
+    vo = np.nan_to_num(v) if kind != "scalar" else v
+    ref = cic.scatter(pmid, disp, vo, np.zeros(mesh_shape), **okw)
+    s0 = _np(hip_scatter_new(P, D, V, mesh_shape, **kw))
+    assert np.all(np.abs(s0 - ref) <= bound + 2.0 ** -24 * np.abs(ref))
+    s1 = _np(hip_scatter(P, D, V, M, **kw))
+    assert np.all(np.abs(s1 - (ref + mesh)) <= bound + 2.0 ** -23 * (np.abs(ref) + np.abs(mesh)))
+    if kind == "scalar":
+        return
+    dcot, mcot = hip_gather_bwd(P, D, M, V, **kw)
+    dref, mref = cic.gather_adj(pmid, disp, mesh, vo, **okw)
+    assert np.all(np.abs(_np(mcot) - mref) <= bound + 2.0 ** -24 * np.abs(mref))
+    # eight mesh values of at most max|mesh| with weights of error per, over the cell size
+    assert np.all(np.abs(_np(dcot) - dref) <= av[:, None] * np.abs(mesh).max() * 8 * per / cell + 1e-30)
+
+
+def test_tiled_path_refuses_and_falls_back(device):
+    from pmpp_amd import _lib
+    from pmpp_amd.cic.kernels import _geom
+
+    n = 1 << 18
+
+    def need(n=n, c=1, ls=(64, 32, 32), gs=None, off=0.0, cell=None):
+        return _lib.size_query("pm_cic_tiled_workspace", n, c, _geom(ls, gs or ls, off, 0.5, cell))
+
+    assert need() > 0
+    for kw in (dict(n=n - 1), dict(ls=(512, 512, 160)), dict(c=2), dict(ls=(64, 32, 24)), dict(ls=(60, 32, 32)), dict(gs=(128, 32, 32)),
+               dict(off=[0.1, 0, 0]), dict(cell=0.5), dict(ls=(256, 256, 48))):
+        assert need(**kw) == 0, kw
+
+    # a value or a position that is not finite: the atomics' results, on the cells it touches only
+    rng = np.random.default_rng(3)
+    pmid = rng.integers(0, 32, (n, 3)).astype(np.int16)
+    disp = rng.uniform(-0.4, 0.4, (n, 3)).astype(np.float32)
+    val = rng.uniform(0.5, 1.0, n).astype(np.float32)
+    kw = dict(offset=0.0, particle_cell_size=1.0, global_shape=(64, 32, 32))
+    P, M = _t(pmid, device, torch.int16), torch.ones((64, 32, 32), device=device)
+    for what in ("nan value", "inf value", "nan position"):
+        d, v = disp.copy(), val.copy()
+        if what == "nan position":
+            d[11, 1] = np.nan
+        else:
+            v[11] = np.nan if what == "nan value" else np.inf
+        D, V = _t(d, device), _t(v, device)
+        plain = M.clone()
+        g = _geom((64, 32, 32), (64, 32, 32), 0.0, 1.0, None)
+        from pmpp_amd._torch import ptr, stream_handle
+        _lib.call("pm_cic_scatter", ptr(P), ptr(D), None, ptr(V), 0.0, n, 1, g, ptr(plain), stream_handle(device))
+        s = hip_scatter(P, D, V, M, **kw)
+        # sums of at most ~100 float32 additions of values up to 1, in another order
+        assert torch.equal(torch.isnan(s), torch.isnan(plain)), what
+        assert torch.allclose(s, plain, rtol=100 * 2.0 ** -24, atol=100 * 2.0 ** -24, equal_nan=True), what
+        dcot, mcot = hip_gather_bwd(P, D, M, V, **kw)
+        bad = torch.isnan(dcot).any(1).nonzero().flatten().tolist()
+        assert bad in ([], [11]) and not torch.isfinite(mcot).all(), what
+    for vs in (0.0, float("inf"), 1e30):
+        D = _t(disp, device)
+        s = hip_scatter(P, D, vs, M, **kw)
+        if vs == 0.0:
+            assert torch.equal(s, M)
+        else:
+            assert not torch.isnan(s).any() and float(s.max()) > 1e29
