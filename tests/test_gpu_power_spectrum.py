@@ -130,3 +130,40 @@ def test_cross_correlation_vjp_matches_central_differences(device):
 
     fd = (f(a + eps * v) - f(a - eps * v)) / (2 * eps)
     assert float((g * v).sum()) == pytest.approx(fd, rel=2e-2)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 2, 2), (3, 5, 7), (1, 64, 4), (12, 9, 10), (65, 64, 66),
+                                   (16, 2050, 8)])
+@pytest.mark.parametrize("cross", [False, True])
+def test_shell_sums_of_any_shape(device, shape, cross):
+    # odd and even axes, axes of one mode, walks cut into chunks; straight from random spectra
+    from pmpp_amd import _lib
+    from pmpp_amd._torch import ptr, stream_handle
+
+    nx, ny, nz = shape
+    nzh = nz // 2 + 1
+    rng = np.random.default_rng(nx + ny + nz)
+    a, b = (rng.normal(size=(nx, ny, nzh, 2)).astype(np.float32) for _ in range(2))
+    m = [np.fft.fftfreq(n) * n for n in (nx, ny)] + [np.fft.rfftfreq(nz) * nz]
+    X, Y, Z = np.meshgrid(*[np.rint(v) for v in m], indexing="ij")
+    shell = np.floor(np.sqrt(X ** 2 + Y ** 2 + Z ** 2) + 1e-9).astype(np.int64)
+    ns = max(int(shell.max()) - 1, 1)  # the last shells are clamped into one
+    shell = np.minimum(shell, ns - 1)
+    mult = np.full(shell.shape, 2.0)
+    mult[..., 0] = 1
+    if nz % 2 == 0:
+        mult[..., -1] = 1
+    w = (np.sinc(X / nx) * np.sinc(Y / ny) * np.sinc(Z / nz)) ** -4.0 * mult
+    A, B = (v[..., 0].astype(np.float64) + 1j * v[..., 1] for v in (a, b))
+    ref = [np.bincount(shell.ravel(), (p * w).ravel(), ns) for p in
+           ([np.abs(A) ** 2, np.abs(B) ** 2, (A * B.conj()).real] if cross else [np.abs(A) ** 2])]
+    size = [np.bincount(shell.ravel(), (p * w).ravel(), ns) for p in
+            ([np.abs(A) ** 2, np.abs(B) ** 2, np.abs(A * B)] if cross else [np.abs(A) ** 2])]
+    ta, tb = torch.from_numpy(a).to(device), torch.from_numpy(b).to(device)
+    sums = torch.empty(3 * ns if cross else ns, dtype=torch.float64, device=device)
+    _lib.call("pm_power_spectrum", ptr(ta), ptr(tb) if cross else None, _lib.int3(shape), 2, ns, 0, ptr(sums),
+              stream_handle(device))
+    # float32 per mode: three sines of a few ulp each to the fourth power, and the product
+    got = sums.cpu().numpy().reshape(-1, ns)
+    for g, r, sz in zip(got, ref, size):
+        assert np.all(np.abs(g - r) <= 60 * 2.0 ** -24 * sz)
