@@ -83,24 +83,31 @@ def _finalize(psum, shape, cell_size):
     return k[:n], pk, nmodes[:n]
 
 
-def _to_torch(x, dev):
-    return torch.as_tensor(np.asarray(x), device=dev)
+def _to_device(dev, *arrays):
+    """Float arrays as float32 and integer ones as int32 tensors on ``dev``, in one host copy."""
+    host = np.empty((len(arrays), len(arrays[0])), np.int32)
+    for row, x in zip(host, arrays):
+        if np.issubdtype(x.dtype, np.floating):
+            row.view(np.float32)[:] = x
+        else:
+            row[:] = x
+    t = torch.from_numpy(host).to(dev)
+    return tuple((r.view(torch.float32) if np.issubdtype(x.dtype, np.floating) else r).clone()
+                 for r, x in zip(t, arrays))
 
 
 def delta_to_pk(delta, conf, mas="CIC"):
     """(k, P(k), nmodes) of an overdensity mesh (power_spectrum.py:287-310)."""
     shape, ns, s = _shell_sums(delta, None, mas, density=False)
     k, pk, nm = _finalize(s, shape, conf.cell_size)
-    dev = delta.device
-    return _to_torch(k, dev).float(), _to_torch(pk, dev).float(), _to_torch(nm, dev).int()
+    return _to_device(delta.device, k, pk, nm)
 
 
 def density_to_pk(density, conf, mas="CIC"):
     """(k, P(k), nmodes) of a density mesh; delta = rho / mean - 1 (power_spectrum.py:348-374)."""
     shape, ns, s = _shell_sums(density, None, mas, density=True)
     k, pk, nm = _finalize(s, shape, conf.cell_size)
-    dev = density.device
-    return _to_torch(k, dev).float(), _to_torch(pk, dev).float(), _to_torch(nm, dev).int()
+    return _to_device(density.device, k, pk, nm)
 
 
 def _cross(a, b, conf, mas, eps, density):
@@ -109,9 +116,7 @@ def _cross(a, b, conf, mas, eps, density):
     _, pb, _ = _finalize(s[ns:2 * ns], shape, conf.cell_size)
     _, pab, _ = _finalize(s[2 * ns:], shape, conf.cell_size)
     r = pab / np.sqrt(np.maximum(pa * pb, eps))
-    dev = a.device
-    f = lambda x: _to_torch(x, dev).float()  # noqa: E731
-    return f(k), f(r), f(pab), f(pa), f(pb), _to_torch(nm, dev).int()
+    return _to_device(a.device, k, r, pab, pa, pb, nm)
 
 
 def delta_to_cross_correlation(delta_a, delta_b, conf, mas="CIC", eps=1e-30):

@@ -33,11 +33,14 @@ def _check(pmid, disp, mesh):
 
 
 def _geom(mesh_spatial, global_shape, offset, particle_cell_size, cell_size):
-    off = torch.as_tensor(offset, dtype=torch.float64).cpu().reshape(-1)
-    if off.numel() == 1:
-        off = off.repeat(3)
-    if off.numel() != 3:
-        raise ValueError("offset must be a scalar or have 3 entries")
+    if type(offset) in (int, float):
+        off = (offset,) * 3
+    else:
+        off = torch.as_tensor(offset, dtype=torch.float64).cpu().reshape(-1)
+        if off.numel() == 1:
+            off = off.repeat(3)
+        if off.numel() != 3:
+            raise ValueError("offset must be a scalar or have 3 entries")
     g = _lib.CicGeom()
     for a in range(3):
         g.local_shape[a] = int(mesh_spatial[a])

@@ -13,6 +13,7 @@ integrated here by an adaptive Dormand-Prince 5(4) pair (Dormand & Prince 1980, 
 from __future__ import annotations
 
 import math
+from bisect import bisect_right
 
 import numpy as np
 
@@ -110,6 +111,7 @@ class GrowthTable:
             tab[m - 1, 1] = m * g + gp
             tab[m - 1, 2] = m * m * g + 2 * m * gp + gpp
         self.table = tab
+        self._nodes, self._rows = self.growth_a.tolist(), tab[0].tolist()  # for the scalar functions
 
     def growth(self, a, order=1, deriv=0):
         a = np.asarray(a, dtype=np.float64)
@@ -123,8 +125,43 @@ class GrowthTable:
         """Growth of the Zel'dovich acceleration, in H_0^2 (nbody/integrator.py:119-122)."""
         return a ** 3 * E2(a, self.cosmo) * (self.growth(a, 1, 2) + (2 + H_deriv(a, self.cosmo)) * self.growth(a, 1, 1))
 
+    # The same functions of one scale factor in Python floats: a step's two kick factors and its drift
+    # factor take 20 us here against 150 us through 0-d arrays, as long as the step's kernels on a
+    # small mesh.  What Python's arithmetic refuses (or makes complex) goes through the arrays.
+
+    def _scalars(self, a, deriv):
+        """(E2, d ln H / d ln a, [linear interpolation of D_1 / a per entry of deriv]) at a > 0."""
+        c = self.cosmo
+        q = -3.0 * (1 + c.w_0 + c.w_a)
+        de = a ** q * math.exp(-3.0 * c.w_a * (1 - a))
+        om, ok, ode = c.Omega_m * a ** -3, c.Omega_k * a ** -2, c.Omega_de * de
+        e2 = om + ok + ode
+        h = 0.5 * (-3.0 * om - 2.0 * ok + ode * (q + 3.0 * c.w_a * a)) / e2
+        x, j = self._nodes, bisect_right(self._nodes, a) - 1
+        if j < 0 or j >= len(x) - 1:
+            return e2, h, [self._rows[d][max(j, 0)] for d in deriv]
+        t, dx = a - x[j], x[j + 1] - x[j]
+        return e2, h, [(f[j + 1] - f[j]) / dx * t + f[j] for f in (self._rows[d] for d in deriv)]
+
+    def _G_D1(self, a):
+        e2, _, (g,) = self._scalars(a, (1,))
+        return a * a * math.sqrt(e2) * (a * g)
+
     def drift_factor(self, a_vel, a_prev, a_next):
+        av, a0, a1 = float(a_vel), float(a_prev), float(a_next)
+        if min(av, a0, a1) > 0:
+            try:
+                return (a1 * self._scalars(a1, (0,))[2][0] - a0 * self._scalars(a0, (0,))[2][0]) / self._G_D1(av)
+            except (ArithmeticError, ValueError):
+                pass
         return float((self.growth(a_next) - self.growth(a_prev)) / self.G_D(a_vel))
 
     def kick_factor(self, a_acc, a_prev, a_next):
+        aa, a0, a1 = float(a_acc), float(a_prev), float(a_next)
+        if min(aa, a0, a1) > 0:
+            try:
+                e2, h, (g1, g2) = self._scalars(aa, (1, 2))
+                return (self._G_D1(a1) - self._G_D1(a0)) / (aa ** 3 * e2 * (aa * g2 + (2 + h) * (aa * g1)))
+            except (ArithmeticError, ValueError):
+                pass
         return float((self.G_D(a_next) - self.G_D(a_prev)) / self.G_K(a_acc))

@@ -26,7 +26,8 @@ def gravity_desc(conf, omega_m) -> _lib.GravityDesc:
     d.cell_size = float(conf.cell_size)
     d.ptcl_spacing = float(conf.ptcl_spacing)
     d.mask_active = int(conf.mask_active)
-    d.omega_m = float(torch.as_tensor(omega_m, dtype=torch.float32))  # cast as gravity.py:630
+    # cast as gravity.py:630 (the field is a float32)
+    d.omega_m = omega_m if type(omega_m) is float else float(torch.as_tensor(omega_m, dtype=torch.float32))
     d.particle_value = float(conf.mesh_size / conf.ptcl_num)
     return d
 
@@ -64,7 +65,9 @@ class _GravityFn(torch.autograd.Function):
     def forward(ctx, disp, omega_m, pmid, valid, conf):
         dev = disp.device
         ensure_init(dev)
-        d = gravity_desc(conf, omega_m.detach())
+        # read back once: the backward needs it too, while the forward's kernels are still running
+        ctx.omega = float(omega_m.detach().to(torch.float32))
+        d = gravity_desc(conf, ctx.omega)
         pm = as_contig(pmid, torch.int16, "pmid")
         dp = as_contig(disp.detach(), torch.float32, "disp")
         n = _check_particles(pm, dp)
@@ -81,7 +84,7 @@ class _GravityFn(torch.autograd.Function):
         dp, omega_m, pm, valid = ctx.saved_tensors
         conf = ctx.conf
         dev = dp.device
-        d = gravity_desc(conf, omega_m.detach())
+        d = gravity_desc(conf, ctx.omega)
         n = _check_particles(pm, dp)
         nbytes = _lib.size_query("pm_gravity_vjp_workspace", d, n)
         ws = workspace(nbytes, dev)

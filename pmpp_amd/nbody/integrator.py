@@ -26,6 +26,7 @@ import torch
 
 from .. import _lib
 from .._torch import as_contig, ensure_init, ptr, stream_handle, workspace
+from ..core.configuration import Configuration
 from ..cosmology import GrowthTable
 
 _TABLES: Dict[tuple, GrowthTable] = {}
@@ -53,7 +54,11 @@ def growth_table(cosmo, conf, omega_m=None) -> GrowthTable:
     om, ok, w0, wa = _cosmo_key(cosmo)
     if omega_m is not None:
         om = float(omega_m)
-    key = (om, ok, w0, wa, tuple(np.asarray(conf.growth_a).tolist()), float(conf.a_lpt_step))
+    if type(conf) is Configuration:  # the fields its nodes are made of, instead of the nodes
+        nodes = (conf.a_start, conf.a_stop, conf.a_nbody_maxstep, conf.a_lpt_maxstep, conf.a_custom)
+    else:
+        nodes = (tuple(np.asarray(conf.growth_a).tolist()), float(conf.a_lpt_step))
+    key = (om, ok, w0, wa, nodes)
     tab = _TABLES.get(key)
     if tab is None:
         tab = GrowthTable(_Background(om, ok, w0, wa), conf.growth_a, conf.a_lpt_step)

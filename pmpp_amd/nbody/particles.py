@@ -8,7 +8,7 @@ torch tensors; ``pmid`` is (N,3) int16, ``disp``/``vel``/``acc`` are (N,3) float
 
 from __future__ import annotations
 
-from dataclasses import dataclass, replace as dc_replace
+from dataclasses import dataclass, fields, replace as dc_replace
 from typing import Any, Optional
 
 import numpy as np
@@ -37,7 +37,19 @@ class Particles:
         return self.pmid.shape[0]
 
     def replace(self, **changes):
-        return dc_replace(self, **changes)
+        if type(self) is not Particles or not changes.keys() <= _FIELDS:
+            return dc_replace(self, **changes)
+        # three of these per step of a run: the fields are set as __init__ and __post_init__ do, which
+        # leaves the unchanged ones as they are
+        p = object.__new__(Particles)
+        d = p.__dict__
+        for name in _FIELDS:
+            v = changes[name] if name in changes else self.__dict__[name]
+            dtype = _DTYPES.get(name)
+            if dtype is not None and (v is not None or name == "pmid") and v.dtype != dtype:
+                v = v.to(dtype)
+            d[name] = v
+        return p
 
     @property
     def valid_mask(self):
@@ -100,3 +112,8 @@ class Particles:
             box = torch.tensor(self.conf.box_size, dtype=dtype, device=p.device)
             p = torch.remainder(p, box)
         return p
+
+
+_FIELDS = {f.name: None for f in fields(Particles)}.keys()
+_DTYPES = {"pmid": torch.int16, "disp": torch.float32, "vel": torch.float32, "acc": torch.float32,
+           "unused_index": torch.bool}

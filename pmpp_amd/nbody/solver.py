@@ -74,7 +74,7 @@ class _Cosmo:
 class _NBodyFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, disp, vel, omega_m, ptcl, cosmo, conf, reverse, correction):
-        c = _Cosmo(cosmo, float(omega_m))
+        c = _Cosmo(cosmo, float(omega_m))  # a tensor is read back here, a float is not
         p = ptcl.replace(disp=disp.detach().contiguous(), vel=vel.detach().contiguous())
         out = _run(p, c, conf, reverse, correction=correction)
         ctx.state = (out, c, conf, reverse, omega_m, correction)
@@ -88,7 +88,9 @@ class _NBodyFn(torch.autograd.Function):
                           vel=vel_cot if vel_cot is not None else zeros,
                           acc=acc_cot if acc_cot is not None else zeros)
         _, cin, om_cot = nbody_adj(out, cot, c, conf, reverse, correction=correction)
-        om = torch.as_tensor(om_cot, dtype=omega_m.dtype, device=omega_m.device).reshape(omega_m.shape)
+        om = None
+        if isinstance(omega_m, torch.Tensor):
+            om = torch.as_tensor(om_cot, dtype=omega_m.dtype, device=omega_m.device).reshape(omega_m.shape)
         return cin.disp, cin.vel, om, None, None, None, None, None
 
 
@@ -111,7 +113,7 @@ def nbody(ptcl, cosmo, conf, reverse=False, correction=None, observer=None):
         with torch.no_grad():
             return _run(ptcl, cosmo, conf, reverse, correction=correction, observer=observer)
     om = cosmo.Omega_m
-    om_t = om if isinstance(om, torch.Tensor) else torch.tensor(float(om), dtype=torch.float64,
-                                                                device=ptcl.disp.device)
-    disp, vel, acc = _NBodyFn.apply(ptcl.disp, ptcl.vel, om_t, ptcl, cosmo, conf, reverse, correction)
+    if not isinstance(om, torch.Tensor):
+        om = float(om)
+    disp, vel, acc = _NBodyFn.apply(ptcl.disp, ptcl.vel, om, ptcl, cosmo, conf, reverse, correction)
     return ptcl.replace(disp=disp, vel=vel, acc=acc)

@@ -125,3 +125,51 @@ def test_validity_mask_is_converted_once_per_mask_and_follows_in_place_changes()
     del p, other, ui, first, changed
     gc.collect()
     assert len(_VALID_MASKS) < n  # entries go with their masks
+
+
+@pytest.mark.parametrize("kw", [{}, dict(Omega_k=0.05, w_0=-0.9, w_a=0.2), dict(w_a=-0.3)])
+def test_step_factors_of_floats_equal_the_array_functions(kw):
+    from pmpp_amd.cosmology import LCDM, GrowthTable
+
+    conf = Configuration(1.0, (8,) * 3)
+    t = GrowthTable(LCDM(Omega_m=0.3, **kw), conf.growth_a, conf.a_lpt_step)
+    nodes = t.growth_a
+    scales = np.concatenate((nodes[1:], 0.5 * (nodes[1:-1] + nodes[2:]), [1.5 * nodes[-1], 0.3 * nodes[1]]))
+    for a in scales:
+        for b in (a + 0.01, 1.1 * a):
+            v = 0.5 * (a + b)
+            d = (t.growth(b) - t.growth(a)) / t.G_D(v)
+            k = (t.G_D(b) - t.G_D(a)) / t.G_K(v)
+            # differences of numbers up to (a, a^2) / (b - a) times larger, each to a few 2^-52
+            tol = 64 * 2.0 ** -52 * b / (b - a)
+            assert t.drift_factor(v, a, b) == pytest.approx(float(d), rel=tol)
+            assert t.kick_factor(v, a, b) == pytest.approx(float(k), rel=tol)
+            assert np.float32(t.drift_factor(v, a, b)) == pytest.approx(np.float32(d), rel=2.0 ** -23)
+    with np.errstate(all="ignore"):  # a scale factor that Python's arithmetic refuses: as the arrays have it
+        assert np.isnan(t.drift_factor(0.0, 0.0, 0.1)) and np.isnan(t.kick_factor(0.1, 0.0, 0.1))
+
+
+def test_growth_tables_are_kept_per_schedule():
+    from pmpp_amd.cosmology import LCDM
+    from pmpp_amd.nbody.integrator import growth_table
+
+    cosmo = LCDM(Omega_m=0.31)
+    a, b = (Configuration(1.0, (8,) * 3, a_nbody_maxstep=s) for s in (1 / 8, 1 / 16))
+    assert growth_table(cosmo, a) is growth_table(cosmo, a.replace(ptcl_spacing=2.0))
+    assert growth_table(cosmo, a) is not growth_table(cosmo, b)
+    for c in (a, b, a.replace(a_custom=(0.1, 0.4, 1.0))):
+        assert np.array_equal(growth_table(cosmo, c).growth_a, c.growth_a)
+
+
+def test_particles_replace_converts_and_refuses_as_the_constructor():
+    import torch
+
+    from pmpp_amd import Particles
+
+    p = Particles(None, torch.zeros(4, 3, dtype=torch.int16), torch.zeros(4, 3))
+    q = p.replace(vel=torch.ones(4, 3, dtype=torch.float64), unused_index=torch.ones(4, dtype=torch.uint8))
+    assert q.vel.dtype == torch.float32 and q.unused_index.dtype == torch.bool
+    assert q.pmid is p.pmid and q.disp is p.disp and p.vel is None
+    assert q.replace(vel=None, pmid=torch.zeros(4, 3)).vel is None
+    with pytest.raises(TypeError):
+        p.replace(velocity=q.vel)
