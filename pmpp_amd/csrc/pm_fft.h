@@ -195,8 +195,25 @@ __device__ __forceinline__ float2 table_tw(const float2* __restrict__ tw, int j)
 // LDS addressing: the logical exchange matrix row = k1 * N2 + n2.  Idx maps a row to a
 // float offset for the calling thread (its column / line slot is folded in by the functor).
 
+// Orders the LDS accesses of a line's threads: a workgroup barrier, or, when they are all in one wave
+// (WAVE), whose LDS instructions run in order anyway, a fence for the compiler only.
+template <bool WAVE>
+__device__ __forceinline__ void line_sync() {
+  if constexpr (WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
+// The line passes' shorter transforms (WAVE, N <= 512) keep four twiddles live at a time: as many waves
+// hide the table's latency (c2r at 512^3 613 -> 594 us; at 1024^3 all at once is faster, 4.5 against
+// 4.6 ms).
+//
 // Forward core.  In: v[n1] = x[N2 n1 + p].  Out: v[j3 N2 + k2] = X[(p + P j3) + N1 k2].
-template <int N, class Idx>
+template <int N, bool WAVE = false, class Idx>
 __device__ __forceinline__ void forward_core(float2* v, float* lds, int p, const Idx& idx,
                                              const float2* __restrict__ tw) {
   using PL = Plan<N>;
@@ -204,33 +221,36 @@ __device__ __forceinline__ void forward_core(float2* v, float* lds, int p, const
   dft<N1, false>(v);
   if constexpr (N2 > 1) {
 #pragma unroll
-    for (int k1 = 1; k1 < N1; ++k1) v[k1] = c_mul(v[k1], table_tw<N, false>(tw, p * k1));
+    for (int k1 = 1; k1 < N1; ++k1) {
+      v[k1] = c_mul(v[k1], table_tw<N, false>(tw, p * k1));
+      if (WAVE && N <= 512 && k1 % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    }
   }
   float tmp[E];
 #pragma unroll
   for (int k1 = 0; k1 < N1; ++k1) lds[idx(k1 * N2 + p)] = v[k1].x;
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int j3 = 0; j3 < PL::J3; ++j3)
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) tmp[j3 * N2 + n2] = lds[idx((p + P * j3) * N2 + n2)];
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int k1 = 0; k1 < N1; ++k1) lds[idx(k1 * N2 + p)] = v[k1].y;
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int j3 = 0; j3 < PL::J3; ++j3)
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2)
       v[j3 * N2 + n2] = make_float2(tmp[j3 * N2 + n2], lds[idx((p + P * j3) * N2 + n2)]);
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int j3 = 0; j3 < PL::J3; ++j3) dft<N2, false>(v + j3 * N2);
 }
 
 // Inverse core (unnormalised).  In: v[j3 N2 + k2] = X[(p + P j3) + N1 k2].
 // Out: v[n1] = x[p + N2 n1].
-template <int N, class Idx>
+template <int N, bool WAVE = false, class Idx>
 __device__ __forceinline__ void inverse_core(float2* v, float* lds, int p, const Idx& idx,
                                              const float2* __restrict__ tw) {
   using PL = Plan<N>;
@@ -241,26 +261,28 @@ __device__ __forceinline__ void inverse_core(float2* v, float* lds, int p, const
 #pragma unroll
     for (int j3 = 0; j3 < PL::J3; ++j3)
 #pragma unroll
-      for (int n2 = 1; n2 < N2; ++n2)
+      for (int n2 = 1; n2 < N2; ++n2) {
         v[j3 * N2 + n2] = c_mul(v[j3 * N2 + n2], table_tw<N, true>(tw, n2 * (p + P * j3)));
+        if (WAVE && N <= 512 && n2 % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+      }
   }
   float tmp[E];
 #pragma unroll
   for (int j3 = 0; j3 < PL::J3; ++j3)
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) lds[idx((p + P * j3) * N2 + n2)] = v[j3 * N2 + n2].x;
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int k1 = 0; k1 < N1; ++k1) tmp[k1] = lds[idx(k1 * N2 + p)];
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int j3 = 0; j3 < PL::J3; ++j3)
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) lds[idx((p + P * j3) * N2 + n2)] = v[j3 * N2 + n2].y;
-  __syncthreads();
+  line_sync<WAVE>();
 #pragma unroll
   for (int k1 = 0; k1 < N1; ++k1) v[k1] = make_float2(tmp[k1], lds[idx(k1 * N2 + p)]);
-  __syncthreads();
+  line_sync<WAVE>();
   dft<N1, true>(v);
 }
 
@@ -357,7 +379,7 @@ struct FoldPlanes {
   int ny_log = 0, b0_log = 0, b1_log = 0, nb0 = 0, nb1 = 0;
 };
 
-// Line pass along the contiguous last axis (real <-> half spectrum).  C2R takes up to three
+// Line pass along the contiguous last axis (real <-> half spectrum), lines in pairs (nlines even).  C2R takes up to three
 // (spectrum, output) pairs in one launch; R2C reads rin into cmain[0].
 struct ZPass {
   const float* rin;    // R2C: real input rows (pitch_r floats)

@@ -272,193 +272,254 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
 }
 
 // --------------------------------------------------------------- z passes ----
-template <int M, bool C2R>
+// Two real lines (2 i and 2 i + 1) of N points per complex transform, z = a + i b: the pair's spectra
+// are A = (Z[k] + conj Z[N-k]) / 2 and B = -i (Z[k] - conj Z[N-k]) / 2.  Against one line as N / 2
+// complex points this has a tenth more butterflies, but no twiddle, no table load and one LDS round
+// less where bins k and N - k meet, which cost as much as the transform: with the loads and stores
+// alone the c2r of three 1024^3 components takes 3.8 ms, with the transform 4.4, with the N / 2-point
+// pairing it took 5.2; now 4.6.  A pair's threads are in one wave, so nothing waits at a barrier.
+// Before -> now, us: c2r 256^3 116 -> 88, 512^3 783 -> 594, 1024^3 5220 -> 4600; r2c with planes
+// 43 -> 33, 256 -> 231, 2050 -> 1450.  Now bound by the memory path (c2r 19.3 GB: 4.2 TB/s; a copy
+// reaches 4.8).
+template <int N>
 struct ZCfg {
-  static constexpr int P = Plan<M>::P;
-  // long lines fill LDS (one slot per line): smaller workgroups let several of them share a CU
-  // and interleave their load / transform / store phases.  From 1024-point lines on, the two
-  // directions part ways (M = 512 against 128 threads for both: c2r 1.795 -> 1.76 ms with 256,
-  // r2c 1.74 -> 1.63 ms with 64)
-  static constexpr int THREADS = M >= 512 ? (C2R ? 256 : 64) : (M >= 256 ? 128 : 256);
-  static constexpr int LINES = THREADS / P;
-  // floats per line slot, with LSTR = P (mod 64) so the 64/P lines of a wave start on
-  // disjoint groups of the 64 LDS banks (the exchange rows of one line are P apart).  R2C
-  // pairs bins k and M - k of the complex transform through a natural-order copy of the line
-  // (M+1 float2); C2R pairs them through a real-only copy in two rounds, so its slot only holds
-  // the larger of that copy (M + 1 floats) and the transform's real/imaginary exchange
-  // (M + M/N2 floats), and twice as many lines fit on a CU.
-  static constexpr int LSTR_MIN =
-      C2R ? (M + M / Plan<M>::N2 > M + 1 ? M + M / Plan<M>::N2 : M + 1) : 2 * (M + 2);
-  static constexpr int LSTR = ((LSTR_MIN + 63) / 64) * 64 + (P % 64);
-  static constexpr int LDS_FLOATS = LINES * LSTR;
+  static constexpr int P = Plan<N>::P;
+  // long lines: more of them per workgroup, so more adjacent rows are written at about the same time
+  // (1024^3, 64 / 128 / 256 / 512 threads: c2r 4.99 / 4.98 / 4.49 / 4.60, r2c 1.70 / 1.65 / 1.62 / 1.45 ms;
+  // 512^3, 256 / 512: 594 / 606, 232 / 238 us)
+  static constexpr int THREADS = N == 1024 ? 512 : 256;
+  static constexpr int PAIRS = THREADS / P;
+  // floats per pair's slot (the transform's real / imaginary exchange), with LSTR = P (mod 64) so the
+  // 64/P pairs of a wave start on disjoint groups of the 64 LDS banks
+  static constexpr int LSTR = ((N + N / Plan<N>::N2 + 63) / 64) * 64 + (P % 64);
+  static constexpr int LDS_FLOATS = PAIRS * LSTR;
+  static_assert(P <= 64, "a pair's threads are in one wave");
 };
 
 // ADD: C2R: the output is rout_add + the scaled line; R2C: rin's planes are folded on load
 // (ZPass::fold).  Separate instantiations, so the plain passes keep their register budget.
-template <int M, bool C2R, bool ADD = false>
-__global__ void __launch_bounds__((ZCfg<M, C2R>::THREADS)) k_zpass(ZPass zp, SpecTables tb,
-                                                                 const float2* __restrict__ tw) {
-  using PL = Plan<M>;
-  using ZC = ZCfg<M, C2R>;
-  constexpr int P = PL::P, E = PL::E, N2 = PL::N2;
+template <int N, bool C2R, bool ADD = false>
+__global__ void __launch_bounds__((ZCfg<N>::THREADS), (C2R && N == 2048 ? 2 : 1))  // c2r: 57 -> 52 us at 64^2 x 2048
+    k_zpass(ZPass zp, SpecTables tb, const float2* __restrict__ tw) {
+  using PL = Plan<N>;
+  using ZC = ZCfg<N>;
+  constexpr int P = PL::P, E = PL::E, N2 = PL::N2, M = N / 2;
   __shared__ float lds[ZC::LDS_FLOATS];
   const int p = threadIdx.x % P;
-  const int line = threadIdx.x / P;
-  const int64_t lg = (int64_t)blockIdx.x * ZC::LINES + line;
-  const bool ok = lg < zp.nlines;
-  float* slot = lds + line * ZC::LSTR;
-  float2* nat = reinterpret_cast<float2*>(slot);
-  auto idx = [&](int row) { return line * ZC::LSTR + row + row / N2; };
+  const int pair = threadIdx.x / P;
+  const int64_t pg = (int64_t)blockIdx.x * ZC::PAIRS + pair;
+  const bool ok = 2 * pg < zp.nlines;
+  const int64_t la = 2 * (ok ? pg : 0);  // clamped: unconditional, batched loads
+  float* slot = lds + pair * ZC::LSTR;
+  auto idx = [&](int row) { return pair * ZC::LSTR + row + row / N2; };
   float2 v[E];
 
-  const int64_t lgl = ok ? lg : zp.nlines - 1;  // clamped line: unconditional, batched loads
   if constexpr (!C2R) {
-    const float* src = zp.rin + lgl * zp.pitch_r;
+    const float* src = zp.rin + la * zp.pitch_r;
 #pragma unroll
-    for (int s = 0; s < E; ++s) v[s] = *reinterpret_cast<const float2*>(src + 2 * nrow<M>(p, s));
+    for (int s = 0; s < E; ++s) v[s] = make_float2(src[nrow<N>(p, s)], src[zp.pitch_r + nrow<N>(p, s)]);
     if constexpr (ADD) {
       // a cell with lx = x mod b0 and ly = y mod b1 takes, from its neighbouring columns (periodic),
       //   lx == 0: XS of column (cx-1, cy) row ly; and when ly == 0 also XS of (cx-1, cy-1) row b1
       //            and YS of (cx, cy-1) row 0
       //   ly == 0: YS of column (cx, cy-1) row lx
       // summed in this order before they are added.  Reading them here saves the pass that
-      // would add them in place (1024^3: 1.67 + 0.54 ms for the two passes, 2.03 ms for this one;
-      // 512^3: 223 + 80 us, 253 us; 256^3: 37 + 11 us, 40 us).
+      // would add them in place.
       const FoldPlanes& fp = zp.fold;
-      const int x = (int)(lgl >> fp.ny_log), y = (int)(lgl & ((1 << fp.ny_log) - 1));
-      const int lx = x & ((1 << fp.b0_log) - 1), ly = y & ((1 << fp.b1_log) - 1);
-      if (lx == 0 || ly == 0) {
-        const int cx = x >> fp.b0_log, cy = y >> fp.b1_log;
-        const int sx = cx == 0 ? fp.nb0 - 1 : cx - 1, sy = cy == 0 ? fp.nb1 - 1 : cy - 1;
-        const int64_t b0 = int64_t(1) << fp.b0_log, b1 = int64_t(1) << fp.b1_log;
-        auto xs_line = [&](int ccy, int64_t row) {
-          return fp.xs + (((int64_t)sx * fp.nb1 + ccy) * (b1 + 1) + row) * zp.pitch_r;
-        };
+      const int x = (int)(la >> fp.ny_log);
+      const int lx = x & ((1 << fp.b0_log) - 1);
+      const int cx = x >> fp.b0_log, sx = cx == 0 ? fp.nb0 - 1 : cx - 1;
+      const int64_t b0 = int64_t(1) << fp.b0_log, b1 = int64_t(1) << fp.b1_log;
+      auto xs_line = [&](int ccy, int64_t row) {
+        return fp.xs + (((int64_t)sx * fp.nb1 + ccy) * (b1 + 1) + row) * zp.pitch_r;
+      };
+      auto fold = [&](int y, auto add) {
+        const int ly = y & ((1 << fp.b1_log) - 1);
+        if (lx != 0 && ly != 0) return;
+        const int cy = y >> fp.b1_log, sy = cy == 0 ? fp.nb1 - 1 : cy - 1;
         const float* ysl = fp.ys + (((int64_t)cx * fp.nb1 + sy) * b0 + lx) * zp.pitch_r;
         const float* p0 = lx == 0 ? xs_line(cy, ly) : ysl;
-        float2 w[E];
+        float w[E];
 #pragma unroll
-        for (int s = 0; s < E; ++s) w[s] = *reinterpret_cast<const float2*>(p0 + 2 * nrow<M>(p, s));
+        for (int s = 0; s < E; ++s) w[s] = p0[nrow<N>(p, s)];
         if (lx == 0 && ly == 0) {
-          // four slots at a time: all at once, the loads would be issued one by one for want of
-          // registers, and the few corner lines would hold up the whole pass (35 % at 1024^3)
+          // eight slots at a time: all at once, the loads would be issued one by one for want of
+          // registers, and the few corner lines would hold up the whole pass
           const float* p1 = xs_line(sy, b1);
-          constexpr int Q = E < 4 ? E : 4;
+          constexpr int Q = E < 8 ? E : 8;
 #pragma unroll
           for (int c = 0; c < E; c += Q) {
-            float2 a[Q], b[Q];
+            float f[Q], g[Q];
 #pragma unroll
             for (int s = 0; s < Q; ++s) {
-              a[s] = *reinterpret_cast<const float2*>(p1 + 2 * nrow<M>(p, c + s));
-              b[s] = *reinterpret_cast<const float2*>(ysl + 2 * nrow<M>(p, c + s));
+              f[s] = p1[nrow<N>(p, c + s)];
+              g[s] = ysl[nrow<N>(p, c + s)];
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s = 0; s < Q; ++s) w[c + s] = c_add(c_add(w[c + s], a[s]), b[s]);
+            for (int s = 0; s < Q; ++s) w[c + s] = (w[c + s] + f[s]) + g[s];
             __builtin_amdgcn_sched_barrier(0);
           }
         }
 #pragma unroll
-        for (int s = 0; s < E; ++s) v[s] = c_add(v[s], w[s]);
-      }
+        for (int s = 0; s < E; ++s) add(s, w[s]);
+      };
+      const int y = (int)(la & ((1 << fp.ny_log) - 1));  // even: both lines have the same x
+      fold(y, [&](int s, float w) { v[s].x += w; });
+      fold(y + 1, [&](int s, float w) { v[s].y += w; });
     }
-    if (zp.rin_add) {  // uniform: the added field's loads join the same batch
-      const float* src2 = zp.rin_add + lgl * zp.pitch_r;
+    if (zp.rin_add) {  // uniform
+      const float* src2 = zp.rin_add + la * zp.pitch_r;
 #pragma unroll
       for (int s = 0; s < E; ++s) {
-        const float2 w = *reinterpret_cast<const float2*>(src2 + 2 * nrow<M>(p, s));
-        v[s] = make_float2(v[s].x + w.x, v[s].y + w.y);
+        v[s].x += src2[nrow<N>(p, s)];
+        v[s].y += src2[zp.pitch_r + nrow<N>(p, s)];
       }
     }
 #pragma unroll
     for (int s = 0; s < E; ++s)
       v[s] = make_float2((v[s].x + zp.src_shift) * zp.src_scale, (v[s].y + zp.src_shift) * zp.src_scale);
-    forward_core<M>(v, lds, p, idx, tw);
+    forward_core<N, true>(v, lds, p, idx, tw);
+    // bins k and N - k meet in a natural-order copy of the transform, real parts first
+    constexpr int H = E / 2;  // bins k = p + P j < N / 2 per thread
+    float sr[H], dr[H], mr, mi;
 #pragma unroll
-    for (int s = 0; s < E; ++s) nat[xrow<M>(p, s)] = v[s];
-    __syncthreads();
-    float2* dst = zp.cmain[0] + lg * zp.pitch_c;
+    for (int s = 0; s < E; ++s) slot[xrow<N>(p, s)] = v[s].x;
+    line_sync<true>();
+    mr = slot[M];
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      int k = p + P * j;
-      float2 a = nat[k];
-      float2 bc = c_conj(nat[(M - k) & (M - 1)]);
-      float2 d = c_sub(a, bc);
-      float2 fe = c_scale(c_add(a, bc), 0.5f);
-      float2 fo = make_float2(0.5f * d.y, -0.5f * d.x);  // -i (a - bc) / 2
-      float2 x = c_add(fe, c_mul(table_tw<2 * M, false>(tw, k), fo));
-      if (ok && k < zp.kz_lim) dst[k] = x;
+    for (int j = 0; j < H; ++j) {
+      const int k = p + P * j;
+      const float a = slot[k], b = slot[(N - k) & (N - 1)];
+      sr[j] = 0.5f * (a + b);
+      dr[j] = 0.5f * (b - a);
     }
-    if (ok && p == 0 && zp.nyq) {
-      float2 z0 = nat[0];
-      dst[M] = make_float2(z0.x - z0.y, 0.f);
+    line_sync<true>();
+#pragma unroll
+    for (int s = 0; s < E; ++s) slot[xrow<N>(p, s)] = v[s].y;
+    line_sync<true>();
+    mi = slot[M];
+    if (!ok) return;
+    float2* da = zp.cmain[0] + la * zp.pitch_c;
+    float2* db = da + zp.pitch_c;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      const int k = p + P * j;
+      if (k < zp.kz_lim) {
+        const float a = slot[k], b = slot[(N - k) & (N - 1)];
+        da[k] = make_float2(sr[j], 0.5f * (a - b));
+        db[k] = make_float2(0.5f * (a + b), dr[j]);
+      }
+    }
+    if (p == 0 && zp.nyq) {
+      da[M] = make_float2(mr, 0.f);
+      db[M] = make_float2(mi, 0.f);
     }
   } else {
-    (void)nat;
+    // Z[k] = A[k] + i B[k], and conj A + i conj B of N - k above N / 2, which a thread gets from the one that
+    // read those through a natural-order copy in LDS, real parts first (reading the half spectra a
+    // second time, in reverse and from the cache, took 15 % longer at N = 1024)
     const int comp = blockIdx.y;
-    const float2* srcm = zp.cmain[comp] + lgl * zp.pitch_c;
-    float2 xn = srcm[zp.nyq ? M : 0];  // unconditional: column 0 stands in when there is none
+    const float2* sa = zp.cmain[comp] + la * zp.pitch_c;
+    const float2* sb = sa + zp.pitch_c;
     const int klim = zp.kz_lim < M ? zp.kz_lim : M;
-#pragma unroll
-    for (int j = 0; j < E; ++j)  // P*j < klim is uniform: columns past the band cost no load
-      v[j] = (P * j < klim) ? srcm[min(p + P * j, klim - 1)] : make_float2(0.f, 0.f);
-#pragma unroll
-    for (int j = 0; j < E; ++j)
-      if (p + P * j >= klim) v[j] = make_float2(0.f, 0.f);
-    if (!zp.nyq) xn = make_float2(0.f, 0.f);
-    if ((zp.deriv >> comp) & 1) {
-#pragma unroll
-      for (int j = 0; j < E; ++j) v[j] = c_imul(tb.negk[2][p + P * j], v[j]);
-      xn = c_imul(tb.negk[2][M], xn);
+    const bool deriv = (zp.deriv >> comp) & 1;
+    // slot s < E / 2 in this order has a bin base + p below N / 2, and E - 1 - s the bins N - base - p
+    auto bin = [](int s) constexpr { return P * (s / N2) + PL::N1 * (s % N2); };
+    float2 ma = make_float2(0.f, 0.f), mb = ma;  // the Nyquist bin
+    if (zp.nyq && p == 0) {
+      ma = sa[M];
+      mb = sb[M];
     }
-    // pair bins k (the X-layout slot) and M - k through a natural-order real copy of the line,
-    // real parts first, then imaginary parts (the slot holds M + 1 floats, not M + 1 float2):
-    // e = (X[k] + conj X[M-k]) / 2, d = X[k] - conj X[M-k]
-    float* rl = lds + line * ZC::LSTR;
-    float ex[E], dx[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) rl[p + P * j] = v[j].x;
-    if (p == 0) rl[M] = xn.x;
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < E; ++s) {
-      const int k = xrow<M>(p, s);
-      const float a = rl[k], b = rl[M - k];
-      ex[s] = a + b;
-      dx[s] = a - b;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < E; ++j) rl[p + P * j] = v[j].y;
-    if (p == 0) rl[M] = xn.y;
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < E; ++s) {
-      const int k = xrow<M>(p, s);
-      // irfft uses only the real parts of the DC and Nyquist bins
-      const float a = k == 0 ? 0.f : rl[k], b = k == 0 ? 0.f : rl[M - k];
-      float2 e = c_scale(make_float2(ex[s], a - b), 0.5f);
-      float2 o = c_scale(c_mulconj(make_float2(dx[s], a + b), table_tw<2 * M, false>(tw, k)), 0.5f);
-      v[s] = make_float2(e.x - o.y, e.y + o.x);  // e + i o
-    }
-    __syncthreads();
-    inverse_core<M>(v, lds, p, idx, tw);
-    if (ok) {
-      float* dst = zp.rout[comp] + lg * zp.pitch_r;
-      if constexpr (ADD) {
-        const float* add = zp.rout_add + lg * zp.pitch_r;
-#pragma unroll
-        for (int s = 0; s < E; ++s) {
-          int m = nrow<M>(p, s);
-          const float2 w = *reinterpret_cast<const float2*>(add + 2 * m);
-          v[s] = make_float2(w.x + v[s].x * zp.out_scale, w.y + v[s].y * zp.out_scale);
+    // the slots below N / 2, at most 16 at a time (64-slot threads would not have the registers)
+    constexpr int H2 = N2 > 1 ? N2 / 2 : 1;
+    auto low = [](int i) constexpr { return (i / H2) * N2 + i % H2; };
+    constexpr int Q = E / 2 < 16 ? E / 2 : 16;
+    static_for<0, E / 2 / Q>([&](auto C) {
+      float2 a[Q], b[Q];
+      static_for<0, Q>([&](auto I) {
+        constexpr int i = decltype(I)::value, k = bin(low(decltype(C)::value * Q + i));
+        a[i] = b[i] = make_float2(0.f, 0.f);
+        if (k + P <= klim) {  // uniform: the whole slot is in the band
+          a[i] = sa[k + p];
+          b[i] = sb[k + p];
+        } else if (k + p < klim) {
+          a[i] = sa[k + p];
+          b[i] = sb[k + p];
         }
-      } else {
-#pragma unroll
-        for (int s = 0; s < E; ++s) v[s] = make_float2(v[s].x * zp.out_scale, v[s].y * zp.out_scale);
+      });
+      if (deriv) {
+        static_for<0, Q>([&](auto I) {
+          constexpr int i = decltype(I)::value, k = bin(low(decltype(C)::value * Q + i));
+          const float m = tb.negk[2][k + p];
+          a[i] = c_imul(m, a[i]);
+          b[i] = c_imul(m, b[i]);
+        });
       }
+      static_for<0, Q>([&](auto I) {
+        constexpr int i = decltype(I)::value, s = low(decltype(C)::value * Q + i);
+        if constexpr (s == 0) {  // irfft uses only the real parts of the DC and Nyquist bins
+          if (p == 0) a[i].y = b[i].y = 0.f;
+        }
+        v[s] = make_float2(a[i].x - b[i].y, a[i].y + b[i].x);
+        v[E - 1 - s].y = b[i].x - a[i].y;
+        if (bin(s) < klim) slot[bin(s) + p] = a[i].x + b[i].y;
+      });
+      if constexpr (E / 2 > Q) __builtin_amdgcn_sched_barrier(0);
+    });
+    if (deriv) {
+      ma = c_imul(tb.negk[2][M], ma);
+      mb = c_imul(tb.negk[2][M], mb);
+    }
+    line_sync<true>();
+    auto mirrored = [&](auto set) {
+      static_for<0, E>([&](auto S) {
+        constexpr int s = decltype(S)::value;
+        if constexpr (bin(s) >= M) {
+          const int k = N - bin(s) - p;  // in (0, N / 2]
+          float f = 0.f;
+          if (N - bin(s) - P + 1 < klim) f = slot[k];  // uniform
+          set(s, k < klim ? f : 0.f);
+        }
+      });
+    };
+    float re[E];
+    mirrored([&](int s, float f) { re[s] = f; });
+    line_sync<true>();
+    static_for<0, E>([&](auto S) {
+      constexpr int s = decltype(S)::value;
+      if constexpr (bin(s) < M) {
+        if (bin(s) < klim) slot[bin(s) + p] = v[E - 1 - s].y;
+      }
+    });
+    line_sync<true>();
+    mirrored([&](int s, float f) { v[s] = make_float2(re[s], f); });
+    line_sync<true>();
+    static_for<0, E>([&](auto S) {
+      constexpr int s = decltype(S)::value;
+      if constexpr (bin(s) == M) {
+        if (p == 0) v[s] = make_float2(ma.x, mb.x);
+      }
+    });
+    asm volatile("" ::: "memory");  // no twiddle loaded before the spectra are in
+    inverse_core<N, true>(v, lds, p, idx, fresh_table(tw));
+    if (!ok) return;
+    float* da = zp.rout[comp] + la * zp.pitch_r;
+    float* db = da + zp.pitch_r;
+    const float sc = 0.5f * zp.out_scale;
+    if constexpr (ADD) {
+      const float* ea = zp.rout_add + la * zp.pitch_r;
 #pragma unroll
-      for (int s = 0; s < E; ++s) *reinterpret_cast<float2*>(dst + 2 * nrow<M>(p, s)) = v[s];
+      for (int s = 0; s < E; ++s)
+        v[s] = make_float2(ea[nrow<N>(p, s)] + v[s].x * sc, ea[zp.pitch_r + nrow<N>(p, s)] + v[s].y * sc);
+    } else {
+#pragma unroll
+      for (int s = 0; s < E; ++s) v[s] = make_float2(v[s].x * sc, v[s].y * sc);
+    }
+#pragma unroll
+    for (int s = 0; s < E; ++s) {
+      da[nrow<N>(p, s)] = v[s].x;
+      db[nrow<N>(p, s)] = v[s].y;
     }
   }
 }
@@ -549,28 +610,28 @@ int launch_cols_n(int mode, const ColPass& cp, int batches, const SpecTables& tb
   }
 }
 
-template <int M>
+template <int N>
 int launch_z_n(bool c2r, const ZPass& zp, const SpecTables& tb, hipStream_t s) {
-  using ZI = ZCfg<M, true>;   // c2r workgroups
-  using ZF = ZCfg<M, false>;  // r2c workgroups
   const float2* tw = twiddle_table();
   PM_RETURN_IF(tw == nullptr, PM_ERROR_HIP, "twiddle table not initialised");
+  PM_RETURN_IF(zp.nlines % 2 != 0, PM_ERROR_UNSUPPORTED, "the FFT line passes take pairs of lines");
   if (zp.nlines == 0) return PM_SUCCESS;
+  const unsigned blocks = (unsigned)ceil_div(zp.nlines / 2, ZCfg<N>::PAIRS);
+  const dim3 threads(ZCfg<N>::THREADS);
   if (c2r) {
-    const dim3 grid((unsigned)ceil_div(zp.nlines, ZI::LINES), (unsigned)zp.ncomp);
+    const dim3 grid(blocks, (unsigned)zp.ncomp);
     if (zp.rout_add) {
-      hipLaunchKernelGGL((k_zpass<M, true, true>), grid, dim3(ZI::THREADS), 0, s, zp, tb, tw);
+      hipLaunchKernelGGL((k_zpass<N, true, true>), grid, threads, 0, s, zp, tb, tw);
       PM_LAUNCHED("fft_z_c2r_add", s);
     } else {
-      hipLaunchKernelGGL((k_zpass<M, true>), grid, dim3(ZI::THREADS), 0, s, zp, tb, tw);
+      hipLaunchKernelGGL((k_zpass<N, true>), grid, threads, 0, s, zp, tb, tw);
       PM_LAUNCHED("fft_z_c2r", s);
     }
   } else {
-    const dim3 grid((unsigned)ceil_div(zp.nlines, ZF::LINES));
     if (zp.fold.xs)
-      hipLaunchKernelGGL((k_zpass<M, false, true>), grid, dim3(ZF::THREADS), 0, s, zp, tb, tw);
+      hipLaunchKernelGGL((k_zpass<N, false, true>), dim3(blocks), threads, 0, s, zp, tb, tw);
     else
-      hipLaunchKernelGGL((k_zpass<M, false>), grid, dim3(ZF::THREADS), 0, s, zp, tb, tw);
+      hipLaunchKernelGGL((k_zpass<N, false>), dim3(blocks), threads, 0, s, zp, tb, tw);
     PM_LAUNCHED("fft_z_r2c", s);
   }
   return PM_SUCCESS;
@@ -595,11 +656,10 @@ int launch_cols(int n, int mode, const ColPass& cp, int batches, const SpecTable
 int launch_z(int nz, bool c2r, const ZPass& zp, const SpecTables& tb, hipStream_t s) {
   if (nz < 2 || nz > 2048 || !is_pow2(nz))
     return fail(PM_ERROR_UNSUPPORTED, "last FFT axis must be a power of two in [2, 2048]");
-  switch (nz / 2) {
+  switch (nz) {
 #define PM_CASE(V) \
   case V: return launch_z_n<V>(c2r, zp, tb, s);
-    PM_CASE(1) PM_CASE(2) PM_CASE(4) PM_CASE(8) PM_CASE(16) PM_CASE(32) PM_CASE(64) PM_CASE(128)
-    PM_CASE(256) PM_CASE(512) PM_CASE(1024)
+    PM_POW2_CASES(PM_CASE)
 #undef PM_CASE
     default: return fail(PM_ERROR_UNSUPPORTED, "last FFT axis must be a power of two in [2, 2048]");
   }

@@ -55,3 +55,35 @@ def test_spectral_force_multiply_matches_oracle(device, ratio, axis):
         got = spectral_force_multiply(torch.from_numpy(X).to(device), gravity_desc(conf, 0.3), axis, adjoint)
         ref = (np.conj(G) if adjoint else G) * X.astype(np.complex128)
         np.testing.assert_allclose(got.cpu().numpy(), ref, rtol=2e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("nz", [2 ** e for e in range(1, 12)])
+def test_line_pairs_of_unlike_size_and_banded_lines(device, nz):
+    # every line length: neighbouring lines (transformed together) a factor 2^10 apart
+    shape = (2, 4, nz)
+    rng = np.random.default_rng(nz)
+    x = rng.normal(size=shape).astype(np.float32)
+    x[:, 1::2] *= 2.0 ** -10
+    X = rfftn(torch.from_numpy(x).to(device)).cpu().numpy()
+    ref = np.fft.rfftn(x.astype(np.float64))
+    tol = 2e-6 * np.log2(x.size)  # of the rms, as for the white noise above
+    assert np.abs(X - ref).max() < tol * np.sqrt(x.size)
+    Y = np.fft.rfft(x.astype(np.float64), axis=2).astype(np.complex64)
+    Y = np.fft.fft(np.fft.fft(Y.astype(np.complex128), axis=0), axis=1).astype(np.complex64)
+    y = irfftn(torch.from_numpy(Y).to(device), s=shape).cpu().numpy()
+    np.testing.assert_allclose(y, np.fft.irfftn(Y.astype(np.complex128), s=shape, axes=(0, 1, 2)), atol=1.5 * tol)
+    # the band of a mesh 1, 2 and 4 times the particle grid: the potential in float64
+    from pmpp_amd.nbody.gravity import gravity_potential
+
+    for ratio in (1, 2, 4):
+        if nz < 2 * ratio:
+            continue
+        conf = Configuration(float(ratio), (8 // ratio, 8 // ratio, nz // ratio), mesh_shape=ratio)
+        rho = rng.normal(size=(8, 8, nz)).astype(np.float32)
+        masks = spectral.particle_nyquist_masks(conf.mesh_shape, conf.ptcl_grid_shape, conf.ptcl_spacing,
+                                                conf.cell_size)
+        G = spectral.green_multiplier(conf.mesh_shape, conf.cell_size, masks)
+        phi = np.fft.irfftn(G * np.fft.rfftn(0.45 * (rho.astype(np.float64) - 1)), s=rho.shape, axes=(0, 1, 2))
+        got = gravity_potential(torch.from_numpy(rho).to(device), 0.3, conf).cpu().numpy()
+        # two transforms and a symbol of a few ulp, of the largest value
+        np.testing.assert_allclose(got, phi, atol=4e-6 * np.log2(rho.size) * max(np.abs(phi).max(), 1e-6))
