@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from .. import _lib
-from .._torch import ensure_init, ptr, require_device, stream_handle
+from .._torch import as_contig, ensure_init, ptr, require_device, stream_handle
 from ..cosmology.background import E2
 from ..nbody.integrator import growth_table
 from ..nbody.particles import Particles
@@ -68,7 +68,7 @@ def lpt(modes, cosmo, conf):
     cell_vol = conf.ptcl_spacing ** 3
     pots = []
     if conf.lpt_order > 0:
-        pots.append(kg.op(modes.to(torch.complex64).contiguous(), POTENTIAL, scale=1.0 / cell_vol))
+        pots.append(kg.op(as_contig(modes, torch.complex64, "modes"), POTENTIAL, scale=1.0 / cell_vol))
     if conf.lpt_order > 1:
         L = second_order_source(kg, pots[0])
         src2 = rfftn(L)

@@ -87,3 +87,12 @@ def test_line_pairs_of_unlike_size_and_banded_lines(device, nz):
         got = gravity_potential(torch.from_numpy(rho).to(device), 0.3, conf).cpu().numpy()
         # two transforms and a symbol of a few ulp, of the largest value
         np.testing.assert_allclose(got, phi, atol=4e-6 * np.log2(rho.size) * max(np.abs(phi).max(), 1e-6))
+
+
+def test_inverse_of_a_conjugate_view(device):
+    shape = (8, 16, 32)
+    X = rfftn(torch.randn(shape, generator=torch.Generator().manual_seed(1)).to(device))
+    lazy = X.conj()
+    assert lazy.is_conj()
+    assert torch.equal(irfftn(lazy, s=shape), irfftn(lazy.resolve_conj().clone(), s=shape))
+    assert not torch.equal(irfftn(lazy, s=shape), irfftn(X, s=shape))

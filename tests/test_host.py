@@ -173,3 +173,22 @@ def test_particles_replace_converts_and_refuses_as_the_constructor():
     assert q.replace(vel=None, pmid=torch.zeros(4, 3)).vel is None
     with pytest.raises(TypeError):
         p.replace(velocity=q.vel)
+
+
+def test_lazy_views_are_written_out_for_the_kernels(monkeypatch):
+    import ctypes
+
+    import torch
+
+    from pmpp_amd import _torch
+
+    monkeypatch.setattr(_torch, "require_device", lambda t, name: t)
+    z = torch.complex(torch.arange(6.0).view(2, 3), 1.0 + torch.arange(6.0).view(2, 3))
+    for t, dtype in ((z.conj(), torch.complex64), (z.conj().T, torch.complex64), (z, torch.complex64),
+                     (torch._neg_view(z.real.clone()), torch.float32), (z.conj().imag, torch.float32)):
+        got = _torch.as_contig(t, dtype, "t")
+        want = t.resolve_conj().resolve_neg().contiguous()
+        # what a kernel reads through the pointer
+        raw = ctypes.string_at(got.data_ptr(), got.numel() * got.element_size())
+        assert raw == want.numpy().tobytes()
+    assert _torch.as_contig(z, torch.complex64, "z") is z  # nothing to do: no copy
