@@ -122,9 +122,8 @@ int pm_cic_scatter_bwd(const int16_t* pmid, const float* disp, const uint8_t* va
  * pm_cic_gather_bwd_tiled  pm_cic_gather_bwd with mesh_cot overwritten, the same way.
  * Both take one-channel meshes without offset, corner drops or a cell size of their own, whose axes
  * are whole bricks, and enough particles; pm_cic_tiled_workspace gives the workspace they need, or 0
- * for a call that only the plain entry points take (PM_ERROR_UNSUPPORTED here).  Values too far below
- * the largest for the fixed point, and all when a value or a position is not finite, go
- * through the plain entry points' float atomics, decided on the device. */
+ * for a call that only the plain entry points take (PM_ERROR_UNSUPPORTED here).  The float32
+ * deposits are those of the plain entry points; a cell's are added in float64. */
 int pm_cic_tiled_workspace(int64_t n, int32_t channels, const pm_cic_geom* geom, size_t* bytes);
 int pm_cic_scatter_tiled(const int16_t* pmid, const float* disp, const uint8_t* valid, const float* val,
                          float val_scalar, int64_t n, const pm_cic_geom* geom, const float* base, float* mesh,

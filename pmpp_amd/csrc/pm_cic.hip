@@ -4,11 +4,9 @@
 // entry points (the reference's pallas_scatter/pallas_gather/*_bwd contract, with offset,
 // explicit mesh cell size, validity mask, channels and local/global shapes).  The gravity
 // step uses its own sorted-order kernels (pm_gravity.hip) built on the same device geometry.
-#include <algorithm>
 #include <mutex>
 #include <vector>
 
-#include "pm_cic.h"
 #include "pm_common.h"
 #include "pm_sort.h"
 
@@ -44,26 +42,20 @@ __global__ void __launch_bounds__(kBlock) k_scatter(const int16_t* __restrict__ 
                                                     const float* __restrict__ disp,
                                                     const uint8_t* __restrict__ valid,
                                                     const float* __restrict__ val, float val_scalar,
-                                                    int64_t n, int C, Geom g, float* __restrict__ mesh,
-                                                    const float* __restrict__ above) {
-  const float lim = above ? *above : 0.f;
-  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
-    if (above) {  // zeros add nothing, unless a position may be NaN
-      const float v = fabsf(val ? val[p] : 1.f);
-      if (v >= lim || (v == 0.f && lim == lim)) continue;
-    }
-    if (valid && !valid[p]) continue;
-    AxisCic ax[3];
-    particle_cic(g, pmid, disp, p, ax);
+                                                    int64_t n, int C, Geom g, float* __restrict__ mesh) {
+  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  if (valid && !valid[p]) return;
+  AxisCic ax[3];
+  particle_cic(g, pmid, disp, p, ax);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      int64_t flat;
-      if (!corner_index(g, ax, c, flat)) continue;
-      float w = corner_weight(ax, c);
-      for (int ch = 0; ch < C; ++ch) {
-        float v = val ? val[p * C + ch] : val_scalar;
-        atomic_add_f32(mesh + flat * C + ch, v * w);
-      }
+  for (int c = 0; c < 8; ++c) {
+    int64_t flat;
+    if (!corner_index(g, ax, c, flat)) continue;
+    float w = corner_weight(ax, c);
+    for (int ch = 0; ch < C; ++ch) {
+      float v = val ? val[p * C + ch] : val_scalar;
+      atomic_add_f32(mesh + flat * C + ch, v * w);
     }
   }
 }
@@ -198,17 +190,6 @@ int check_cic_args(const int16_t* pmid, const float* disp, int64_t n, int32_t C,
 }
 
 }  // namespace
-
-int cic_scatter_rest(const int16_t* pmid, const float* disp, const uint8_t* valid, const float* val, float val_scalar,
-                     int64_t n, const pm_cic_geom* geom, float* mesh, const float* above, hipStream_t s) {
-  // a bounded grid: mostly it only looks at the values
-  const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kBlock), 8192);
-  hipLaunchKernelGGL(k_scatter, dim3(blocks), dim3(kBlock), 0, s, pmid, disp, valid, val, val_scalar, n, 1,
-                     make_geom(*geom), mesh, above);
-  PM_LAUNCHED("k_scatter", s);
-  return PM_SUCCESS;
-}
-
 }  // namespace pm
 
 using namespace pm;
@@ -271,7 +252,7 @@ int pm_cic_scatter(const int16_t* pmid, const float* disp, const uint8_t* valid,
   if (n == 0) return PM_SUCCESS;
   hipLaunchKernelGGL(k_scatter, dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0,
                      as_stream(stream), pmid, disp, valid, val, val_scalar, n, channels,
-                     make_geom(*geom), mesh, nullptr);
+                     make_geom(*geom), mesh);
   PM_LAUNCHED("k_scatter", as_stream(stream));
   return PM_SUCCESS;
 }

@@ -17,8 +17,8 @@
 // passes: 4R + 14C bytes of mesh traffic instead of 4R + 20C.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
-#include "pm_cic.h"
 #include "pm_common.h"
 #include "pm_fft_launch.h"
 #include "pm_sort.h"
@@ -111,7 +111,8 @@ __global__ void __launch_bounds__(kBlock) k_gather3_sorted(const int16_t* __rest
 // mesh: scatter 2.26 -> 1.54 ms, gather 4.95 -> 4.71 ms).
 //
 // Scatter (owner computes): a run of a column's bricks is accumulated one after the other into an
-// LDS tile of (BX+1)(BY+1)(BZ+1) int64 fixed-point cells with LDS atomics.  The tile's upper z
+// LDS tile of (BX+1)(BY+1)(BZ+1) 64-bit cells (int64 fixed point; the CIC entry points' are float64) with
+// LDS atomics.  The tile's upper z
 // plane belongs to the next brick of the column and is carried to it inside LDS; the lower plane
 // of the run's first brick gets the carry of the brick below (the one above the periodic
 // wrap for the first) from that brick's own particles in its last z plane, read a second time.
@@ -124,10 +125,10 @@ __global__ void __launch_bounds__(kBlock) k_gather3_sorted(const int16_t* __rest
 // are read as aligned rows; the z = BZ plane is the lower plane of the brick above, kept in
 // LDS from the previous step (read directly for the first), so no row costs a second cache line.
 constexpr int kTileMaxFloats = 19100;  // gather f32 tile: (32+1)*(16+1)*(32+2) = 19074 fits
-constexpr int kTileMaxWords = 9900;    // scatter int64 tile: (16+1)*(16+1)*(32+2) = 9826 (78.6 KB: 2 WG/CU)
+constexpr int kTileMaxWords = 9900;    // scatter 64-bit tile: (16+1)*(16+1)*(32+2) = 9826 (78.6 KB: 2 WG/CU)
 constexpr int kPlaneMax = 1100;        // (b0+1)*(b1+1) cells of one z plane of a tile
-// Scatter accumulation is exact 64-bit fixed point (2^-32 units): gfx950's LDS integer atomics run
-// an order of magnitude faster than its LDS float atomics, and integer sums are order independent,
+// The force step's scatter accumulation is exact 64-bit fixed point (2^-32 units): gfx950's LDS integer atomics run
+// an order of magnitude faster than its LDS float32 atomics, and integer sums are order independent,
 // so the density is deterministic; each cell is rounded to float32 once when stored.
 constexpr float kFix = 4294967296.0f;         // 2^32
 constexpr float kUnfix = 2.3283064365386963e-10f;  // 2^-32
@@ -242,41 +243,32 @@ __device__ __forceinline__ float frac_weight(const float f[3], int c) {
   return wx * wy * wz;
 }
 
-// What the CIC entry points' scatter has beyond the force step's (CIC = true): its fixed point, left by
-// k_cic_scale, a factor on output, and a mesh that the owned cells are added to (base, null: none).
-struct CicScale {
-  float vs;    // power of two that brings the largest value to [1/2, 1)
-  float fix;   // power of two: the fixed point's unit is 1 / fix
-  float tiny;  // values of smaller magnitude are left to the atomics (NaN: all are)
-};
-struct ScatterOpt {
-  const CicScale* cic = nullptr;
-  float scale = 1.f;
-  const float* base = nullptr;
-};
+// A tile's sum: the force step's fixed point, or (CIC) float64.  The CIC entry points take values of any
+// range, so no common unit serves them: their deposits are the float32 products that float atomics
+// would add, summed in float64, so that every cell is as good as its own deposits (ds_add_f64: 128^3
+// particles on a 256^3 mesh in 36 us, as with the fixed point).
+template <bool CIC>
+using TileSum = std::conditional_t<CIC, double, unsigned long long>;
 
 template <int BX, int BY, int BZ, bool CIC>
 __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_columns(
     const float4* __restrict__ rec, const int32_t* __restrict__ bin_off, float val, Bricks k, int run,
     float* __restrict__ mesh, float* __restrict__ xs, float* __restrict__ ys, const float* __restrict__ vals,
-    const float* __restrict__ vscale, ScatterOpt opt) {
+    const float* __restrict__ vscale, const float* __restrict__ base) {
   using B_ = BrickShape<BX, BY, BZ>;
+  using Sum = TileSum<CIC>;
   constexpr int NT = B_::NT;
-  __shared__ __align__(16) unsigned long long tile[B_::TW];
-  // per-particle values (sorted order) are brought to |v| <= 1 by vscale[0] before the fixed
-  // point and scaled back on output; a constant value is used as it is (CIC: times opt.scale on output)
-  float fix = kFix, unfix1 = kUnfix, vs = 1.f, tiny = 0.f, post = 1.f;
-  if constexpr (CIC) {
-    fix = opt.cic->fix;
-    unfix1 = 1.f / fix;
-    tiny = opt.cic->tiny;
-    post = tiny == tiny ? opt.scale : 0.f;  // all left to the atomics: zeros on the base, whatever the factor
-    if (vals) vs = opt.cic->vs;
-  } else {
-    if (vals) vs = vscale[0];
-  }
-  const float us = (vals ? unfix1 / vs : unfix1) * post;
-  auto unfix = [&](unsigned long long x) { return (float)(long long)x * us; };
+  __shared__ __align__(16) Sum tile[B_::TW];
+  // fixed point: per-particle values (sorted order) are brought to |v| <= 1 by vscale[0] and scaled
+  // back on output; a constant value is used as it is
+  const float vs = !CIC && vals ? vscale[0] : 1.f;
+  const float us = !CIC && vals ? kUnfix / vs : kUnfix;
+  auto unfix = [&](Sum x) {
+    if constexpr (CIC)
+      return (float)x;
+    else
+      return (float)(long long)x * us;
+  };
   const B_ B(k);
   const int col = column_of(blockIdx.x, gridDim.x);
   const int cx = col / k.nb[1], cy = col - cx * k.nb[1];
@@ -284,7 +276,7 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
   const int64_t n1 = k.n[1], n2 = k.n[2];
   const int bz0 = blockIdx.y * run, bz1 = min(k.nb[2], bz0 + run);
   const int32_t* off = bin_off + (int64_t)col * k.nb[2];
-  for (int i = threadIdx.x; i < tf; i += NT) tile[i] = 0ull;
+  for (int i = threadIdx.x; i < tf; i += NT) tile[i] = Sum(0);
   // Particles stream in chunks of NT * PPT in index order (the bricks' bins are contiguous).  The
   // loads of the next chunk are issued before the current one is accumulated, so they are in
   // flight across the flush between bricks.
@@ -299,13 +291,16 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
   };
   auto add = [&](const float4& r, int64_t j, int c0, int c_begin) {  // corners c_begin .. 7 (4: the upper z plane)
     const float fr[3] = {r.x, r.y, r.z};
-    float v = vals ? vals[j] : val;
-    if (CIC && !(fabsf(v) >= tiny)) return;
-    if (vals) v *= vs;
+    const float v = vals ? vals[j] * vs : val;
 #pragma unroll
     for (int c = 0; c < 8; ++c)
-      if (c >= c_begin)
-        atomicAdd(&tile[c0 + B.corner_off(c)], (unsigned long long)__float2ll_rn(v * frac_weight(fr, c) * fix));
+      if (c >= c_begin) {
+        const float dep = v * frac_weight(fr, c);
+        if constexpr (CIC)
+          atomicAdd(&tile[c0 + B.corner_off(c)], (double)dep);
+        else
+          atomicAdd(&tile[c0 + B.corner_off(c)], (unsigned long long)__float2ll_rn(dep * kFix));
+      }
   };
   const int64_t run0 = off[bz0], run1 = off[bz1];
   float4 raw[PPT];
@@ -343,10 +338,10 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
     __syncthreads();
     // z carry: the plane z = b2 is the next brick's z = 0 plane
     for (int r = threadIdx.x; r < rows; r += NT) {
-      unsigned long long* row = tile + r * P;
-      const unsigned long long cin = row[carry];
+      Sum* row = tile + r * P;
+      const Sum cin = row[carry];
       row[carry] = row[B.b2];
-      row[B.b2] = 0ull;
+      row[B.b2] = Sum(0);
       row[0] += cin;
     }
     __syncthreads();
@@ -377,12 +372,12 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
           y = BY;
           dst = &ys[((int64_t)col * BX + x) * n2 + o[2] + 4 * c4];
         }
-        longlong2* src = reinterpret_cast<longlong2*>(&tile[B.cell(x, y, 4 * c4)]);
-        const longlong2 lo = src[0], hi = src[1];
-        src[0] = src[1] = make_longlong2(0, 0);
-        float4 o = make_float4((float)lo.x * us, (float)lo.y * us, (float)hi.x * us, (float)hi.y * us);
-        if (CIC && opt.base && it < OWN) {
-          const float4 m = *reinterpret_cast<const float4*>(opt.base + (dst - mesh));
+        Sum* src = &tile[B.cell(x, y, 4 * c4)];  // 16-byte aligned
+        const Sum x0 = src[0], x1 = src[1], x2 = src[2], x3 = src[3];
+        src[0] = src[1] = src[2] = src[3] = Sum(0);
+        float4 o = make_float4(unfix(x0), unfix(x1), unfix(x2), unfix(x3));
+        if (CIC && base && it < OWN) {
+          const float4 m = *reinterpret_cast<const float4*>(base + (dst - mesh));
           o = make_float4(m.x + o.x, m.y + o.y, m.z + o.z, m.w + o.w);
         }
         *reinterpret_cast<float4*>(dst) = o;
@@ -390,7 +385,7 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
     } else {
       const int own = B.b0 * B.b1 * B.b2, xp = B.t1() * B.b2, yp = B.b0 * B.b2;
       for (int i = threadIdx.x; i < own + xp + yp; i += NT) {
-        unsigned long long* src;
+        Sum* src;
         float* dst;
         if (i < own) {
           int r = i / B.b2, z = i - r * B.b2;
@@ -407,9 +402,9 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_scatter_column
           src = &tile[B.cell(r, B.b1, z)];
         }
         float o = unfix(*src);
-        if (CIC && opt.base && i < own) o = opt.base[dst - mesh] + o;
+        if (CIC && base && i < own) o = base[dst - mesh] + o;
         *dst = o;
-        *src = 0ull;
+        *src = Sum(0);
       }
     }
     __syncthreads();
@@ -1116,15 +1111,15 @@ int effective_desc(const pm_gravity_desc* d, int64_t n, pm_gravity_desc* out) {
 // <= 1; then, with fold, the neighbouring columns' upper x/y planes (otherwise the R2C pass that
 // reads the mesh adds them: fold_planes).
 int scatter_planes(const Bricks& k, const sort::Sorted& srt, float value, float* mesh, float* xs, float* ys,
-                   const float* vals, const float* vscale, const ScatterOpt& opt, bool fold, hipStream_t s) {
+                   const float* vals, const float* vscale, bool cic, const float* base, bool fold, hipStream_t s) {
   const Walk w = column_walk(k);
   auto launch = [&](auto kern, int threads) {
     hipLaunchKernelGGL(kern, w.grid, dim3(threads), 0, s, srt.rec, srt.bins, value, k, w.run, mesh, xs, ys, vals,
-                       vscale, opt);
+                       vscale, base);
   };
-  if (opt.cic && is_brick(k, 16, 16, 32))
+  if (cic && is_brick(k, 16, 16, 32))
     launch(k_scatter_columns<16, 16, 32, true>, BrickShape<16, 16, 32>::NT);
-  else if (opt.cic)  // cic_plan takes no other bricks
+  else if (cic)  // cic_plan takes no other bricks
     launch(k_scatter_columns<8, 8, 16, true>, BrickShape<8, 8, 16>::NT);
   else if (is_brick(k, 16, 16, 32))
     launch(k_scatter_columns<16, 16, 32, false>, BrickShape<16, 16, 32>::NT);
@@ -1144,7 +1139,7 @@ int scatter_planes(const Bricks& k, const sort::Sorted& srt, float value, float*
 int scatter_tiled(const pm_gravity_desc* d, const Buffers& b, float* mesh, const float* vals, const float* vscale,
                   bool fold, hipStream_t s) {
   return scatter_planes(make_bricks(d->mesh_shape, d->brick), b.srt, d->particle_value, mesh, b.xs, b.ys, vals, vscale,
-                        ScatterOpt(), fold, s);
+                        false, nullptr, fold, s);
 }
 
 // The plane buffers of an unfolded tiled scatter, for the R2C pass (mesh and brick extents are
@@ -1475,79 +1470,23 @@ int prepare(const pm_gravity_desc* d, int64_t n, void* workspace, size_t workspa
 // ---------------------------------------------------------------- tiled CIC seam ----
 // The scatter and the gather adjoint of the kernel seam (pm_cic.hip) through the force step's
 // binning and column kernels, for one-channel meshes without offset, drops or a cell size of their
-// own.  Float atomics run at 27 G/s here (128^3 particles on a 256^3 mesh: 546 us with the mesh's
-// zeros); binning the particles (50 us), their values (16 us) and adding each brick up in LDS (36 us)
-// take 118 us.
+// own.  Float atomics run at 23-27 G/s here (128^3 displaced particles onto a 256^3 mesh: 744 us with
+// the copy of the mesh); binning the particles (56 us), ordering their values (10), adding each brick up
+// in LDS (36) and the column planes (11) take 122 us.
 //
-// Precision: values are scaled by a power of two and counted in units of 1 / fix of the largest, with
-// as many bits as the fullest bin lets a 64-bit sum have (2 max_bin deposits per cell; 51 bits at 1024
-// particles in a bin).  Values too small to keep their 24 bits there are left out and go through the float
-// atomics afterwards, and so does everything when a value or a position is not finite or the
-// values are beyond what the output factor holds.  The sums are exact and rounded once, where
-// float atomics round at every addition.
-constexpr int kCicBlocks = 1024;
-
-// Values in sorted order, and per block: their largest magnitude (infinite when a value or a position is
-// not finite) and the fullest bin.  vals null: ones.
-__global__ void __launch_bounds__(kBlock) k_cic_values(const float4* __restrict__ rec, const int32_t* __restrict__ perm,
+// Precision: a deposit is the float32 product v W of the atomics' kernel, and a cell's deposits are added in
+// float64 and rounded once per column that touches it, where float atomics round at every addition; so the
+// range of the values, zeros, infinities and NaN need no rule.  (Fixed point in units of the largest
+// value, tried first, cost the cells far below it their bits: one value 2^16 times the others left 1.2e-4
+// rms in the cells without it.)
+//
+// The values in sorted order.
+__global__ void __launch_bounds__(kBlock) k_cic_values(const int32_t* __restrict__ perm,
                                                        const int32_t* __restrict__ bins, int nbins,
-                                                       const float* __restrict__ val, float* __restrict__ val_s,
-                                                       float* __restrict__ part) {
-  const int64_t n = bins[nbins];
-  const int64_t t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x, step = (int64_t)gridDim.x * kBlock;
-  float mx = 0.f, mb = 0.f;  // counts up to 2^31, rounded: a bit more or less is spared below
-  for (int64_t j = t0; j < n; j += step) {
-    const float4 r = rec[j];
-    float v = 1.f;
-    if (val) {
-      v = val[perm[j]];
-      val_s[j] = v;
-    }
-    if (!isfinite(v) || !isfinite(r.x + r.y + r.z)) mx = INFINITY;
-    mx = fmaxf(mx, fabsf(v));
-  }
-  for (int64_t b = t0; b < nbins; b += step) mb = fmaxf(mb, (float)(bins[b + 1] - bins[b]));
-  for (int off = 32; off > 0; off >>= 1) {
-    mx = fmaxf(mx, __shfl_xor(mx, off));
-    mb = fmaxf(mb, __shfl_xor(mb, off));
-  }
-  __shared__ float sm[2][kBlock / 64];
-  if ((threadIdx.x & 63) == 0) {
-    sm[0][threadIdx.x / 64] = mx;
-    sm[1][threadIdx.x / 64] = mb;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / 64; ++w) {
-      mx = fmaxf(mx, sm[0][w]);
-      mb = fmaxf(mb, sm[1][w]);
-    }
-    part[blockIdx.x] = mx;
-    part[kCicBlocks + blockIdx.x] = mb;
-  }
-}
-
-// |value| < 1 after vs, at most 2 max_bin of them in a tile cell (a bin and the one below it): with
-// fix = 2^(60 - ceil(log2 max_bin)) the sums stay below 2^62.
-__global__ void k_cic_scale(const float* __restrict__ part, int nb, float factor, CicScale* __restrict__ out) {
-  float mx = 0.f, mb = 0.f;
-  for (int i = threadIdx.x; i < nb; i += 64) {  // one wave
-    mx = fmaxf(mx, part[i]);
-    mb = fmaxf(mb, part[kCicBlocks + i]);
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    mx = fmaxf(mx, __shfl_xor(mx, off));
-    mb = fmaxf(mb, __shfl_xor(mb, off));
-  }
-  if (threadIdx.x != 0) return;
-  const int bits = 60 - (ilogbf(fmaxf(mb, 1.f)) + 1);
-  const float f = fabsf(factor);
-  // the output factor 2^-bits / vs (times the scalar) must be a normal number, and so must vs
-  const bool ok = (mx == 0.f || (mx <= 0x1p100f && mx >= 0x1p-60f)) && f <= 0x1p100f && f >= 0x1p-60f;
-  const int e = ok && mx > 0.f ? ilogbf(mx) + 1 : 0;  // mx < 2^e
-  out->vs = ldexpf(1.f, -e);
-  out->fix = ldexpf(1.f, bits);
-  out->tiny = ok ? ldexpf(1.f, e + 24 - bits) : NAN;
+                                                       const float* __restrict__ val, float* __restrict__ val_s) {
+  const int64_t n = bins[nbins];  // the valid ones
+  for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < n; j += (int64_t)gridDim.x * kBlock)
+    val_s[j] = val[perm[j]];
 }
 
 struct CicPlan {
@@ -1558,9 +1497,9 @@ struct CicPlan {
 
 // Whether a call takes the tiled path: one channel, no offset, the particles' own cell size, the whole
 // periodic mesh, axes in whole bricks, enough particles for the launches and enough per cell for the
-// passes over the mesh.  Atomics / tiled, us, of 64^3 particles on meshes of 64^3: 59 / 56,
-// 128^3: 73 / 51, 256^3: 96 / 69, 384^3: 123 / 142, 512^3: 193 / 271; 96^3 on 512^3: 397 / 308;
-// 128^3 on 128^3: 454 / 110.
+// passes over the mesh.  Atomics / tiled, us, of 64^3 particles with normal displacements of 1.5 cells, onto
+// meshes of 64^3: 87 / 48, 128^3: 97 / 39, 256^3: 122 / 61, 384^3: 195 / 207, 512^3: 339 / 340; 96^3 on
+// 512^3: 551 / 358; 128^3 on 128^3: 704 / 97.
 constexpr int64_t kCicTiled = int64_t(1) << 18;
 constexpr int64_t kCicSparse = 128;
 bool cic_plan(const pm_cic_geom* g, int64_t n, int32_t channels, CicPlan* p) {
@@ -1584,8 +1523,7 @@ bool cic_plan(const pm_cic_geom* g, int64_t n, int32_t channels, CicPlan* p) {
 struct CicBuffers {
   sort::Sorted srt;
   int32_t *count, *partial;
-  float *xs, *ys, *val_s, *part;
-  CicScale* scale;
+  float *xs, *ys, *val_s;
 };
 
 bool cic_carve(Arena& ws, const pm_cic_geom* g, const CicPlan& p, int64_t n, CicBuffers& b) {
@@ -1598,8 +1536,6 @@ bool cic_carve(Arena& ws, const pm_cic_geom* g, const CicPlan& p, int64_t n, Cic
   b.xs = ws.take<float>(xs_floats(p.k));
   b.ys = ws.take<float>(ys_floats(p.k));
   b.val_s = ws.take<float>(n);
-  b.part = ws.take<float>(2 * kCicBlocks);
-  b.scale = ws.take<CicScale>(1);
   return ws.ok();
 }
 
@@ -1610,7 +1546,7 @@ size_t cic_bytes(const pm_cic_geom* g, const CicPlan& p, int64_t n) {
   return probe.used + 256;
 }
 
-// out = base + sum val W through the tiles, then the atomics for what they left out.
+// out = base + sum val W (val null: val_scalar) through the tiles.
 int cic_scatter_tiled(const int16_t* pmid, const float* disp, const uint8_t* valid, const float* val, float val_scalar,
                       int64_t n, const pm_cic_geom* g, const CicPlan& p, const float* base, float* out, CicBuffers& b,
                       hipStream_t s) {
@@ -1619,19 +1555,13 @@ int cic_scatter_tiled(const int16_t* pmid, const float* disp, const uint8_t* val
   const int32_t grid[3] = {c, c, c};
   PM_TRY(sort::bucket_cells(pmid, disp, valid, n, g->local_shape, g->particle_cell, p.brick, grid, b.srt, b.count,
                             b.partial, false, s));
-  const int nbins = p.k.nb[0] * p.k.nb[1] * p.k.nb[2];
-  const unsigned nb = (unsigned)std::min<int64_t>(ceil_div(n, kBlock), kCicBlocks);
-  hipLaunchKernelGGL(k_cic_values, dim3(nb), dim3(kBlock), 0, s, b.srt.rec, b.srt.perm, b.srt.bins, nbins, val, b.val_s,
-                     b.part);
-  PM_LAUNCHED("k_cic_values", s);
-  hipLaunchKernelGGL(k_cic_scale, dim3(1), dim3(64), 0, s, b.part, (int)nb, val ? 1.f : val_scalar, b.scale);
-  PM_LAUNCHED("k_cic_scale", s);
-  ScatterOpt opt;
-  opt.cic = b.scale;
-  opt.scale = val ? 1.f : val_scalar;  // a scalar's deposits are counted as ones
-  opt.base = base;
-  PM_TRY(scatter_planes(p.k, b.srt, 1.f, out, b.xs, b.ys, val ? b.val_s : nullptr, nullptr, opt, true, s));
-  return cic_scatter_rest(pmid, disp, valid, val, val_scalar, n, g, out, &b.scale->tiny, s);
+  if (val) {
+    const int nbins = p.k.nb[0] * p.k.nb[1] * p.k.nb[2];
+    const unsigned nb = (unsigned)std::min<int64_t>(ceil_div(n, kBlock), 1024);
+    hipLaunchKernelGGL(k_cic_values, dim3(nb), dim3(kBlock), 0, s, b.srt.perm, b.srt.bins, nbins, val, b.val_s);
+    PM_LAUNCHED("k_cic_values", s);
+  }
+  return scatter_planes(p.k, b.srt, val_scalar, out, b.xs, b.ys, val ? b.val_s : nullptr, nullptr, true, base, true, s);
 }
 
 }  // namespace

@@ -230,3 +230,39 @@ def test_tiled_path_refuses_and_falls_back(device):
             assert torch.equal(s, M)
         else:
             assert not torch.isnan(s).any() and float(s.max()) > 1e29
+
+
+@pytest.mark.parametrize("mesh_shape", [(128, 128, 128), (256, 128, 128)])  # small and large bricks
+@pytest.mark.parametrize("outlier", [1.0, 2.0 ** 16, 2.0 ** 24, 2.0 ** 100])
+def test_tiled_deposits_keep_their_own_precision(device, mesh_shape, outlier):
+    """Every cell as good as the deposits in it, whatever the other values and however small its
+    weights: against the float64 sum of the float32 deposits v W, to the roundings of the stored
+    sum and of the three column planes a cell may get, 2^-24 of the sum of |v W| each."""
+    rng = np.random.default_rng(int(np.log2(outlier)) + mesh_shape[0])
+    n = 1 << 18
+    pmid = np.stack(np.meshgrid(*[np.arange(0, m, 2) for m in mesh_shape], indexing="ij"), -1).reshape(-1, 3)
+    pmid = pmid[rng.permutation(len(pmid))[:n]].astype(np.int16)
+    disp = (0.05 * rng.normal(size=(n, 3))).astype(np.float32)
+    val = (rng.choice([-1.0, 1.0], n) * rng.uniform(0.5, 1.0, n)).astype(np.float32)
+    val[n // 3] *= np.float32(outlier)
+    one = np.float32(1)
+    lo = np.floor(disp)
+    f = disp - lo
+    w = (one - np.abs(f), one - np.abs(f - one))
+    ref, absum = np.zeros(mesh_shape), np.zeros(mesh_shape)
+    for c in range(8):
+        b = [(c >> a) & 1 for a in range(3)]
+        dep = val * (w[b[0]][:, 0] * w[b[1]][:, 1] * w[b[2]][:, 2])
+        assert dep.dtype == np.float32
+        ix = tuple((pmid[:, a] + lo[:, a].astype(np.int64) + b[a]) % mesh_shape[a] for a in range(3))
+        np.add.at(ref, ix, dep.astype(np.float64))
+        np.add.at(absum, ix, np.abs(dep).astype(np.float64))
+    bound = 4 * 2.0 ** -24 * absum + 1e-44  # and of subnormal sums
+    P, D, V = _t(pmid, device, torch.int16), _t(disp, device), _t(val, device)
+    kw = dict(offset=0.0, particle_cell_size=1.0, global_shape=mesh_shape)
+    M = torch.zeros(mesh_shape, device=device)
+    for got in (hip_scatter(P, D, V, M, **kw), hip_gather_bwd(P, D, M, V, **kw)[1]):
+        assert np.all(np.abs(_np(got) - ref) <= bound)
+    if outlier == 1.0:
+        s = _np(hip_scatter(P, D, float(val[0]), M, **kw))
+        assert np.all(s[absum == 0] == 0) and s.sum() == pytest.approx(n * float(val[0]), rel=1e-6)
