@@ -72,9 +72,10 @@ class Particles:
             dp_t = torch.empty((n, 3), dtype=torch.float32, device=dev)
             v = torch.empty_like(dp_t) if vel else None
             g1, g2, *factors = lpt if lpt is not None else (None, None, 0.0, 0.0, 0.0, 0.0)
-            _lib.call("pm_ic_lpt_particles", _lib.int3(conf.ptcl_grid_shape), _lib.int3(conf.mesh_shape),
-                      float(conf.cell_size), ptr(g1), ptr(g2), *factors, ptr(pm_t), ptr(dp_t), ptr(v),
-                      stream_handle(dev))
+            with torch.cuda.device(dev):  # a default stream's handle names the current device's
+                _lib.call("pm_ic_lpt_particles", _lib.int3(conf.ptcl_grid_shape), _lib.int3(conf.mesh_shape),
+                          float(conf.cell_size), ptr(g1), ptr(g2), *factors, ptr(pm_t), ptr(dp_t), ptr(v),
+                          stream_handle(dev))
             unused = torch.zeros(n, dtype=torch.bool, device=dev)
             return cls(conf, pm_t, dp_t, vel=v, acc=torch.zeros_like(dp_t) if acc else None, unused_index=unused)
         pmid, disp = [], []

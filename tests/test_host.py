@@ -192,3 +192,33 @@ def test_lazy_views_are_written_out_for_the_kernels(monkeypatch):
         raw = ctypes.string_at(got.data_ptr(), got.numel() * got.element_size())
         assert raw == want.numpy().tobytes()
     assert _torch.as_contig(z, torch.complex64, "z") is z  # nothing to do: no copy
+
+
+def test_the_particle_grid_is_made_on_the_device_it_is_asked_for(monkeypatch):
+    # a default stream's handle is 0 on every device, so the launch goes to the current one
+    import torch
+
+    from pmpp_amd import Particles, _lib, _torch
+
+    current, launched = ["cuda:0"], []
+
+    class Device:
+        def __init__(self, dev):
+            self.dev = str(dev)
+
+        def __enter__(self):
+            current.append(self.dev)
+
+        def __exit__(self, *exc):
+            current.pop()
+
+    def on_cpu(f):
+        return lambda *a, device=None, **kw: f(*a, **kw)
+
+    for name in ("empty", "zeros"):
+        monkeypatch.setattr(torch, name, on_cpu(getattr(torch, name)))
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(_torch, "stream_handle", lambda dev: None)
+    monkeypatch.setattr(_lib, "call", lambda name, *a: launched.append((name, current[-1])))
+    p = Particles.gen_grid(Configuration(1.0, (4, 4, 4)), vel=True, device="cuda:1")
+    assert len(p) == 64 and launched == [("pm_ic_lpt_particles", "cuda:1")] and current == ["cuda:0"]
