@@ -146,9 +146,10 @@ __global__ void __launch_bounds__(kBlock) k_lpt2_source(const float* __restrict_
 
 // Particles on the Lagrangian grid (g0, g1, g2) of a mesh (m0, m1, m2): per axis the anchor rint(i
 // (m / g)) and what is left of the position as a displacement (i m - anchor g) (cell / g), both in
-// float64 as the host would form them; to it the LPT terms D1 grad1 + D2 grad2 (component-major
-// meshes on the grid; null: none), and the velocities V1 grad1 + V2 grad2.  Bound by HBM (18
-// bytes written per particle, with LPT 30, and 24 read); four particles per thread, whole vectors.
+// float64 as the host would form them (an anchor past int16 wraps as there); to it the LPT terms D1
+// grad1 + D2 grad2 (component-major meshes on the grid; null: none), and the velocities V1 grad1 + V2
+// grad2.  Bound by HBM (18 bytes written per particle, with LPT 30, and 24 read); four particles per
+// thread, whole vectors.
 struct LatticeAxes {
   int g[3], m[3];
   double step[3], left[3];  // m / g, cell / g
@@ -195,7 +196,7 @@ __global__ void __launch_bounds__(kBlock) k_lpt_particles(LatticeAxes ax, const 
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
         const int anchor = (int)rint((double)idx[a] * ax.step[a]);
-        const int left = idx[a] * ax.m[a] - anchor * ax.g[a];
+        const int64_t left = (int64_t)idx[a] * ax.m[a] - (int64_t)anchor * ax.g[a];
         float x = (float)((double)left * ax.left[a]), u = 0.f;
         if (grad1) {
           x += D1 * ga[a][e];
@@ -373,8 +374,8 @@ int pm_ic_lpt_particles(const int32_t grid[3], const int32_t mesh[3], double cel
   ic::LatticeAxes ax;
   int64_t n = 1;
   for (int a = 0; a < 3; ++a) {
-    PM_RETURN_IF(grid[a] < 1 || mesh[a] < grid[a] || mesh[a] > 32767, PM_ERROR_INVALID_ARGUMENT,
-                 "the mesh must be at least the particle grid and its cells fit int16");
+    PM_RETURN_IF(grid[a] < 1 || mesh[a] < grid[a], PM_ERROR_INVALID_ARGUMENT,
+                 "the mesh must be at least the particle grid");
     ax.g[a] = grid[a];
     ax.m[a] = mesh[a];
     ax.step[a] = (double)mesh[a] / (double)grid[a];

@@ -229,6 +229,15 @@ def test_particle_lattice_on_the_device_equals_the_host_one(device, grid, mesh, 
         assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
 
 
+@pytest.mark.parametrize("grid,ratio", [((4, 2, 2), 16384), ((2, 4, 8), 8192), ((6, 9, 3), 40000)])
+def test_particle_lattice_of_meshes_at_and_past_int16(device, grid, ratio):
+    """Axes of 32768 cells (whose last anchors still fit int16) and longer ones (whose anchors wrap, as
+    the host's do; past 2^31 for the product of an index and the axis): the host's values."""
+    conf = Configuration(1.0, grid, mesh_shape=ratio)
+    a, b = (Particles.gen_grid(conf, device=d) for d in (device, "cpu"))
+    assert torch.equal(a.pmid.cpu(), b.pmid) and torch.equal(a.disp.cpu(), b.disp)
+
+
 @pytest.mark.parametrize("grid", [(2, 2, 2), (8, 8, 8), (64, 4, 16), (4, 128, 32), (32, 16, 256), (512, 4, 4)])
 def test_symbol_inverses_match_multiply_then_transform(device, grid):
     """The three strains, cross strains and gradient components of one call against the symbol
