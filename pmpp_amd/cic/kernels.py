@@ -68,6 +68,17 @@ def _is_scalar(val):
     return not isinstance(val, torch.Tensor) or val.ndim == 0
 
 
+def _tiled_workspace(nbytes, device):
+    """The workspace of a tiled call, or None for a call that is not one (0 bytes) or where it does not fit
+    (about 40 bytes per particle): the plain entry points need none."""
+    if not nbytes:
+        return None
+    try:
+        return workspace(nbytes, device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def hip_scatter(pmid, disp, val, mesh, *, offset, particle_cell_size, cell_size=None, global_shape,
                 valid_mask=None):
     """mesh + sum_p val_p W_p (returns a new mesh)."""
@@ -89,21 +100,20 @@ def hip_scatter(pmid, disp, val, mesh, *, offset, particle_cell_size, cell_size=
     g = _geom(mesh.shape[:3], global_shape, offset, particle_cell_size, cell_size)
     base = as_contig(mesh, torch.float32, "mesh")
     nbytes = 0 if base.data_ptr() % 16 else _lib.size_query("pm_cic_tiled_workspace", n, C, g)
-    if nbytes:
-        return _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, nbytes)
-    out = base.clone()
+    out = torch.empty_like(base)
+    ws = _tiled_workspace(nbytes, mesh.device)
+    if ws is not None:
+        return _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, out, ws)
+    out.copy_(base)
     _lib.call("pm_cic_scatter", ptr(pm), ptr(dp), ptr(valid), ptr(vt), vs, n, C, g, ptr(out),
               stream_handle(mesh.device))
     return out
 
 
-def _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, nbytes):
-    """base (None: 0) + sum val W through ``pm_cic_scatter_tiled``, on checked arguments."""
-    dev = dp.device
-    out = torch.empty(tuple(g.local_shape) if base is None else base.shape, dtype=torch.float32, device=dev)
-    ws = workspace(nbytes, dev)
+def _scatter_tiled(pm, dp, valid, vt, vs, n, g, base, out, ws):
+    """out = base (None: 0) + sum val W through ``pm_cic_scatter_tiled``, on checked arguments."""
     _lib.call("pm_cic_scatter_tiled", ptr(pm), ptr(dp), ptr(valid), ptr(vt), vs, n, g, ptr(base), ptr(out), ptr(ws),
-              nbytes, stream_handle(dev))
+              ws.numel(), stream_handle(dp.device))
     return out
 
 
@@ -116,10 +126,14 @@ def hip_scatter_new(pmid, disp, val, shape, *, offset, particle_cell_size, cell_
         g = _geom(shape, global_shape, offset, particle_cell_size, cell_size)
         nbytes = _lib.size_query("pm_cic_tiled_workspace", n, 1, g)
         if nbytes and (_is_scalar(val) or tuple(val.shape) == (n,)):
-            vt = None if _is_scalar(val) else as_contig(val, torch.float32, "val")
-            return _scatter_tiled(as_contig(pmid, torch.int16, "pmid"), as_contig(disp, torch.float32, "disp"),
-                                  _valid(valid_mask, n, disp.device), vt, float(val) if vt is None else 0.0, n, g, None,
-                                  nbytes)
+            out = torch.empty(tuple(shape), dtype=torch.float32, device=disp.device)
+            ws = _tiled_workspace(nbytes, disp.device)
+            if ws is not None:
+                vt = None if _is_scalar(val) else as_contig(val, torch.float32, "val")
+                return _scatter_tiled(as_contig(pmid, torch.int16, "pmid"), as_contig(disp, torch.float32, "disp"),
+                                      _valid(valid_mask, n, disp.device), vt, float(val) if vt is None else 0.0, n, g,
+                                      None, out, ws)
+            del out
     mesh = torch.zeros(tuple(shape), dtype=torch.float32, device=disp.device)
     return hip_scatter(pmid, disp, val, mesh, offset=offset, particle_cell_size=particle_cell_size,
                        cell_size=cell_size, global_shape=global_shape, valid_mask=valid_mask)
@@ -160,13 +174,13 @@ def hip_gather_bwd(pmid, disp, mesh, val_cot, *, offset, particle_cell_size, cel
     valid = _valid(valid_mask, n, mesh.device)
     g = _geom(mesh.shape[:3], global_shape, offset, particle_cell_size, cell_size)
     nbytes = 0 if m.data_ptr() % 16 or vc.numel() != n else _lib.size_query("pm_cic_tiled_workspace", n, C, g)
-    if nbytes:
-        mesh_cot = torch.empty_like(m)
-        ws = workspace(nbytes, mesh.device)
+    mesh_cot = torch.empty_like(m)
+    ws = _tiled_workspace(nbytes, mesh.device)
+    if ws is not None:
         _lib.call("pm_cic_gather_bwd_tiled", ptr(pm), ptr(dp), ptr(valid), n, g, ptr(m), ptr(vc), ptr(disp_cot),
-                  ptr(mesh_cot), ptr(ws), nbytes, stream_handle(mesh.device))
+                  ptr(mesh_cot), ptr(ws), ws.numel(), stream_handle(mesh.device))
         return disp_cot, mesh_cot
-    mesh_cot = torch.zeros_like(m)
+    mesh_cot.zero_()
     _lib.call("pm_cic_gather_bwd", ptr(pm), ptr(dp), ptr(valid), n, C, g, ptr(m), ptr(vc), ptr(disp_cot),
               ptr(mesh_cot), stream_handle(mesh.device))
     return disp_cot, mesh_cot

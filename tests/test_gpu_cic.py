@@ -266,3 +266,27 @@ def test_tiled_deposits_keep_their_own_precision(device, mesh_shape, outlier):
     if outlier == 1.0:
         s = _np(hip_scatter(P, D, float(val[0]), M, **kw))
         assert np.all(s[absum == 0] == 0) and s.sum() == pytest.approx(n * float(val[0]), rel=1e-6)
+
+
+def test_calls_whose_tiled_workspace_does_not_fit_take_the_atomics(device, monkeypatch):
+    from pmpp_amd.cic import kernels
+
+    shape, n = (64, 32, 32), 1 << 18
+    rng = np.random.default_rng(7)
+    P = _t(rng.integers(0, 32, (n, 3)), device, torch.int16)
+    D, V, M = (_t(rng.uniform(0.25, 0.75, s), device) for s in ((n, 3), (n,), shape))
+    kw = dict(offset=0.0, particle_cell_size=1.0, global_shape=shape)
+
+    def outputs():
+        return (hip_scatter(P, D, V, M, **kw), kernels.hip_scatter_new(P, D, V, shape, **kw),
+                kernels.hip_scatter_new(P, D, 0.5, shape, **kw), *hip_gather_bwd(P, D, M, V, **kw))
+
+    tiled = outputs()
+
+    def full(nbytes, dev):
+        raise torch.cuda.OutOfMemoryError("no room for %d bytes" % nbytes)
+
+    monkeypatch.setattr(kernels, "workspace", full)
+    for a, b in zip(outputs(), tiled):
+        # up to about 100 float32 additions of positive values in another order
+        assert torch.allclose(a, b, rtol=100 * 2.0 ** -24, atol=1e-6)
