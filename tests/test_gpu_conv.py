@@ -199,3 +199,30 @@ def test_weight_gradient_tile_edges(device, cin, one, shape):
     uz.copy_(src)
     dw2, db2 = conv3d_bwd_weight(uz, ux)
     assert torch.equal(dw2, dw) and torch.equal(db2, db)
+
+
+def test_weight_gradient_error_on_a_large_mesh(device):
+    """The float32 sums of 256^3 voxels (65536 per workgroup) against 64 bits, rms over the weights
+    of three taps.  A rounding of a sum of k of K zero-mean terms adds 2^-24 / sqrt(3) sqrt(k / K) of
+    the whole sum's size: over the L = 128 steps of 32 products that an accumulator takes, at most
+    eight roundings each, sqrt(8 * 128 / 2) 2^-24 / sqrt(3) = 7.8e-7 of its sum, so also of the sum of
+    independent accumulators; the few sums after them (8 per wave, 2 waves, 16 + 16 rows) sqrt(42 / 2)
+    2^-24 / sqrt(3) = 1.6e-7."""
+    shape, cin = (256, 256, 256), 8
+    g = torch.Generator(device=device).manual_seed(5)
+    dz = torch.randn(shape + (16,), device=device, generator=g)
+    x = torch.randn(shape + (cin,), device=device, generator=g).to(torch.bfloat16)
+    dw, _ = conv3d_bwd_weight(dz, x)
+    dzb = dz.to(torch.bfloat16)
+    del dz
+    err = ref = 0.0
+    for tap in (0, 13, 26):
+        off = tuple(1 - o for o in (tap // 9, tap // 3 % 3, tap % 3))
+        xs = torch.roll(x, off, (0, 1, 2))
+        e = torch.zeros(16, cin, dtype=torch.float64, device=device)
+        for i in range(0, 256, 32):
+            a = dzb[i:i + 32].double().reshape(2048, -1, 16).transpose(1, 2).contiguous()
+            e += (a @ xs[i:i + 32].double().reshape(2048, -1, cin)).sum(0)
+        err += float((dw[tap].double() - e).square().sum())
+        ref += float(e.square().sum())
+    assert (err / ref) ** 0.5 < 8e-7
