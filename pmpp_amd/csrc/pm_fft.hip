@@ -80,7 +80,7 @@ struct ColCfg {
 
 // Column tiles are visited in an XCD-aware order: workgroups are dispatched round-robin
 // over the 8 XCDs, so logical item q is given to workgroup (q % g8) * 8 + q / g8 ... i.e.
-// consecutive logical items (the two halves of a tile, and neighbouring tiles, which share
+// consecutive logical items (the workgroups of a tile, and neighbouring tiles, which share
 // cache lines when T*8 < 128 bytes) run on the same XCD at nearly the same time.
 template <int N, int T, int MODE, int HALVES>
 __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
@@ -118,6 +118,7 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
   float* my = lds;
   auto idx = [&](int row) { return row * T + col + (row / N2) * CF::PADK; };
 
+  static_assert((HALVES == 3) == (MODE == kColInv3 || MODE == kColSym), "three workgroups per tile: one per output");
   float2 v[E];
   if constexpr (MODE == kColAdj) {
     // Spectral adjoint of the force step, x pass (the columns are kz, the batches the packed ky
@@ -192,8 +193,8 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
     return;
   } else {
     if constexpr (MODE == kColGreen || MODE == kColPot) {
-      // mask x Poisson symbol (gravity.py:174-196, 263-287); kColGreen's second half also
-      // applies D_x = i*negk_x (configuration.py:365-376), kColPot has one half (the potential)
+      // mask x Poisson symbol (gravity.py:174-196, 263-287); for kColGreen's second output also
+      // D_x = i*negk_x (configuration.py:365-376), below
       int ky = (int)(b * io.ky_b) + cgl * io.ky_c;
       ky += ky > io.ky_split ? io.ky_shift : 0;
       int kz = (int)(b * io.kz_b) + cgl * io.kz_c + io.kz0;
@@ -209,10 +210,9 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
         bool keep = keep_yz && spec_keep(kxv, tb) && k2 != 0.f;
         const float r = recip_nr(k2);
         float g = keep ? -r : 0.f;  // one reciprocal per mode, shared by both parts
-        float2 phi = make_float2(v[s].x * g, v[s].y * g);
-        v[s] = (half == 1) ? c_imul(spec_negk(kxv, tb), phi) : phi;
+        v[s] = make_float2(v[s].x * g, v[s].y * g);
       }
-      if constexpr (MODE == kColGreen && HALVES == 1) {
+      if constexpr (MODE == kColGreen) {
         // one workgroup per tile: the multiplied spectrum phi is parked in out0 at this
         // thread's own output rows (where it writes its out0 values at the end, so no other
         // thread touches them), D_x phi is inverted into out1, then phi is read back and
