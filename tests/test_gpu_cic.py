@@ -290,3 +290,35 @@ def test_calls_whose_tiled_workspace_does_not_fit_take_the_atomics(device, monke
     for a, b in zip(outputs(), tiled):
         # up to about 100 float32 additions of positive values in another order
         assert torch.allclose(a, b, rtol=100 * 2.0 ** -24, atol=1e-6)
+
+
+@pytest.mark.parametrize("n,invalid", [((1 << 19) + 3, 0.0), ((1 << 19) + 3, 0.2), ((1 << 21) + 5, 0.1)])
+def test_tiles_of_particles_in_no_grid_equal_the_plain_entry_points(device, n, invalid):
+    """Particle counts that are no cube at the second and the largest chunk of the binning (index
+    ranges), against the same float32 deposits added one by one with float atomics."""
+    from pmpp_amd import _lib
+    from pmpp_amd._torch import ptr, stream_handle
+    from pmpp_amd.cic.kernels import _geom
+
+    shape = (128, 144, 128)
+    g = torch.Generator(device=device).manual_seed(n)
+    P = torch.randint(0, 128, (n, 3), device=device, generator=g, dtype=torch.int16)
+    D = torch.randn((n, 3), device=device, generator=g)
+    V = torch.rand(n, device=device, generator=g) + 0.5
+    M = torch.rand(shape, device=device, generator=g)
+    ok = torch.rand(n, device=device, generator=g) >= invalid
+    geo = _geom(shape, shape, 0.0, 1.0, None)
+    assert _lib.size_query("pm_cic_tiled_workspace", n, 1, geo) > 0
+    kw = dict(offset=0.0, particle_cell_size=1.0, global_shape=shape, valid_mask=ok)
+    u8 = ok.to(torch.uint8)
+    s = stream_handle(device)
+    plain, mc, dc = M.clone(), torch.zeros_like(M), torch.empty_like(D)
+    _lib.call("pm_cic_scatter", ptr(P), ptr(D), ptr(u8), ptr(V), 0.0, n, 1, geo, ptr(plain), s)
+    _lib.call("pm_cic_gather_bwd", ptr(P), ptr(D), ptr(u8), n, 1, geo, ptr(M), ptr(V), ptr(dc), ptr(mc), s)
+    got = hip_scatter(P, D, V, M, **kw)
+    gdc, gmc = hip_gather_bwd(P, D, M, V, **kw)
+    # positive sums of up to about 100 deposits, one rounding each
+    assert torch.allclose(got, plain, rtol=100 * 2.0 ** -24, atol=0)
+    assert torch.allclose(gmc, mc, rtol=100 * 2.0 ** -24, atol=0)
+    # eight products of mesh values up to 1, weights of sum 4 and a cotangent up to 1.5, in another order
+    assert torch.allclose(gdc, dc, rtol=0, atol=32 * 1.5 * 2.0 ** -24)

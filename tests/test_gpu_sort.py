@@ -190,3 +190,53 @@ def test_bin_offsets_at_the_edges_of_the_scan(device, mesh):
     np.testing.assert_array_equal(key[perm], np.sort(key))
     assert np.array_equal(np.sort(perm), np.arange(n))
     np.testing.assert_array_equal(pm_s, pmid[perm])
+
+
+@pytest.mark.parametrize("grid,hint,valid_frac", [
+    ((130, 129, 128), False, None),  # level 2 (past 2^21 without a grid), index ranges
+    ((130, 129, 129), False, 0.7),   # the same with a ragged end and invalid particles
+    ((260, 256, 256), True, 0.98),   # level 2 (past 2^24 with a grid), blocks of the grid
+    ((128, 130, 40), True, None),    # level 1, a grid whose blocks leave 37 % of the slots empty: index ranges
+    ((128, 130, 60), False, 0.05),   # level 1, index ranges, many invalid particles
+])
+def test_bucketing_of_large_chunks_and_index_ranges(device, grid, hint, valid_frac):
+    mesh, brick, cell = tuple(2 * g for g in grid), (16, 16, 32), 0.5
+    rng = np.random.default_rng(sum(grid))
+    pm = np.stack(np.meshgrid(*[2 * np.arange(g, dtype=np.int16) for g in grid], indexing="ij"), -1).reshape(-1, 3)
+    n = len(pm)
+    disp = rng.normal(size=(n, 3), scale=0.8).astype(np.float32)
+    valid = None if valid_frac is None else rng.random(n) < valid_frac
+    perm, offs, pm_s, dp_s, v_s = hip_bucket(pm, disp, valid, mesh, cell, brick, grid if hint else None, device)
+    print(f"binned {n} particles", flush=True)
+    nb = [-(-m // b) for m, b in zip(mesh, brick)]
+    key = np.zeros(n, np.int64)
+    for a in range(3):
+        c = np.mod(pm[:, a].astype(np.int64) + np.floor(disp[:, a] / np.float32(cell)).astype(np.int64), mesh[a])
+        key = key * nb[a] + c // brick[a]
+    if valid is not None:
+        key = np.where(valid, key, int(np.prod(nb)))
+    count = np.bincount(key, minlength=int(np.prod(nb)) + 1)
+    np.testing.assert_array_equal(offs, np.concatenate([[0], np.cumsum(count)]))
+    assert np.array_equal(key[perm], np.repeat(np.arange(len(count)), count))
+    assert np.array_equal(np.bincount(perm, minlength=n), np.ones(n))
+    assert np.array_equal(pm_s, pm[perm]) and np.array_equal(dp_s.view(np.uint32), disp[perm].view(np.uint32))
+    assert np.array_equal(v_s, np.ones(n) if valid is None else valid[perm])
+
+
+@pytest.mark.parametrize("mesh", [(262079, 1, 1), (64, 63, 65)])
+def test_bin_offsets_on_both_sides_of_the_single_launch_scan(device, mesh):
+    # 262,079 bins and 65 counters more are the 2^18 the single launch takes, 262,080 one too many
+    assert int(np.prod(mesh)) in (262079, 262080)
+    rng = np.random.default_rng(mesh[0])
+    n = 300007
+    disp = np.stack([rng.integers(0, m, n) for m in mesh], 1).astype(np.float32)  # whole cells
+    disp[: n // 8] = [m - 1 for m in mesh]
+    pmid = np.zeros((n, 3), np.int16)
+    valid = rng.random(n) < 0.9
+    perm, offs, _, dp_s, _ = hip_bucket(pmid, disp, valid, mesh, 1.0, (1, 1, 1), None, device)
+    c = disp.astype(np.int64)
+    key = np.where(valid, (c[:, 0] * mesh[1] + c[:, 1]) * mesh[2] + c[:, 2], int(np.prod(mesh)))
+    count = np.bincount(key, minlength=int(np.prod(mesh)) + 1)
+    np.testing.assert_array_equal(offs, np.concatenate([[0], np.cumsum(count)]))
+    np.testing.assert_array_equal(key[perm], np.sort(key))
+    assert np.array_equal(np.sort(perm), np.arange(n)) and np.array_equal(dp_s, disp[perm])
