@@ -61,7 +61,8 @@ typedef struct pm_cic_geom {
  *   mask_active     1 when conf.mesh_shape != conf.ptcl_grid_shape (utils.py:31-32)
  *   omega_m         cosmo.Omega_m (cast to float32 as at gravity.py:630)
  *   particle_value  conf.mesh_size / conf.ptcl_num       (cic/scatter.py:258-265)
- *   brick           cell-sort granularity (cells per brick along each axis) */
+ *   brick           cell-sort granularity (cells per brick along each axis); on meshes of up to 2^21
+ *                   cells the force step cuts bricks that (8, 8, 16) divides into those */
 typedef struct pm_gravity_desc {
   int32_t mesh_shape[3];
   float cell_size;

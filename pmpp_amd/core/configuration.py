@@ -34,7 +34,8 @@ class Configuration:
     a_custom: Optional[Tuple[float, ...]] = None
     symp_splits: Tuple[Tuple[float, float], ...] = ((0, 0.5), (1, 0.5))
     lpt_order: int = 2
-    # cell-sort / CIC-tile granularity (cells per brick along each axis); None: (16, 16, 32)
+    # cell-sort / CIC-tile granularity (cells per brick along each axis); None: (16, 16, 32).  The force
+    # step cuts bricks that (8, 8, 16) divides into those on meshes of up to 2^21 cells
     brick: Optional[Tuple[int, int, int]] = None
     # the PM step is float32 with int16 anchors, as PM++'s defaults (configuration.py:183-185)
     float_dtype: str = "float32"

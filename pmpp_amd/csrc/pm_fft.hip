@@ -280,13 +280,18 @@ __global__ void __launch_bounds__((ColCfg<N, T, HALVES>::THREADS))
 // pairing it took 5.2; now 4.6.  A pair's threads are in one wave, so nothing waits at a barrier.
 // Before -> now, us: c2r 256^3 116 -> 88, 512^3 783 -> 594, 1024^3 5220 -> 4600; r2c with planes
 // 43 -> 33, 256 -> 231, 2050 -> 1450.  Now bound by the memory path (c2r 19.3 GB: 4.2 TB/s; a copy
-// reaches 4.8).
+// reaches 4.8).  A line's rounding goes with the larger of its pair: rms error of a forward or
+// inverse transform of white noise against 64 bits, before -> now, 64^3 1.50e-7 -> 1.49e-7, 256^3 1.86e-7 ->
+// 1.89e-7, 512^3 2.07e-7 -> 2.11e-7; on the smaller half of a log-normal field's cells, of their rms, 256^3
+// 8.9e-6 and 512^3 1.2e-5 either way.
 template <int N>
 struct ZCfg {
   static constexpr int P = Plan<N>::P;
   // long lines: more of them per workgroup, so more adjacent rows are written at about the same time
   // (1024^3, 64 / 128 / 256 / 512 threads: c2r 4.99 / 4.98 / 4.49 / 4.60, r2c 1.70 / 1.65 / 1.62 / 1.45 ms;
-  // 512^3, 256 / 512: 594 / 606, 232 / 238 us)
+  // 512^3, 256 / 512: 594 / 606, 232 / 238 us).  At 2048 points, whose threads hold 64 slots, 512 only helps
+  // the r2c of many lines (256 / 512: 64^2 lines c2r 25 / 29, r2c 22 / 26 us; 256^2 311 / 316, 258 / 274; 512^2
+  // 1077 / 1138, 945 / 878)
   static constexpr int THREADS = N == 1024 ? 512 : 256;
   static constexpr int PAIRS = THREADS / P;
   // floats per pair's slot (the transform's real / imaginary exchange), with LSTR = P (mod 64) so the
