@@ -748,8 +748,13 @@ int rfft3d_pitched(const float* in, float2* spec, const int32_t* shape, int64_t 
   return launch_cols(nx, kColFwd, cx, ny, tb, 0, s);
 }
 
-// Row pitch of a scratch half spectrum: rows start on cache lines.
-int64_t scratch_pitch(const int32_t* shape) { return (int64_t)align_up((size_t)shape[2] / 2 + 1, 16); }
+// Row pitch of a scratch half spectrum: rows start on cache lines where they are several lines long.  Shorter
+// ones would only get longer: inverse transform with / without, us, 2048^2 x 2 522 / 210, 1024^2 x 8 94 / 72,
+// 512 x 256 x 64 57 / 50, 256^2 x 128 51 / 47, but 256^3 79 / 93, 512^3 898 / 1000, 256^2 x 2048 725 / 811.
+int64_t scratch_pitch(const int32_t* shape) {
+  const int64_t n = shape[2] / 2 + 1;
+  return shape[2] >= 256 ? (int64_t)align_up((size_t)n, 16) : n;
+}
 
 // The y and z passes of ncomp inverse transforms whose x inverses lie one after the other in
 // `spec` (pitched rows), into ncomp meshes one after the other (1/N normalised).

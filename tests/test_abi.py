@@ -81,3 +81,12 @@ def test_transforms_require_pm_init():
     st = lib.pm_rfft3d(dummy, ctypes.c_void_p(512), _lib.int3((8, 8, 8)), None, 0, None)
     assert st == _lib.PM_ERROR_INVALID_ARGUMENT
     assert b"pm_init" in lib.pm_last_error()
+
+
+def test_inverse_transform_scratch_stays_near_the_spectrum():
+    # rows are padded to cache lines only where that adds little: thin meshes kept up to 8 spectra
+    for shape in ((2048, 2048, 2), (1024, 512, 8), (64, 64, 64), (64, 64, 128), (64, 64, 256), (8, 8, 2048)):
+        spectrum = 8 * shape[0] * shape[1] * (shape[2] // 2 + 1)
+        need = _lib.size_query("pm_irfft3d_keep_workspace", _lib.int3(shape))
+        assert spectrum <= need <= 1.125 * spectrum, shape
+        assert _lib.size_query("pm_ic_symbol_inverse_workspace", _lib.int3(shape)) == 3 * need
