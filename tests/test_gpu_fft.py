@@ -96,3 +96,15 @@ def test_inverse_of_a_conjugate_view(device):
     assert lazy.is_conj()
     assert torch.equal(irfftn(lazy, s=shape), irfftn(lazy.resolve_conj().clone(), s=shape))
     assert not torch.equal(irfftn(lazy, s=shape), irfftn(X, s=shape))
+
+
+@pytest.mark.parametrize("shape", [(4, 2, 4), (32, 64, 4), (4, 2, 8), (32, 64, 8), (32, 64, 16)])
+def test_short_lines_at_any_alignment(device, shape):
+    # rows read as whole vectors, from a mesh that starts 4 bytes past an aligned address
+    n = int(np.prod(shape))
+    x = np.random.default_rng(n).normal(size=shape).astype(np.float32)
+    buf = torch.zeros(n + 1, device=device)
+    buf[1:] = torch.from_numpy(x).to(device).view(-1)
+    ref = np.fft.rfftn(x.astype(np.float64))
+    for t in (buf[1:].view(shape), torch.from_numpy(x).to(device)):
+        assert np.abs(rfftn(t).cpu().numpy() - ref).max() < 2e-6 * np.log2(n) * np.sqrt(n)
