@@ -322,3 +322,33 @@ def test_tiles_of_particles_in_no_grid_equal_the_plain_entry_points(device, n, i
     assert torch.allclose(gmc, mc, rtol=100 * 2.0 ** -24, atol=0)
     # eight products of mesh values up to 1, weights of sum 4 and a cotangent up to 1.5, in another order
     assert torch.allclose(gdc, dc, rtol=0, atol=32 * 1.5 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("mesh_shape,brick", [((128, 64, 64), (8, 8, 16)), ((256, 128, 128), (16, 16, 32))])
+def test_tiled_gather_adjoint_of_bricks_of_every_count(device, mesh_shape, brick):
+    """Bricks of no, one, and around 256, 512, 1024 and 2048 particles (a workgroup's threads and the
+    rounds of four per thread), the rest anywhere: the displacement cotangent of the plain entry point."""
+    from pmpp_amd import _lib
+    from pmpp_amd._torch import ptr, stream_handle
+    from pmpp_amd.cic.kernels import _geom
+
+    rng = np.random.default_rng(mesh_shape[0])
+    n, counts = 1 << 18, [0, 1, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4097]
+    nb = [m // b for m, b in zip(mesh_shape, brick)]
+    ids = np.repeat(np.arange(len(counts)) * 3, counts)  # every third brick of the first columns
+    ids = np.concatenate([ids, rng.integers(3 * len(counts), np.prod(nb), n - len(ids))])
+    corner = np.stack(np.unravel_index(ids, nb), 1) * np.array(brick)
+    pmid = (corner + rng.integers(0, brick, (n, 3))).astype(np.int16)
+    disp = rng.uniform(0, 1, (n, 3)).astype(np.float32)
+    order = rng.permutation(n)
+    P, D = _t(pmid[order], device, torch.int16), _t(np.minimum(disp, np.float32(0.999))[order], device)
+    V, M = _t(rng.normal(size=n), device), _t(rng.normal(size=mesh_shape), device)
+    geo = _geom(mesh_shape, mesh_shape, 0.0, 1.0, None)
+    assert _lib.size_query("pm_cic_tiled_workspace", n, 1, geo) > 0
+    dc, mc = torch.empty_like(D), torch.zeros_like(M)
+    _lib.call("pm_cic_gather_bwd", ptr(P), ptr(D), None, n, 1, geo, ptr(M), ptr(V), ptr(dc), ptr(mc),
+              stream_handle(device))
+    got, _ = hip_gather_bwd(P, D, M, V, offset=0.0, particle_cell_size=1.0, global_shape=mesh_shape)
+    # eight products of a mesh value, two weights (sum 4 over the corners) and a cotangent, in another order
+    scale = float(M.abs().max()) * V.abs()[:, None]
+    assert torch.all((got - dc).abs() <= 32 * 2.0 ** -24 * scale)
