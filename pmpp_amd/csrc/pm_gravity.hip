@@ -210,12 +210,11 @@ struct BrickShape {
   static constexpr int NT = BX == 8 ? 256 : 512;
   // particles of one brick processed per tile staging by the gathers: their results wait in LDS,
   // so each tile is read once per brick unless the brick holds more (~2x the mean occupancy at
-  // 1/8 particle per cell)
-  static constexpr int CAP = BX == 8 ? 512 : 2048;
+  // 1/8 particle per cell).  1024 for the small bricks, one staging per brick at one particle per cell
+  // (against 512: 128^3 particles on 128^3 53 -> 44 us, 64^3 on 64^3 20 -> 17 us; no different at 1/8 per
+  // cell)
+  static constexpr int CAP = BX == 8 ? 1024 : 2048;
   static constexpr int PPT = CAP / NT;
-  // the gather's: 1024 for the small bricks, one staging per brick at one particle per cell (128^3
-  // particles on 128^3: 53 -> 44 us, 64^3 on 64^3: 20 -> 17 us; no different at 1/8 per cell)
-  static constexpr int GATHER_CAP = BX == 8 ? 1024 : CAP;
   // LDS tile sizes: gather (float), scatter (int64) and one z plane
   static constexpr int TF = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxFloats;
   static constexpr int TW = BX ? (BX + 1) * (BY + 1) * (BZ + 2) : kTileMaxWords;
@@ -553,7 +552,7 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_gather_columns
     int run, const float* __restrict__ f0, const float* __restrict__ f1, const float* __restrict__ f2, int64_t nzero,
     float* __restrict__ acc) {
   using B_ = BrickShape<BX, BY, BZ>;
-  constexpr int NT = B_::NT, CAP = B_::GATHER_CAP, PPT = CAP / NT;
+  constexpr int NT = B_::NT, CAP = B_::CAP, PPT = B_::PPT;
   __shared__ __align__(16) float tile[B_::TF];
   __shared__ float res[3][CAP];
   __shared__ float plane[2][3][B_::PL];  // [parity of bz][component]: lower z plane of brick bz
@@ -630,8 +629,8 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_gather_columns
 // particle value), written as dc / a1 through perm: the reverse of the three gathers
 // (pallas.py:321-355) and the scatter adjoint's displacement term (pallas.py:358-409) in one
 // pass.  grad W_c = (s_x w_y w_z, w_x s_y w_z, w_x w_y s_z) with s = sign(-(f - b)), sign(0) =
-// 0 (the corner_grad convention).  Each mesh's tile is staged in turn; a particle's partial sums
-// wait in its thread's own LDS slots.  With a zero particle value the density term is skipped.
+// 0 (the corner_grad convention).  Each mesh's tile is staged in turn, a particle's partial sums
+// waiting in its thread's own LDS slots; small bricks' tiles are staged together.  With a zero particle value the density term is skipped.
 template <int BX, int BY, int BZ>
 __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_columns(
     const float4* __restrict__ rec, const int32_t* __restrict__ bin_off, const int32_t* __restrict__ perm, float cell,
@@ -640,8 +639,9 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_colum
     float* __restrict__ disp_cot, int accum) {
   using B_ = BrickShape<BX, BY, BZ>;
   constexpr int NT = B_::NT, CAP = B_::CAP, PPT = B_::PPT;
-  __shared__ __align__(16) float tile[B_::TF];
-  __shared__ float res[3][CAP];
+  constexpr bool ALL = BX == 8;  // every mesh's tile at once
+  __shared__ __align__(16) float tile[ALL ? 4 * B_::TF : B_::TF];
+  __shared__ float res[3][ALL ? 1 : CAP];
   __shared__ float plane[2][4][B_::PL];  // [parity of bz][mesh]: lower z plane of brick bz
   const B_ B(k);
   const int col = patch_column_of(blockIdx.x, gridDim.x, k.nb[0], k.nb[1]);
@@ -666,20 +666,22 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_colum
         load_plane(plane[me][m], m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot)), B, k, cx, cy, bz);
       continue;
     }
+    auto mesh = [&](int m) { return m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot)); };
     // mesh m's tile (and this brick's lower plane, for the brick below)
     auto stage = [&](int m) {
-      const float* __restrict__ F = m == 0 ? f0 : (m == 1 ? f1 : (m == 2 ? f2 : dcot));
       __syncthreads();  // the previous mesh's pass is done with the tile
-      stage_rows<BX, BY, BZ>(tile, F, B, k, cx, cy, bz);
+      stage_rows<BX, BY, BZ>(tile, mesh(m), B, k, cx, cy, bz);
       for (int i = threadIdx.x; i < rows; i += NT) tile[i * P + B.b2] = plane[up][m][i];
       __syncthreads();
       for (int i = threadIdx.x; i < rows; i += NT) plane[me][m][i] = tile[i * P];
     };
-    // sum_c M(c) grad W_c of the staged mesh
-    auto grads = [&](const float4& r, float gs[3]) {
-      const float fr[3] = {r.x, r.y, r.z};
-      const int c0 = sort::rec_cell(__float_as_uint(r.w));
+    // a particle's weights and the signs of their derivatives
+    struct Weights {
       float w[3][2], sg[3][2];
+    };
+    auto weights = [&](const float4& r) {
+      Weights W;
+      const float fr[3] = {r.x, r.y, r.z};
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
         float f = fr[a];
@@ -687,25 +689,76 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_colum
 #pragma unroll
         for (int bb = 0; bb < 2; ++bb) {
           const float delta = f - (float)bb;
-          w[a][bb] = 1.f - fabsf(delta);
-          sg[a][bb] = cic_sign(delta);
+          W.w[a][bb] = 1.f - fabsf(delta);
+          W.sg[a][bb] = cic_sign(delta);
         }
-        gs[a] = 0.f;
       }
+      return W;
+    };
+    // sum_c M(c) grad W_c over a staged mesh's corners from c0
+    auto grads = [&](const Weights& W, int c0, float gs[3]) {
+      gs[0] = gs[1] = gs[2] = 0.f;
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         const int bx = c & 1, by = (c >> 1) & 1, bzz = (c >> 2) & 1;
         const float v = tile[c0 + B.corner_off(c)];
-        gs[0] = gs[0] + v * (sg[0][bx] * w[1][by] * w[2][bzz]);
-        gs[1] = gs[1] + v * (w[0][bx] * sg[1][by] * w[2][bzz]);
-        gs[2] = gs[2] + v * (w[0][bx] * w[1][by] * sg[2][bzz]);
+        gs[0] = gs[0] + v * (W.sg[0][bx] * W.w[1][by] * W.w[2][bzz]);
+        gs[1] = gs[1] + v * (W.w[0][bx] * W.sg[1][by] * W.w[2][bzz]);
+        gs[2] = gs[2] + v * (W.w[0][bx] * W.w[1][by] * W.sg[2][bzz]);
       }
     };
-    // One mesh alone: staged once for the brick and the results written as they come.  With a staging and two
-    // barriers per CAP particles, bricks of many particles took longer than the float atomics had: CIC gather
-    // adjoint of 64^3 particles in one brick of a 128^3 mesh 2.21 -> 1.10 ms (atomics 1.21), shuffled on
-    // 128^3 128 -> 114 us (111), in C order 62 -> 49 (99), 128^3 on 256^3 168 -> 143 (736).
-    if (nm - m0 == 1) {
+    if constexpr (ALL) {
+      // Small bricks: the meshes are staged together, once per brick, and a particle's sums stay in
+      // registers.  Mesh by mesh and 512 particles at a time, a brick that holds most particles of a
+      // state was staged 2048 times: 64^3 particles in one brick of 128^3 3.29 ms (1.89 in the
+      // 512-thread walk of large bricks before), the whole VJP 6.07 -> 3.42 ms, CIC gather adjoint 2.21 -> 1.19
+      // (float atomics 1.21); VJP of 64^3 on 64^3 204 -> 196 us
+      constexpr int U = 4;
+      __syncthreads();
+      for (int m = m0; m < nm; ++m) {
+        float* T = tile + m * B_::TF;
+        stage_rows<BX, BY, BZ>(T, mesh(m), B, k, cx, cy, bz);
+        for (int i = threadIdx.x; i < rows; i += NT) T[i * P + B.b2] = plane[up][m][i];
+      }
+      __syncthreads();
+      for (int m = m0; m < nm; ++m)
+        for (int i = threadIdx.x; i < rows; i += NT) plane[me][m][i] = tile[m * B_::TF + i * P];
+      for (int64_t s0 = j0; s0 < j1; s0 += U * NT) {
+        float4 r[U];
+        float cf[U][4];
+        int32_t row[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {  // clamped loads
+          int64_t jq = s0 + threadIdx.x + (int64_t)q * NT;
+          jq = jq < j1 ? jq : j1 - 1;
+          r[q] = rec[jq];
+          row[q] = perm[jq];
+#pragma unroll
+          for (int m = 0; m < 4; ++m) cf[q][m] = m < 3 && m >= m0 && m < nm ? cot_s[(int64_t)m * n + jq] : val;
+        }
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+          if (s0 + threadIdx.x + (int64_t)q * NT >= j1) continue;
+          const Weights W = weights(r[q]);
+          const int c0 = sort::rec_cell(__float_as_uint(r[q].w));
+          float sum[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            if (m < m0 || m >= nm) continue;  // uniform
+            float gs[3];
+            grads(W, c0 + m * B_::TF, gs);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) sum[a] = sum[a] + cf[q][m] * gs[a];
+          }
+          float* out = disp_cot + (int64_t)row[q] * 3;
+#pragma unroll
+          for (int a = 0; a < 3; ++a) out[a] = (accum ? out[a] : 0.f) + sum[a] / cell;
+        }
+      }
+    } else if (nm - m0 == 1) {
+      // One mesh alone: staged once for the brick and the results written as they come.  With a staging and
+      // two barriers per CAP particles, bricks of many particles took long: CIC gather adjoint of 64^3
+      // particles in one brick of 256^3 1.00 -> 0.74 ms (float atomics 0.43), 128^3 on 256^3 168 -> 143 us (736)
       constexpr int U = 4;
       stage(m0);
       for (int64_t s0 = j0; s0 < j1; s0 += U * NT) {
@@ -724,49 +777,49 @@ __global__ void __launch_bounds__((BrickShape<BX, BY, BZ>::NT)) k_disp_cot_colum
         for (int q = 0; q < U; ++q) {
           if (s0 + threadIdx.x + (int64_t)q * NT >= j1) continue;
           float gs[3];
-          grads(r[q], gs);
+          grads(weights(r[q]), sort::rec_cell(__float_as_uint(r[q].w)), gs);
           float* out = disp_cot + (int64_t)row[q] * 3;
 #pragma unroll
           for (int a = 0; a < 3; ++a) out[a] = (accum ? out[a] : 0.f) + cf[q] * gs[a] / cell;
         }
       }
-      continue;
-    }
-    for (int64_t s0 = j0; s0 < j1; s0 += CAP) {
-      const int64_t s1 = s0 + CAP < j1 ? s0 + CAP : j1;
-      // each particle's record, once for every mesh
-      float4 r[PPT];
-#pragma unroll
-      for (int q = 0; q < PPT; ++q) {
-        const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
-        r[q] = rec[j < s1 ? j : s1 - 1];
-      }
-#pragma unroll 1
-      for (int m = m0; m < nm; ++m) {
-        stage(m);
-        float cf[PPT];
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {  // this mesh's coefficients (clamped loads)
-          const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
-          cf[q] = m < 3 ? cot_s[(int64_t)m * n + (j < s1 ? j : s1 - 1)] : val;
-        }
+    } else {
+      for (int64_t s0 = j0; s0 < j1; s0 += CAP) {
+        const int64_t s1 = s0 + CAP < j1 ? s0 + CAP : j1;
+        // each particle's record, once for every mesh
+        float4 r[PPT];
 #pragma unroll
         for (int q = 0; q < PPT; ++q) {
-          const int jl = threadIdx.x + q * NT;
-          if (s0 + jl >= s1) continue;
-          float gs[3];
-          grads(r[q], gs);
-#pragma unroll
-          for (int a = 0; a < 3; ++a) res[a][jl] = (m == m0 ? 0.f : res[a][jl]) + cf[q] * gs[a];
+          const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
+          r[q] = rec[j < s1 ? j : s1 - 1];
         }
-      }
+#pragma unroll 1
+        for (int m = m0; m < nm; ++m) {
+          stage(m);
+          float cf[PPT];
 #pragma unroll
-      for (int q = 0; q < PPT; ++q) {  // a thread's own results: no barrier
-        const int jl = threadIdx.x + q * NT;
-        if (s0 + jl < s1) {
-          const int64_t i = perm[s0 + jl];
+          for (int q = 0; q < PPT; ++q) {  // this mesh's coefficients (clamped loads)
+            const int64_t j = s0 + threadIdx.x + (int64_t)q * NT;
+            cf[q] = m < 3 ? cot_s[(int64_t)m * n + (j < s1 ? j : s1 - 1)] : val;
+          }
 #pragma unroll
-          for (int a = 0; a < 3; ++a) disp_cot[i * 3 + a] = res[a][jl] / cell;
+          for (int q = 0; q < PPT; ++q) {
+            const int jl = threadIdx.x + q * NT;
+            if (s0 + jl >= s1) continue;
+            float gs[3];
+            grads(weights(r[q]), sort::rec_cell(__float_as_uint(r[q].w)), gs);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) res[a][jl] = (m == m0 ? 0.f : res[a][jl]) + cf[q] * gs[a];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {  // a thread's own results: no barrier
+          const int jl = threadIdx.x + q * NT;
+          if (s0 + jl < s1) {
+            const int64_t i = perm[s0 + jl];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) disp_cot[i * 3 + a] = res[a][jl] / cell;
+          }
         }
       }
     }
