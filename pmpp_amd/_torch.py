@@ -37,10 +37,13 @@ def require_device(t: torch.Tensor, name: str) -> torch.Tensor:
 def as_contig(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
     """``t`` as a contiguous ``dtype`` tensor whose storage holds its values (a lazily conjugated or
     negated view is written out: ``contiguous`` alone would hand its storage over as it is)."""
-    require_device(t, name)
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        require_device(t, name)  # raises
     if t.dtype != dtype:
         t = t.to(dtype)
-    return t.resolve_conj().resolve_neg().contiguous()
+    if t.is_neg() or (dtype.is_complex and t.is_conj()):
+        t = t.clone()
+    return t.contiguous()
 
 
 def workspace(nbytes: int, device) -> torch.Tensor:
